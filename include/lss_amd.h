@@ -203,11 +203,11 @@ int lss_plan_problem_shape(const lss_adi_plan *plan, int64_t p, int64_t *nx, int
  * Batched plain tridiagonal systems (replaces one thomas_lu_solver::solve per line,
  * sparse_solvers/tridiagonal/thomas_lu_solver/lss_thomas_lu_solver.hpp:125-191, with Neumann(0) ends
  * and a[0] = c[n-1] = 0, i.e. the plain algorithm).  B systems of length n; layout CONTIGUOUS
- * (x[k*n+i]) or STRIDED (x[i*B+k]); device pointers; enqueued on `stream`.  Systems of up to 1024
- * unknowns (contiguous fp64: 512) are solved by the register-resident partitioned elimination with
- * no scratch; longer ones one lane per system, with B*n values of scratch allocated on `stream`
- * (stream-ordered, hipMallocAsync) and freed on it after the solve, so that calls on different streams
- * never share scratch.
+ * (x[k*n+i]) or STRIDED (x[i*B+k]); device pointers; enqueued on `stream`.  Contiguous systems of up to
+ * 7168 (fp64) or 8192 (fp32) unknowns and strided ones of up to 2048 are solved by the register-resident
+ * partitioned elimination with no scratch; longer ones one lane per system, with B*n values of scratch
+ * allocated on `stream` (stream-ordered, hipMallocAsync) and freed on it after the solve, so that calls on
+ * different streams never share scratch.
  */
 int lss_tridiag_batched(int32_t fp, int32_t layout, int64_t B, int64_t n, const void *a, const void *b,
                         const void *c, const void *d, void *x, void *stream);
@@ -236,10 +236,10 @@ int lss_tridiag_batched_bc(int32_t fp, int32_t layout, int64_t B, int64_t n, con
  * No counterpart in the reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc): the solve of
  * lss_tridiag_batched (lower == upper == NULL) or lss_tridiag_batched_bc (both non-NULL) that calls
- * no hipMalloc/hipFree or allocating routine.  The one-lane-per-system kernel (systems of more than
- * 1024 unknowns, or contiguous fp64 systems of more than 512) takes its B*n values of scratch from a
- * static per-device array of LSS_TRIDIAG_SCRATCH_BYTES, which each device holds until the process
- * ends; larger B*n*sizeof(fp) is rejected with LSS_ERR_INVALID.  Every call on a device shares that
+ * no hipMalloc/hipFree or allocating routine.  The one-lane-per-system kernel takes its B*n values of
+ * scratch from a static per-device array of LSS_TRIDIAG_SCRATCH_BYTES, which each device holds until the
+ * process ends; for systems of more than 1024 unknowns, and contiguous fp64 systems of more than 512, a
+ * larger B*n*sizeof(fp) is rejected with LSS_ERR_INVALID.  Every call on a device shares that
  * array: calls that overlap on one device (different streams or threads) race and give wrong results.
  * The caller passes inputs and outputs as for lss_tridiag_batched.
  */

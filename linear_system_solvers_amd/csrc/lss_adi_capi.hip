@@ -49,8 +49,10 @@ __global__ void k_adj_g(const Prob<T> *, const Adj<T> *, const Tile *, int, doub
 template <typename T> __global__ void k_copy_jobs(const CopyJob *);
 template <typename T, int M>
 __global__ void k_tridiag_rows(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
-template <typename T, int M>
+template <typename T, int M, int W, int NC>
 __global__ void k_tridiag_cols(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
+template <typename T, int NTMAX>
+__global__ void k_tridiag_long(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
 constexpr int P_NCH = 64, P_XTJ = 16, P_VROWS = 4;
 
 }  // namespace lssamd
@@ -1926,34 +1928,109 @@ template <typename T> lss_adi_plan *model_plan(const lss_model *models, int64_t 
 
 constexpr int TRI_WAVES_H = 4;  // systems per workgroup of k_tridiag_rows
 
-template <typename T, int M>
-void tridiag_part_m(int layout, int64_t B, int n, const void *a, const void *b, const void *c, const void *d, void *x,
-                    size_t lds_rows, const LineBC<T> &bc, hipStream_t st)
+template <typename T> struct TriArgs {
+    int64_t B;
+    int n;
+    const T *a, *b, *c, *d;
+    T *x;
+    LineBC<T> bc;
+    hipStream_t st;
+};
+
+template <int M, typename T> void tridiag_rows(const TriArgs<T> &t, size_t lds)
 {
-    const T *pa = (const T *)a, *pb = (const T *)b, *pc = (const T *)c, *pd = (const T *)d;
-    T *px = (T *)x;
-    if (layout == LSS_LAYOUT_CONTIGUOUS) {
-        const unsigned blocks = (unsigned)((B + TRI_WAVES_H - 1) / TRI_WAVES_H);
-        hipLaunchKernelGGL((k_tridiag_rows<T, M>), dim3(blocks), dim3(64 * TRI_WAVES_H), (unsigned)lds_rows, st, B, n,
-                           pa, pb, pc, pd, px, bc);
-    } else {
-        const unsigned blocks = (unsigned)((B + P_XTJ - 1) / P_XTJ);
-        hipLaunchKernelGGL((k_tridiag_cols<T, M>), dim3(blocks), dim3(P_XTJ * P_NCH), 0, st, B, n, pa, pb, pc, pd,
-                           px, bc);
-    }
+    hipLaunchKernelGGL((k_tridiag_rows<T, M>), dim3((unsigned)((t.B + TRI_WAVES_H - 1) / TRI_WAVES_H)),
+                       dim3(64 * TRI_WAVES_H), (unsigned)lds, t.st, t.B, t.n, t.a, t.b, t.c, t.d, t.x, t.bc);
+}
+template <int M, int W, int NC, typename T> void tridiag_cols(const TriArgs<T> &t)
+{
+    hipLaunchKernelGGL((k_tridiag_cols<T, M, W, NC>), dim3((unsigned)((t.B + W - 1) / W)), dim3(W * NC), 0, t.st, t.B,
+                       t.n, t.a, t.b, t.c, t.d, t.x, t.bc);
 }
 
-template <typename T>
-void tridiag_part(int M, int layout, int64_t B, int n, const void *a, const void *b, const void *c, const void *d,
-                  void *x, size_t lds_rows, const LineBC<T> &bc, hipStream_t st)
+// Threads of k_tridiag_long for nf unknowns (TRI_LONG_C each, whole wavefronts), or 0 when the system does
+// not fit a workgroup or its one staged array does not fit 64 KiB of LDS (more than 7168 unknowns in fp64,
+// 8192 in fp32: those keep one lane per system).
+template <typename T> int tridiag_long_threads(int64_t nf)
 {
-    switch (M) {
-    case 1: tridiag_part_m<T, 1>(layout, B, n, a, b, c, d, x, lds_rows, bc, st); break;
-    case 2: tridiag_part_m<T, 2>(layout, B, n, a, b, c, d, x, lds_rows, bc, st); break;
-    case 4: tridiag_part_m<T, 4>(layout, B, n, a, b, c, d, x, lds_rows, bc, st); break;
-    case 8: tridiag_part_m<T, 8>(layout, B, n, a, b, c, d, x, lds_rows, bc, st); break;
-    default: tridiag_part_m<T, 16>(layout, B, n, a, b, c, d, x, lds_rows, bc, st); break;
+    const int64_t nt = ((nf + TRI_LONG_C - 1) / TRI_LONG_C + 63) / 64 * 64;
+    return nt <= 1024 && (size_t)nt * (TRI_LONG_C + 1) * sizeof(T) <= 65536 ? (int)nt : 0;
+}
+
+// Contiguous systems.  One wavefront per system while four staged systems fit 64 KiB of LDS (fp64: 512
+// unknowns, fp32: 1024), else one workgroup per system (k_tridiag_long; 1000 x 2000 in fp64: 16 us against
+// 3380 us with one lane per system).  Returns false when neither takes the size.
+template <typename T> bool tridiag_part_rows(const TriArgs<T> &t, int64_t nf)
+{
+    const size_t lds = (size_t)TRI_WAVES_H * 4 * (size_t)t.n * sizeof(T);
+    if (nf <= 1024 && lds <= 65536) {
+        if (nf <= 64)
+            tridiag_rows<1>(t, lds);
+        else if (nf <= 128)
+            tridiag_rows<2>(t, lds);
+        else if (nf <= 256)
+            tridiag_rows<4>(t, lds);
+        else if (nf <= 512)
+            tridiag_rows<8>(t, lds);
+        else
+            tridiag_rows<16>(t, lds);
+        return true;
     }
+    const int nt = tridiag_long_threads<T>(nf);
+    if (nt == 0)
+        return false;
+    const size_t l = (size_t)nt * (TRI_LONG_C + 1) * sizeof(T);
+    if (nt <= 256)
+        hipLaunchKernelGGL((k_tridiag_long<T, 256>), dim3((unsigned)t.B), dim3(nt), (unsigned)l, t.st, t.B, t.n, t.a,
+                           t.b, t.c, t.d, t.x, t.bc);
+    else
+        hipLaunchKernelGGL((k_tridiag_long<T, 1024>), dim3((unsigned)t.B), dim3(nt), (unsigned)l, t.st, t.B, t.n, t.a,
+                           t.b, t.c, t.d, t.x, t.bc);
+    return true;
+}
+
+// Interleaved systems: W systems x NC chunks per workgroup.  Measured (systems x unknowns, us):
+//   fp32, up to 512: 32 x 32 against 16 x 64 (a whole 128-byte line per row, one reduction step less):
+//         65536 x 256: 70 against 84; 32768 x 509: 81 against 88;
+//   fp64, 257..512:  8 x 64 against 16 x 64 (two workgroups' registers where one fitted): 33554 x 500:
+//         169 against 195; 65536 x 256: 194 against 158, so shorter systems keep 16 x 64;
+//   fp64, 513..1024: 8 x 128 against 16 x 64 (chunks of 8, not 16, which spilled): 205 against 223;
+//   1025..2048: fp64 4 x 128 (209) against 4 x 256 (214), fp32 8 x 128 (121) against 4 x 256 (140), at
+//         8388 x 2000; longer systems keep one lane per system.
+template <typename T> bool tridiag_part_cols(const TriArgs<T> &t, int64_t nf)
+{
+    if constexpr (sizeof(T) == 4) {
+        if (nf <= 64)
+            tridiag_cols<2, 32, 32>(t);
+        else if (nf <= 128)
+            tridiag_cols<4, 32, 32>(t);
+        else if (nf <= 256)
+            tridiag_cols<8, 32, 32>(t);
+        else if (nf <= 512)
+            tridiag_cols<16, 32, 32>(t);
+        else if (nf <= 1024)
+            tridiag_cols<16, 16, 64>(t);
+        else if (nf <= 2048)
+            tridiag_cols<16, 8, 128>(t);
+        else
+            return false;
+    } else {
+        if (nf <= 64)
+            tridiag_cols<1, 16, 64>(t);
+        else if (nf <= 128)
+            tridiag_cols<2, 16, 64>(t);
+        else if (nf <= 256)
+            tridiag_cols<4, 16, 64>(t);
+        else if (nf <= 512)
+            tridiag_cols<8, 8, 64>(t);
+        else if (nf <= 1024)
+            tridiag_cols<8, 8, 128>(t);
+        else if (nf <= 2048)
+            tridiag_cols<16, 4, 128>(t);
+        else
+            return false;
+    }
+    return true;
 }
 
 }  // namespace
@@ -1999,10 +2076,48 @@ template <typename T> LineBC<T> line_bc(const lss_line_bc *lo, const lss_line_bc
     return bc;
 }
 
-// lss_tridiag_batched(_bc, _noalloc): lower/upper null = plain rows.  The one-lane-per-system kernel
-// needs B * n values of scratch: with noalloc it uses tridiag_scratch (sizes beyond it are rejected),
-// otherwise a stream-ordered allocation that is freed on `st` after the kernel, so that calls on
-// different streams never share scratch memory.
+// lss_tridiag_batched(_bc, _noalloc): lower/upper null = plain rows.  Only the one-lane-per-system kernel
+// (systems too long for the partitioned kernels) needs B * n values of scratch: with noalloc it uses
+// tridiag_scratch, otherwise a stream-ordered allocation that is freed on `st` after the kernel, so that
+// calls on different streams never share scratch memory.  noalloc rejects the same sizes whichever kernel
+// takes them: contiguous systems whose four staged arrays exceed 64 KiB of LDS for four systems, and any
+// system of more than 1024 unknowns, of which B * n values exceed the static array.
+template <typename T>
+void tridiag_run_t(int32_t layout, int64_t B, int64_t n, const void *a, const void *b, const void *c, const void *d,
+                   const lss_line_bc *lo, const lss_line_bc *hi, void *x, hipStream_t st, bool noalloc)
+{
+    // unknowns of the folded system
+    const int64_t nf = n - ((lo && lo->type == LSS_BC_DIRICHLET) ? 1 : 0) - ((hi && hi->type == LSS_BC_DIRICHLET) ? 1 : 0);
+    const size_t bytes = (size_t)B * (size_t)n * sizeof(T);
+    const bool rows = layout == LSS_LAYOUT_CONTIGUOUS;
+    if (noalloc && (nf > 1024 || (rows && (size_t)TRI_WAVES_H * 4 * (size_t)n * sizeof(T) > 65536)))
+        require(bytes <= TRIDIAG_SCRATCH_BYTES,
+                "lss_tridiag_batched_noalloc: B * n * sizeof(fp) = " + std::to_string(bytes) +
+                    " bytes of scratch exceeds its static maximum of " + std::to_string(TRIDIAG_SCRATCH_BYTES) +
+                    " bytes (systems of more than 1024 unknowns, or contiguous fp64 systems of more than 512, "
+                    "need B * n values of scratch)");
+    const TriArgs<T> t{B, (int)n, (const T *)a, (const T *)b, (const T *)c, (const T *)d, (T *)x,
+                       line_bc<T>(lo, hi, n), st};
+    if (rows ? tridiag_part_rows(t, nf) : tridiag_part_cols(t, nf)) {
+        HIPCHK(hipGetLastError());
+        return;
+    }
+    void *scr = nullptr;
+    if (noalloc) {
+        scr = static_scratch();
+    } else {
+        hipError_t e = hipMallocAsync(&scr, bytes, st);
+        if (e != hipSuccess)
+            throw lss_error(LSS_ERR_ALLOC, std::string("scratch hipMallocAsync failed: ") + hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(k_tridiag_lane<T>, dim3((unsigned)((B + 255) / 256)), dim3(256), 0, st, B, (int)n, (int)layout,
+                       t.a, t.b, t.c, t.d, t.x, (T *)scr, t.bc);
+    const hipError_t le = hipGetLastError();
+    if (!noalloc)
+        HIPCHK(hipFreeAsync(scr, st));
+    HIPCHK(le);
+}
+
 void tridiag_run(int32_t fp, int32_t layout, int64_t B, int64_t n, const void *a, const void *b, const void *c,
                  const void *d, const lss_line_bc *lo, const lss_line_bc *hi, void *x, hipStream_t st,
                  bool noalloc = false)
@@ -2016,52 +2131,10 @@ void tridiag_run(int32_t fp, int32_t layout, int64_t B, int64_t n, const void *a
                 "end condition type must be LSS_BC_DIRICHLET, LSS_BC_NEUMANN or LSS_BC_ROBIN");
     if (B == 0)
         return;
-    const size_t es = fp == LSS_FP64 ? 8 : 4;
-    // unknowns of the folded system
-    const int64_t nf = n - ((lo && lo->type == LSS_BC_DIRICHLET) ? 1 : 0) - ((hi && hi->type == LSS_BC_DIRICHLET) ? 1 : 0);
-    // partitioned solvers for lines of up to NCH * 16 unknowns (rows: while the staged systems fit
-    // 64 KiB of LDS), otherwise one lane per system with a scratch workspace
-    int M = 1;
-    while (M * P_NCH < nf && M < 32)
-        M *= 2;
-    const size_t lds_rows = (size_t)TRI_WAVES_H * 4 * (size_t)n * es;
-    const bool part = M <= 16 && (layout == LSS_LAYOUT_STRIDED || lds_rows <= 65536);
-    if (part) {
-        if (fp == LSS_FP64)
-            tridiag_part<double>(M, layout, B, (int)n, a, b, c, d, x, lds_rows, line_bc<double>(lo, hi, n), st);
-        else
-            tridiag_part<float>(M, layout, B, (int)n, a, b, c, d, x, lds_rows, line_bc<float>(lo, hi, n), st);
-    } else {
-        const size_t bytes = (size_t)B * (size_t)n * es;
-        void *scr = nullptr;
-        if (noalloc) {
-            require(bytes <= TRIDIAG_SCRATCH_BYTES,
-                    "lss_tridiag_batched_noalloc: B * n * sizeof(fp) = " + std::to_string(bytes) +
-                        " bytes of scratch exceeds its static maximum of " + std::to_string(TRIDIAG_SCRATCH_BYTES) +
-                        " bytes (systems of more than 1024 unknowns, or contiguous fp64 systems of more than 512, "
-                        "need B * n values of scratch)");
-            scr = static_scratch();
-        } else {
-            hipError_t e = hipMallocAsync(&scr, bytes, st);
-            if (e != hipSuccess)
-                throw lss_error(LSS_ERR_ALLOC, std::string("scratch hipMallocAsync failed: ") + hipGetErrorString(e));
-        }
-        const unsigned blocks = (unsigned)((B + 255) / 256);
-        if (fp == LSS_FP64)
-            hipLaunchKernelGGL(k_tridiag_lane<double>, dim3(blocks), dim3(256), 0, st, B, (int)n, (int)layout,
-                               (const double *)a, (const double *)b, (const double *)c, (const double *)d,
-                               (double *)x, (double *)scr, line_bc<double>(lo, hi, n));
-        else
-            hipLaunchKernelGGL(k_tridiag_lane<float>, dim3(blocks), dim3(256), 0, st, B, (int)n, (int)layout,
-                               (const float *)a, (const float *)b, (const float *)c, (const float *)d,
-                               (float *)x, (float *)scr, line_bc<float>(lo, hi, n));
-        const hipError_t le = hipGetLastError();
-        if (!noalloc)
-            HIPCHK(hipFreeAsync(scr, st));
-        HIPCHK(le);
-        return;
-    }
-    HIPCHK(hipGetLastError());
+    if (fp == LSS_FP64)
+        tridiag_run_t<double>(layout, B, n, a, b, c, d, lo, hi, x, st, noalloc);
+    else
+        tridiag_run_t<float>(layout, B, n, a, b, c, d, lo, hi, x, st, noalloc);
 }
 
 }  // namespace

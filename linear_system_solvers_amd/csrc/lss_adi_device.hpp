@@ -204,6 +204,8 @@ template <typename T> struct LineBC {
     }
 };
 
+constexpr int TRI_LONG_C = 8;  // unknowns per thread of k_tridiag_long
+
 // one device-to-device copy of n elements (checkpoint and lambda transfers)
 struct CopyJob {
     const void *src;

@@ -116,3 +116,42 @@ def test_end_condition_type_is_checked():
     with pytest.raises(L.LssError):
         L.tridiag_batched_bc(L.FP64, L.LAYOUT_CONTIGUOUS, 2, 8, t.data_ptr(), t.data_ptr(), t.data_ptr(),
                              t.data_ptr(), t.data_ptr(), (7, 0.0), (L.BC_DIRICHLET, 0.0))
+
+
+# ---------------------------------------------------------------------------------------------
+# Edges of the kernels' size ranges: one wavefront per system up to 512 (f64) / 1024 (f32) contiguous
+# unknowns, one workgroup up to 7168 / 8192, one lane beyond; interleaved systems change their tile
+# at 64, 128, 256, 512, 1024 and 2048.  B is odd and not a multiple of any tile.
+# Tolerance as above: the rows dominate (|a| + |c| <= 2 against b >= 2.5 + |a| + |c|), so neither
+# elimination amplifies rounding and both stay within tens of eps of the exact solution.
+# ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("layout,n", [(L.LAYOUT_CONTIGUOUS, n) for n in (512, 513, 1024, 1025, 1537, 2048, 2049, 4099,
+                                                                       7168, 7169, 8192, 8193)] +
+                         [(L.LAYOUT_STRIDED, n) for n in (64, 65, 129, 257, 512, 513, 1024, 1025, 2047, 2048, 2049)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_edges_of_the_size_ranges(oracle, fp, layout, n, in_place):
+    torch = pytest.importorskip("torch")
+    dt, B = L.np_dtype(fp), 35
+    a, b, c, d = _systems(B, n, dt, seed=n)
+    ref = oracle.thomas_batched(a, b, c, d, B, n, strided=False, fp="f64" if fp == L.FP64 else "f32").reshape(B, n)
+    if layout == L.LAYOUT_STRIDED:
+        a, b, c, d = (np.ascontiguousarray(v.T) for v in (a, b, c, d))
+    ta, tb, tc, td = (torch.from_numpy(v).cuda() for v in (a, b, c, d))
+    tx = td if in_place else torch.full_like(td, float("nan"))
+    L.tridiag_batched(fp, layout, B, n, ta.data_ptr(), tb.data_ptr(), tc.data_ptr(), td.data_ptr(), tx.data_ptr(),
+                      torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    x = tx.cpu().numpy().astype(np.float64)
+    x = x.T if layout == L.LAYOUT_STRIDED else x
+    err = np.abs(x - ref).max() / np.abs(ref).max()
+    print(f"n={n} layout={layout} fp={fp} in place {in_place}: err {err:.2e}", flush=True)
+    assert err <= (1e-13 if fp == L.FP64 else 1e-5)
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("layout", [L.LAYOUT_CONTIGUOUS, L.LAYOUT_STRIDED])
+@pytest.mark.parametrize("n", [513, 1026, 2050])
+def test_end_conditions_of_long_systems_match_the_oracle(oracle, fp, layout, n):
+    # (with two Dirichlet ends 1026 and 2050 points hold 1024 and 2048 unknowns)
+    test_end_conditions_match_the_oracle(oracle, fp, layout, n)
