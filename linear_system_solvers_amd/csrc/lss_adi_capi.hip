@@ -1990,8 +1990,10 @@ template <typename T> bool tridiag_part_rows(const TriArgs<T> &t, int64_t nf)
 }
 
 // Interleaved systems: W systems x NC chunks per workgroup.  Measured (systems x unknowns, us):
-//   fp32, up to 512: 32 x 32 against 16 x 64 (a whole 128-byte line per row, one reduction step less):
-//         65536 x 256: 70 against 84; 32768 x 509: 81 against 88;
+//   fp32, up to 256, batches that fill the GPU (two workgroups of 1024 threads per CU): 32 x 32 against
+//         16 x 64 (a whole 128-byte line per row, one reduction step less): 65536 x 256: 73 against 85;
+//         smaller batches keep 16 x 64, which makes twice the workgroups;
+//   fp32, 257..512:  16 x 64 against 32 x 32: 12289 x 509: 38 against 39; 1000 x 509: 8.7 against 10.2;
 //   fp64, 257..512:  8 x 64 against 16 x 64 (two workgroups' registers where one fitted): 33554 x 500:
 //         169 against 195; 65536 x 256: 194 against 158, so shorter systems keep 16 x 64;
 //   fp64, 513..1024: 8 x 128 against 16 x 64 (chunks of 8, not 16, which spilled): 205 against 223;
@@ -2000,14 +2002,15 @@ template <typename T> bool tridiag_part_rows(const TriArgs<T> &t, int64_t nf)
 template <typename T> bool tridiag_part_cols(const TriArgs<T> &t, int64_t nf)
 {
     if constexpr (sizeof(T) == 4) {
+        const bool wide = t.B >= 32 * 512;
         if (nf <= 64)
-            tridiag_cols<2, 32, 32>(t);
+            wide ? tridiag_cols<2, 32, 32>(t) : tridiag_cols<1, 16, 64>(t);
         else if (nf <= 128)
-            tridiag_cols<4, 32, 32>(t);
+            wide ? tridiag_cols<4, 32, 32>(t) : tridiag_cols<2, 16, 64>(t);
         else if (nf <= 256)
-            tridiag_cols<8, 32, 32>(t);
+            wide ? tridiag_cols<8, 32, 32>(t) : tridiag_cols<4, 16, 64>(t);
         else if (nf <= 512)
-            tridiag_cols<16, 32, 32>(t);
+            tridiag_cols<8, 16, 64>(t);
         else if (nf <= 1024)
             tridiag_cols<16, 16, 64>(t);
         else if (nf <= 2048)

@@ -14,8 +14,8 @@
 //
 // Memory bounds all three (5 values moved per unknown).  Measured on one MI355X, where a 4 + 4 GiB copy
 // reaches 4.8 TB/s: rows 65536 x 256 fp64 5.4 TB/s; long 1000 x 2000 fp64 16.3 us (4.9 TB/s; one lane per
-// system took 3380 us), 8388 x 2000 5.5 TB/s; cols 12289 x 509 fp32 27.6 us (53 us with 16 x 64 systems x
-// chunks in launch order).
+// system took 3380 us), 8388 x 2000 5.5 TB/s; cols 12289 x 509 fp32 38 us (3.3 TB/s; 53 us in launch
+// order).
 
 // The fast path may fuse multiply-adds (the library is built with -ffp-contract=off so that the exact
 // line solver keeps the reference's rounding; this translation unit opts back in).
@@ -79,7 +79,7 @@ __global__ void __launch_bounds__(64 * TRI_WAVES) k_tridiag_rows(int64_t B, int 
 
 // W systems x NC chunks of at most M points per workgroup.  Neighbouring workgroups share the cache lines at
 // the edges of their rows (all of them when B is odd), so each XCD takes a contiguous run of workgroups and
-// meets the shared lines in its own L2: 12289 x 509 in fp32 goes from 53 to 30 us by that alone.
+// meets the shared lines in its own L2: 12289 x 509 in fp32 goes from 53 to 38 us by that alone.
 template <typename T, int M, int W, int NC>
 __global__ void __launch_bounds__(W *NC) k_tridiag_cols(int64_t B, int n, const T *__restrict__ a,
                                                         const T *__restrict__ b, const T *__restrict__ c,
@@ -251,7 +251,10 @@ LSS_INST_C(double, 16, 4, 128)
 LSS_INST_C(float, 2, 32, 32)
 LSS_INST_C(float, 4, 32, 32)
 LSS_INST_C(float, 8, 32, 32)
-LSS_INST_C(float, 16, 32, 32)
+LSS_INST_C(float, 1, 16, 64)
+LSS_INST_C(float, 2, 16, 64)
+LSS_INST_C(float, 4, 16, 64)
+LSS_INST_C(float, 8, 16, 64)
 LSS_INST_C(float, 16, 16, 64)
 LSS_INST_C(float, 16, 8, 128)
 #undef LSS_INST_R
