@@ -1,8 +1,8 @@
-// lss_heat1d.hip -- the 1-D implicit heat / Black-Scholes solver: the exact kernel (one lane per problem,
+// lss_heat1d.hip -- the 1-D implicit heat / Black-Scholes solver: the exact kernel (four lanes per problem,
 // the reference's sequential Thomas LU / double-sweep order), the host plan and the C-ABI of
 // include/lss_heat1d.h.
 //
-// The exact kernel runs a problem's whole time loop in one lane: per step it forms each row of the
+// The exact kernel runs a problem's whole time loop in four lanes: per step it forms each row of the
 // theta scheme (implicit_heat_scheme::rhs / rhs_source and heat_implicit_solver_method::split,
 // pde_solvers/one_dimensional/heat_type/solver_method/lss_heat_implicit_solver_method.hpp:36-210) and
 // sweeps it as thomas_lu_solver (lss_thomas_lu_solver.hpp:125-191 with lss_thomas_lu_boundary.hpp:
@@ -16,6 +16,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 #include <vector>
 
 #include "lss/lss_heat1d_sampler.hpp"
@@ -28,196 +29,403 @@ namespace lssamd {
 template <typename T, int M>
 __global__ void k_h1_wave(const H1Prob<T> *, int, const T *const *, T *const *, T *const *);
 
-// boundary value pair of a step
-template <typename T> struct H1Bc {
-    int type;
-    T lin, val;
+// Lane i of a quad takes lane (CTRL >> 2i) & 3's value (DPP quad_perm).
+template <int CTRL> __device__ __forceinline__ int quad_mov(int v)
+{
+    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, true);
+}
+template <int CTRL> __device__ __forceinline__ float quad_perm(float v)
+{
+    return __int_as_float(quad_mov<CTRL>(__float_as_int(v)));
+}
+template <int CTRL> __device__ __forceinline__ double quad_perm(double v)
+{
+    return __hiloint2double(quad_mov<CTRL>(__double2hiint(v)), quad_mov<CTRL>(__double2loint(v)));
+}
+constexpr int QUAD_UP = 0x90, QUAD_DOWN = 0xf9;                      // lane q takes lane q - 1's / q + 1's
+template <int Q> constexpr int QUAD_BCAST = Q * 0x55;                // every lane takes lane Q's
+
+template <typename T> struct H1Vec {
+    typedef T v2 __attribute__((ext_vector_type(2)));
 };
 
+// Row N after the chain, among the lane's points t0 .. t0 + 3 (x the intermediate solution, gm gamma, gp
+// gamma of the point before, sp the intermediate solution before x[0]): a Dirichlet end is the end value;
+// the double sweep's Neumann / Robin end is lss_double_sweep_boundary.hpp:140-190 (L = -gamma).
 template <typename T>
-__global__ void __launch_bounds__(H1_EXACT_TILE) k_h1_exact(const H1Prob<T> *__restrict__ probs, int count,
-                                                             const T *const *__restrict__ uin,
-                                                             T *const *__restrict__ uout, T *const *__restrict__ surf)
+__device__ __forceinline__ void finish_end(T (&x)[4], const T (&gm)[4], const T (&gp)[4], T sp, int t0, int N, bool dhi,
+                                           bool dsweep, int hi_type, T h, T hi_lin, T hi_val)
 {
-    const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= count)
-        return;
-    const H1Prob<T> &P = probs[p];
-    const int n = P.n, N = n - 1, steps = P.steps;
-    const T one = (T)1.0, two = (T)2.0, mone = (T)-1.0, theta = P.theta, k = P.k, h = P.step;
-    T *prev = P.w0, *next = P.w1, *aux = P.w2;
-    const T *in = uin[p];
-    for (int g = 0; g < n; ++g)
-        prev[g] = in[g];
-    T *sf = surf ? surf[p] : nullptr;
-    const bool fwd = P.direction == H1_FORWARD;
-    if (sf)
-        for (int g = 0; g < n; ++g)
-            sf[(size_t)(fwd ? 0 : steps) * n + g] = prev[g];
-    for (int st = 0; st < steps; ++st) {
-        const T *cs = P.coeff + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)n;
-        const T *A = cs, *B = cs + n, *D = cs + 2 * n;
-        const T *bs = P.bnd + (P.bnd_sets > 1 ? st : 0) * 4;
-        const H1Bc<T> lo{P.lo_type, bs[0], bs[1]}, hi{P.hi_type, bs[2], bs[3]};
-        const T *src = P.src ? P.src + (size_t)st * 2 * (size_t)n : nullptr;
-        const T *srcn = src ? src + n : nullptr;
-        // rows of split (:200-210): low = -theta A, diag = 1 + 2 theta B, high = -theta D
-        auto ra = [&](int t) { return (-theta * A[t]); };
-        auto rb = [&](int t) { return (one + two * theta * B[t]); };
-        auto rc = [&](int t) { return (-theta * D[t]); };
-        // right-hand side of row t (rhs / rhs_source, :36-171); rows 0 and N only for Neumann / Robin ends
-        auto rf = [&](int t) -> T {
-            T r;
-            if (t == 0) {
-                const T beta = two * h * lo.val;
-                if (lo.type == BC_NEUMANN) {
-                    r = (one - theta) * beta * A[0] + (one - two * (one - theta) * B[0]) * prev[0] +
-                        (one - theta) * (A[0] + D[0]) * prev[1];
-                } else {
-                    const T alpha = two * h * lo.lin;
-                    r = (one - theta) * beta * A[0] + (one - (one - theta) * (two * B[0] - alpha * A[0])) * prev[0] +
-                        (one - theta) * (A[0] + D[0]) * prev[1];
-                }
-                if (src)
-                    r = r + theta * k * srcn[0] + (one - theta) * k * src[0];
-            } else if (t == N) {
-                const T delta = two * h * hi.val;
-                if (hi.type == BC_NEUMANN) {
-                    r = (one - theta) * (A[N] + D[N]) * prev[N - 1] + (one - two * (one - theta) * B[N]) * prev[N] -
-                        (one - theta) * delta * D[N];
-                } else {
-                    const T gamma = two * h * hi.lin;
-                    r = (one - theta) * (A[N] + D[N]) * prev[N - 1] +
-                        (one - (one - theta) * (two * B[N] + gamma * D[N])) * prev[N] - (one - theta) * delta * D[N];
-                }
-                if (src)
-                    r = r + theta * k * srcn[N] + (one - theta) * k * src[N];
+    const T one = (T)1.0, two = (T)2.0;
+#pragma unroll
+    for (int j = 3; j >= 0; --j) {
+        if (t0 + j != N)
+            continue;
+        if (dhi) {
+            x[j] = hi_val;
+        } else if (dsweep) {
+            const T LN = -gm[j], L1 = -gp[j], K1 = j > 0 ? x[j > 0 ? j - 1 : 0] : sp;
+            const T cst = two * h * hi_val;
+            if (hi_type == BC_NEUMANN) {
+                x[j] = (LN * (K1 - cst) + x[j]) / (one - LN * L1);
             } else {
-                r = (D[t] * (one - theta) * prev[t + 1]) + ((one - two * B[t] * (one - theta)) * prev[t]) +
-                    (A[t] * (one - theta) * prev[t - 1]);
-                if (src)
-                    r = r + k * (theta * srcn[t] + (one - theta) * src[t]);
+                const T lin = two * h * hi_lin;
+                x[j] = (LN * (K1 - cst) + x[j]) / (one - LN * (L1 - lin));
             }
-            return r;
-        };
-        if (P.tri == TRI_DSWEEP) {
-            // double_sweep_solver: L in aux, K in next, then the solution in place in next
-            T *L = aux, *K = next;
-            int start;
-            T k0, l0;
-            if (lo.type == BC_DIRICHLET) {
-                start = 1;
-                k0 = lo.val;
-                l0 = (T)0;
-            } else if (lo.type == BC_NEUMANN) {
-                start = 0;
-                k0 = (rf(0) - ra(0) * h * two * lo.val) / rb(0);
-                l0 = mone * (ra(0) + rc(0)) / rb(0);
-            } else {
-                const T tmp = rb(0) + ra(0) * h * two * lo.lin;
-                start = 0;
-                k0 = (rf(0) - ra(0) * h * two * lo.val) / tmp;
-                l0 = mone * (ra(0) + rc(0)) / tmp;
-            }
-            const int end = hi.type == BC_DIRICHLET ? n - 2 : n - 1;
-            L[0] = l0;
-            K[0] = k0;
-            for (int t = 1; t <= end; ++t) {
-                const T at = ra(t);
-                const T tmp = rb(t) + (at * L[t - 1]);
-                L[t] = mone * rc(t) / tmp;
-                K[t] = (rf(t) - (at * K[t - 1])) / tmp;
-            }
-            if (hi.type == BC_DIRICHLET) {
-                next[N] = hi.val;
-            } else if (hi.type == BC_NEUMANN) {
-                const T cst = two * h * hi.val;
-                next[N] = (L[N] * (K[N - 1] - cst) + K[N]) / (one - L[N] * L[N - 1]);
-            } else {
-                const T lin = two * h * hi.lin, cst = two * h * hi.val;
-                next[N] = (L[N] * (K[N - 1] - cst) + K[N]) / (one - L[N] * (L[N - 1] - lin));
-            }
-            for (int t = N - 1; t >= start; --t)
-                next[t] = (L[t] * next[t + 1]) + K[t];
-            if (start == 1)
-                next[0] = lo.val;
-        } else {
-            // thomas_lu_solver: gamma in aux, x in next, back-substitution in place in next
-            T *gam = aux, *x = next;
-            int start, end;
-            T beta0, gamma0, r0, z0, an, bn, rn;
-            if (lo.type == BC_DIRICHLET) {
-                start = 1;
-                beta0 = rb(1);
-                gamma0 = rc(1) / beta0;
-                r0 = rf(1) - ra(1) * lo.val;
-                z0 = r0 / beta0;
-            } else if (lo.type == BC_NEUMANN) {
-                const T cst = two * h * lo.val;
-                start = 0;
-                beta0 = rb(0);
-                gamma0 = (ra(0) + rc(0)) / beta0;
-                r0 = rf(0) - ra(0) * cst;
-                z0 = r0 / beta0;
-            } else {
-                const T lin = two * h * lo.lin, cst = two * h * lo.val;
-                start = 0;
-                beta0 = rb(0) + ra(0) * lin;
-                gamma0 = (ra(0) + rc(0)) / beta0;
-                r0 = rf(0) - ra(0) * cst;
-                z0 = r0 / beta0;
-            }
-            if (hi.type == BC_DIRICHLET) {
-                end = n - 2;
-                an = ra(N - 1);
-                bn = rb(N - 1);
-                rn = rf(N - 1) - rc(N - 1) * hi.val;
-            } else if (hi.type == BC_NEUMANN) {
-                const T cst = two * h * hi.val;
-                end = n - 1;
-                an = ra(N) + rc(N);
-                bn = rb(N);
-                rn = rf(N) + rc(N) * cst;
-            } else {
-                const T lin = two * h * hi.lin, cst = two * h * hi.val;
-                end = n - 1;
-                an = ra(N) + rc(N);
-                bn = rb(N) - rc(N) * lin;
-                rn = rf(N) + rc(N) * cst;
-            }
-            gam[start] = gamma0;
-            x[start] = z0;
-            for (int t = start + 1; t < end; ++t) {
-                const T at = ra(t);
-                const T beta = rb(t) - (at * gam[t - 1]);
-                gam[t] = rc(t) / beta;
-                x[t] = (rf(t) - (at * x[t - 1])) / beta;
-            }
-            const T beta_end = bn - (an * gam[end - 1]);
-            x[end] = (rn - (an * x[end - 1])) / beta_end;
-            for (int t = end - 1; t >= start; --t)
-                x[t] = x[t] - (gam[t] * x[t + 1]);
-            if (start == 1)
-                x[0] = lo.val;
-            if (end == N - 1)
-                x[N] = hi.val;
         }
-        T *tmp = prev;
-        prev = next;
-        next = tmp;
-        if (sf)
-            for (int g = 0; g < n; ++g)
-                sf[(size_t)(fwd ? st + 1 : steps - 1 - st) * n + g] = prev[g];
     }
-    T *out = uout[p];
-    for (int g = 0; g < n; ++g)
-        out[g] = prev[g];
 }
 
-template __global__ void k_h1_exact<double>(const H1Prob<double> *, int, const double *const *, double *const *,
-                                            double *const *);
-template __global__ void k_h1_exact<float>(const H1Prob<float> *, int, const float *const *, float *const *,
-                                           float *const *);
+// -------------------------------------------------------------------------------------------------
+// The exact kernel: four lanes (a quad) per problem, 16 problems per wavefront, the whole time loop in one
+// launch.  A line goes through the quad in groups of 16 points; lane q holds points 4q .. 4q + 3 of the
+// group.  Everything that does not depend on the previous point -- the loads, the rows of the theta scheme
+// and, once gamma is known, the divisors -- is formed by the four lanes at once; the recurrence of the
+// sweep then passes from lane to lane by DPP, each lane running its four points in the reference's order.
+// That chain (a multiplication, a subtraction and an IEEE division per point) bounds a wavefront; a large
+// book is bound by the 40 bytes of A, B, D and gamma (twice) that each point of each step reads: 16384
+// problems x 256 points x 1000 steps in fp64 take 29.4 ms, 5.7 TB/s from the last-level cache.  With one
+// lane per problem, each access in a cache line of its own, they took 304 ms (1.2 us a point).  Four lanes
+// make 1024 wavefronts of that book, one per SIMD.
+//
+// Layouts: a problem's A, B and D are padded to whole groups (16-byte aligned), so a quad reads whole
+// 128-byte lines; the level u (LDS when it fits, else the workspace) and gamma (workspace) are kept by lane,
+// so no lane ever reads another's memory.  The coefficients and gamma of the group after next are loaded
+// while a group's chain runs.
+//
+// Coefficients and boundary weights that do not change in time give the same gamma every step: it is
+// computed in the first step of a solve and read afterwards, which takes one of the two divisions out of
+// the chain.  The double sweep is the Thomas sweep with L = -gamma (b + a L = b - a gamma,
+// -c / beta = -(c / beta), L x + K = K - gamma x: negation is exact), so both run the same recurrence and
+// differ in the end rows only.
+// -------------------------------------------------------------------------------------------------
+template <typename T, bool LDSU>
+__global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ probs, int count,
+                                                 const T *const *__restrict__ uin, T *const *__restrict__ uout,
+                                                 T *const *__restrict__ surf)
+{
+    typedef typename H1Vec<T>::v2 v2;
+    extern __shared__ unsigned char h1_lds[];
+    const int lane = (int)threadIdx.x, ql = lane & 3;
+    const int p = (int)blockIdx.x * H1_EXACT_PROBS + (lane >> 2);
+    if (p >= count)
+        return;  // whole quads; there is no barrier
+    const H1Prob<T> &P = probs[p];
+    const int n = P.n, N = n - 1, steps = P.steps, ng = (n + 15) / 16, ld = P.ld;
+    const T one = (T)1.0, two = (T)2.0, theta = P.theta, k = P.k, h = P.step, omt = one - theta;
+    const bool dlo = P.lo_type == BC_DIRICHLET, dhi = P.hi_type == BC_DIRICHLET, dsweep = P.tri == TRI_DSWEEP;
+    const bool fwd = P.direction == H1_FORWARD, has_src = P.src != nullptr;
+    const bool const_gamma =
+        P.coeff_sets == 1 && (P.bnd_sets == 1 || (P.lo_type != BC_ROBIN && P.hi_type != BC_ROBIN));
+    T *const gbase = P.gamma, *const ubase = P.level;
+    lptr<T> ush = (lptr<T>)h1_lds;
+    // four own values of group g in the lane-ordered workspace / the level
+    auto ld4 = [&](const T *b, int g, T(&v)[4]) {
+        const v2 x = *(const v2 *)(b + ((size_t)(2 * g) * 64 + lane) * 2),
+                 y = *(const v2 *)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2);
+        v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
+    };
+    auto st4 = [&](T *b, int g, const T(&v)[4]) {
+        *(v2 *)(b + ((size_t)(2 * g) * 64 + lane) * 2) = v2{v[0], v[1]};
+        *(v2 *)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2) = v2{v[2], v[3]};
+    };
+    auto uget = [&](int g, T(&v)[4]) {
+        if constexpr (LDSU) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = ush[(4 * g + j) * 64 + lane];
+        } else {
+            ld4(ubase, g, v);
+        }
+    };
+    auto uput = [&](int g, const T(&v)[4]) {
+        if constexpr (LDSU) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                ush[(4 * g + j) * 64 + lane] = v[j];
+        } else {
+            st4(ubase, g, v);
+        }
+    };
+    auto store_level = [&](T *row, int g, const T(&v)[4]) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            if (16 * g + 4 * ql + j < n)
+                row[16 * g + 4 * ql + j] = v[j];
+    };
+    T *sf = surf ? surf[p] : nullptr, *out = uout[p];
+    {
+        const T *in = uin[p];
+        for (int g = 0; g < ng; ++g) {
+            T v[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                v[j] = in[min(16 * g + 4 * ql + j, N)];
+            uput(g, v);
+            if (sf)
+                store_level(sf + (size_t)(fwd ? 0 : steps) * n, g, v);
+        }
+    }
+    struct Stage {
+        T A[4], B[4], D[4], G[4];
+    };
+    for (int st = 0; st < steps; ++st) {
+        const T *cs = P.coeff + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)ld;
+        const T *bs = P.bnd + (P.bnd_sets > 1 ? st : 0) * 4;
+        const T lo_lin = bs[0], lo_val = bs[1], hi_lin = bs[2], hi_val = bs[3];
+        const T *src = has_src ? P.src + (size_t)st * 2 * (size_t)n : nullptr;
+        const bool reuse = const_gamma && st > 0;  // gamma of this problem is in the workspace
+        auto load = [&](int g, Stage &s) {
+            const int o = 16 * g + 4 * ql;
+            auto two_of = [&](const T *b, T(&v)[4]) {
+                const v2 x = *(const v2 *)(b + o), y = *(const v2 *)(b + o + 2);
+                v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
+            };
+            two_of(cs, s.A);
+            two_of(cs + ld, s.B);
+            two_of(cs + 2 * ld, s.D);
+            if (reuse)
+                ld4(gbase, g, s.G);
+        };
+        // ---- forward sweep: rows (a, b, c, f), gamma and the intermediate solution, which replaces the level
+        Stage s0, s1;
+        load(0, s0);
+        load(min(1, ng - 1), s1);
+        T uc[4], ulast = (T)0, glast = (T)0, gcar = (T)0, scar = (T)0;
+        uget(0, uc);
+        for (int g = 0; g < ng; ++g) {
+            Stage s2;
+            load(min(g + 2, ng - 1), s2);
+            T un[4];
+            uget(min(g + 1, ng - 1), un);
+            T left = quad_perm<QUAD_UP>(uc[3]), right = quad_perm<QUAD_DOWN>(uc[0]);
+            const T nfirst = quad_perm<QUAD_BCAST<0>>(un[0]);
+            left = ql == 0 ? ulast : left;
+            right = ql == 3 ? nfirst : right;
+            T a[4], b[4], c[4], f[4], gp[4], x[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const T A = s0.A[j], B = s0.B[j], D = s0.D[j];
+                const T um = j > 0 ? uc[j - 1] : left, up = j < 3 ? uc[j + 1] : right;
+                // rows of split (:200-210): low = -theta A, diag = 1 + 2 theta B, high = -theta D; interior
+                // right-hand side (:88-94)
+                a[j] = (-theta * A);
+                b[j] = (one + two * theta * B);
+                c[j] = (-theta * D);
+                f[j] = (D * omt * up) + ((one - two * B * omt) * uc[j]) + (A * omt * um);
+            }
+            const bool edge = g == 0 || 16 * g + 16 >= N;  // holds row 0, N - 1, N or points past the line
+            if (edge || has_src) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int t = 16 * g + 4 * ql + j;
+                    const T A = s0.A[j], B = s0.B[j], D = s0.D[j];
+                    const T um = j > 0 ? uc[j - 1] : left, up = j < 3 ? uc[j + 1] : right;
+                    const T sr = has_src ? src[min(t, N)] : (T)0, srn = has_src ? src[n + min(t, N)] : (T)0;
+                    if (t == 0) {
+                        if (dlo) {  // the end value; row 1 then folds it as f - a lo
+                            a[j] = c[j] = (T)0;
+                            b[j] = one;
+                            f[j] = lo_val;
+                        } else {  // Neumann / Robin lower row (:52-67) and its folding
+                            const T beta = two * h * lo_val;
+                            T r;
+                            if (P.lo_type == BC_NEUMANN) {
+                                r = omt * beta * A + (one - two * omt * B) * uc[j] + omt * (A + D) * up;
+                            } else {
+                                const T alpha = two * h * lo_lin;
+                                r = omt * beta * A + (one - omt * (two * B - alpha * A)) * uc[j] + omt * (A + D) * up;
+                            }
+                            if (has_src)
+                                r = r + theta * k * srn + omt * k * sr;
+                            const T ra = a[j];
+                            if (dsweep) {  // lss_double_sweep_boundary.hpp:88-190
+                                if (P.lo_type == BC_ROBIN)
+                                    b[j] = b[j] + ra * h * two * lo_lin;
+                                f[j] = r - ra * h * two * lo_val;
+                            } else {  // lss_thomas_lu_boundary.hpp:114-205
+                                if (P.lo_type == BC_ROBIN)
+                                    b[j] = b[j] + ra * (two * h * lo_lin);
+                                f[j] = r - ra * (two * h * lo_val);
+                            }
+                            c[j] = ra + c[j];
+                            a[j] = (T)0;
+                        }
+                    } else if (t == N) {
+                        if (dhi) {
+                            a[j] = c[j] = f[j] = (T)0;
+                            b[j] = one;
+                        } else {  // Neumann / Robin upper row (:70-86)
+                            const T delta = two * h * hi_val;
+                            T r;
+                            if (P.hi_type == BC_NEUMANN) {
+                                r = omt * (A + D) * um + (one - two * omt * B) * uc[j] - omt * delta * D;
+                            } else {
+                                const T gamma = two * h * hi_lin;
+                                r = omt * (A + D) * um + (one - omt * (two * B + gamma * D)) * uc[j] -
+                                    omt * delta * D;
+                            }
+                            if (has_src)
+                                r = r + theta * k * srn + omt * k * sr;
+                            f[j] = r;
+                            if (!dsweep) {
+                                const T ra = a[j], rc = c[j];
+                                a[j] = ra + rc;
+                                if (P.hi_type == BC_ROBIN)
+                                    b[j] = b[j] - rc * (two * h * hi_lin);
+                                f[j] = r + rc * (two * h * hi_val);
+                            }
+                        }
+                    } else if (t > N) {
+                        a[j] = c[j] = f[j] = (T)0;
+                        b[j] = one;
+                    } else {
+                        if (has_src)
+                            f[j] = f[j] + k * (theta * srn + omt * sr);
+                        if (t == N - 1 && dhi && !dsweep)
+                            f[j] = f[j] - c[j] * hi_val;
+                    }
+                }
+            }
+            // the chain: s = (f - a s) / (b - a gamma), gamma = c / (b - a gamma)
+            if (reuse) {
+                const T gup = quad_perm<QUAD_UP>(s0.G[3]);
+                T beta[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    gp[j] = j > 0 ? s0.G[j - 1] : (ql == 0 ? glast : gup);
+                    beta[j] = b[j] - (a[j] * gp[j]);
+                }
+                auto run = [&](auto qq) {
+                    constexpr int Q = decltype(qq)::value;
+                    if (ql == Q) {
+                        T sv = scar;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            x[j] = sv = (f[j] - (a[j] * sv)) / beta[j];
+                    }
+                    scar = quad_perm<QUAD_BCAST<Q>>(x[3]);
+                };
+                const T sprev = scar;
+                x[0] = x[1] = x[2] = x[3] = sprev;
+                run(std::integral_constant<int, 0>{});
+                run(std::integral_constant<int, 1>{});
+                run(std::integral_constant<int, 2>{});
+                run(std::integral_constant<int, 3>{});
+                if (edge) {
+                    const T xup = quad_perm<QUAD_UP>(x[3]);
+                    finish_end(x, s0.G, gp, ql == 0 ? sprev : xup, 16 * g + 4 * ql, N, dhi, dsweep, P.hi_type, h, hi_lin,
+                               hi_val);
+                }
+                glast = quad_perm<QUAD_BCAST<3>>(s0.G[3]);
+            } else {
+                T gm[4];
+                const T sprev = scar;
+                x[0] = x[1] = x[2] = x[3] = sprev;
+                gm[0] = gm[1] = gm[2] = gm[3] = gcar;
+                gp[0] = gp[1] = gp[2] = gp[3] = gcar;
+                auto run = [&](auto qq) {
+                    constexpr int Q = decltype(qq)::value;
+                    if (ql == Q) {
+                        T sv = scar, gv = gcar;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            gp[j] = gv;
+                            const T beta = b[j] - (a[j] * gv);
+                            gm[j] = gv = c[j] / beta;
+                            x[j] = sv = (f[j] - (a[j] * sv)) / beta;
+                        }
+                    }
+                    scar = quad_perm<QUAD_BCAST<Q>>(x[3]);
+                    gcar = quad_perm<QUAD_BCAST<Q>>(gm[3]);
+                };
+                run(std::integral_constant<int, 0>{});
+                run(std::integral_constant<int, 1>{});
+                run(std::integral_constant<int, 2>{});
+                run(std::integral_constant<int, 3>{});
+                st4(gbase, g, gm);
+                if (edge) {
+                    const T xup = quad_perm<QUAD_UP>(x[3]);
+                    finish_end(x, gm, gp, ql == 0 ? sprev : xup, 16 * g + 4 * ql, N, dhi, dsweep, P.hi_type, h, hi_lin,
+                               hi_val);
+                }
+            }
+            uput(g, x);
+            ulast = quad_perm<QUAD_BCAST<3>>(uc[3]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                uc[j] = un[j];
+            s0 = s1;
+            s1 = s2;
+        }
+        // ---- back substitution x = s - gamma x, from the last group down
+        T *lv = sf ? sf + (size_t)(fwd ? st + 1 : steps - 1 - st) * n : nullptr;
+        T g0[4], g1[4], sc[4], xcar = (T)0;
+        ld4(gbase, ng - 1, g0);
+        ld4(gbase, max(ng - 2, 0), g1);
+        uget(ng - 1, sc);
+        for (int g = ng - 1; g >= 0; --g) {
+            T g2[4], sn[4], x[4];
+            ld4(gbase, max(g - 2, 0), g2);
+            uget(max(g - 1, 0), sn);
+            x[0] = x[1] = x[2] = x[3] = xcar;
+            if (g == 0 || 16 * g + 16 >= N) {
+                auto run = [&](auto qq) {
+                    constexpr int Q = decltype(qq)::value;
+                    if (ql == Q) {
+                        T xv = xcar;
+#pragma unroll
+                        for (int j = 3; j >= 0; --j) {
+                            const int t = 16 * g + 4 * ql + j;
+                            // the forward sweep left the value itself at row N, at a Dirichlet row 0 and at
+                            // the Thomas sweep's last row before a Dirichlet end
+                            const bool own = t >= N || (t == 0 && dlo) || (t == N - 1 && dhi && !dsweep);
+                            x[j] = xv = own ? sc[j] : (sc[j] - (g0[j] * xv));
+                        }
+                    }
+                    xcar = quad_perm<QUAD_BCAST<Q>>(x[0]);
+                };
+                run(std::integral_constant<int, 3>{});
+                run(std::integral_constant<int, 2>{});
+                run(std::integral_constant<int, 1>{});
+                run(std::integral_constant<int, 0>{});
+            } else {
+                auto run = [&](auto qq) {
+                    constexpr int Q = decltype(qq)::value;
+                    if (ql == Q) {
+                        T xv = xcar;
+#pragma unroll
+                        for (int j = 3; j >= 0; --j)
+                            x[j] = xv = sc[j] - (g0[j] * xv);
+                    }
+                    xcar = quad_perm<QUAD_BCAST<Q>>(x[0]);
+                };
+                run(std::integral_constant<int, 3>{});
+                run(std::integral_constant<int, 2>{});
+                run(std::integral_constant<int, 1>{});
+                run(std::integral_constant<int, 0>{});
+            }
+            uput(g, x);
+            if (lv)
+                store_level(lv, g, x);
+            if (st == steps - 1)
+                store_level(out, g, x);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                g0[j] = g1[j];
+                g1[j] = g2[j];
+                sc[j] = sn[j];
+            }
+        }
+    }
+}
+
+#define LSS_INST_H1E(T)                                                                                             \
+    template __global__ void k_h1_exact<T, true>(const H1Prob<T> *, int, const T *const *, T *const *, T *const *); \
+    template __global__ void k_h1_exact<T, false>(const H1Prob<T> *, int, const T *const *, T *const *, T *const *);
+LSS_INST_H1E(double)
+LSS_INST_H1E(float)
+#undef LSS_INST_H1E
 
 }  // namespace lssamd
 
@@ -238,7 +446,10 @@ namespace {
 template <typename T> struct H1Plan final : lss_heat1d_plan {
     std::vector<H1Prob<T>> probs;
     dev_buffer mem, probs_dev, table_dev;
+    dev_buffer ws_dev;  // exact plans: gamma (and levels that do not fit LDS) of each wavefront, by lane
     int line_solver = LSS_LINE_EXACT;
+    int ngmax = 0;           // groups of 16 points of the longest line
+    bool lds_level = false;  // the level of every problem stays in LDS
     int pm = 1;  // chunk bound of the partitioned kernel
     std::vector<const void *> table;  // u_in, u_out, surfaces pointers of the last device run
     bool table_valid = false;
@@ -274,10 +485,11 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
             validate(d[q]);
             require(d[q].line_solver == line_solver, "all problems of a plan share line_solver");
             const size_t nq = (size_t)d[q].n;
+            const size_t ldq = (nq + 15) / 16 * 16;
             off[q] = total;
-            total += round(3 * nq * (size_t)d[q].coeff_sets) + round(4 * (size_t)d[q].bnd_sets) +
-                     (d[q].source ? round(2 * nq * (size_t)d[q].steps) : 0) +
-                     (line_solver == LSS_LINE_EXACT ? 3 * round(nq) : 0);
+            total += round(3 * ldq * (size_t)d[q].coeff_sets) + round(4 * (size_t)d[q].bnd_sets) +
+                     (d[q].source ? round(2 * nq * (size_t)d[q].steps) : 0);
+            ngmax = std::max(ngmax, (int)(ldq / 16));
             const int64_t nu = d[q].n - (d[q].lo_type == LSS_BC_DIRICHLET) - (d[q].hi_type == LSS_BC_DIRICHLET);
             while (pm * 64 < nu && pm < 16)
                 pm *= 2;
@@ -287,6 +499,7 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
         n.resize(cnt);
         steps.resize(cnt);
         T *base = (T *)mem.p;
+        std::vector<T> padded;
         for (int64_t q = 0; q < cnt; ++q) {
             const lss_heat1d_desc &e = d[q];
             const size_t nq = (size_t)e.n;
@@ -305,10 +518,15 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
             P.step = (T)1 / (T)(e.n - 1);  // grid_config<One>: one / (n - 1)
             T *o = base + off[q];
             T *c = o;
-            o += round(3 * nq * (size_t)e.coeff_sets);
+            const size_t ldq = (nq + 15) / 16 * 16, rows = 3 * (size_t)e.coeff_sets;
+            P.ld = (int32_t)ldq;
+            o += round(ldq * rows);
             T *b = o;
             o += round(4 * (size_t)e.bnd_sets);
-            LSS_HIPCHK(hipMemcpy(c, e.coeff, 3 * nq * (size_t)e.coeff_sets * sizeof(T), hipMemcpyHostToDevice));
+            padded.assign(ldq * rows, (T)0);
+            for (size_t r = 0; r < rows; ++r)
+                std::memcpy(padded.data() + r * ldq, (const T *)e.coeff + r * nq, nq * sizeof(T));
+            LSS_HIPCHK(hipMemcpy(c, padded.data(), padded.size() * sizeof(T), hipMemcpyHostToDevice));
             LSS_HIPCHK(hipMemcpy(b, e.bnd, 4 * (size_t)e.bnd_sets * sizeof(T), hipMemcpyHostToDevice));
             P.coeff = c;
             P.bnd = b;
@@ -317,18 +535,30 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
                 P.src = o;
                 o += round(2 * nq * (size_t)e.steps);
             }
-            if (line_solver == LSS_LINE_EXACT) {
-                P.w0 = o;
-                P.w1 = o + round(nq);
-                P.w2 = o + 2 * round(nq);
-            }
             n[q] = e.n;
             steps[q] = e.steps;
+        }
+        if (line_solver == LSS_LINE_EXACT) {  // each wavefront's workspace follows its longest line
+            lds_level = level_bytes() <= 65536;
+            std::vector<size_t> first(1, 0);
+            for (int64_t q = 0; q < cnt; q += H1_EXACT_PROBS) {
+                size_t ngw = 0;
+                for (int64_t z = q; z < std::min(cnt, q + H1_EXACT_PROBS); ++z)
+                    ngw = std::max(ngw, (size_t)probs[z].ld / 16);
+                first.push_back(first.back() + ngw * 256);
+            }
+            ws_dev.alloc(first.back() * (lds_level ? 1 : 2) * sizeof(T));
+            for (int64_t q = 0; q < cnt; ++q) {
+                probs[q].gamma = (T *)ws_dev.p + first[q / H1_EXACT_PROBS];
+                probs[q].level = lds_level ? nullptr : probs[q].gamma + first.back();
+            }
         }
         probs_dev.alloc(cnt * sizeof(H1Prob<T>));
         LSS_HIPCHK(hipMemcpy(probs_dev.p, probs.data(), cnt * sizeof(H1Prob<T>), hipMemcpyHostToDevice));
         table_dev.alloc(3 * cnt * sizeof(void *));
     }
+
+    size_t level_bytes() const { return (size_t)ngmax * 256 * sizeof(T); }  // levels of a wavefront's problems
 
     template <int M> void launch_wave(hipStream_t st, const T *const *ui, T *const *uo, T *const *sf)
     {
@@ -344,9 +574,13 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
         T *const *uo = (T *const *)(tb + count);
         T *const *sf = with_surf ? (T *const *)(tb + 2 * count) : nullptr;
         if (line_solver == LSS_LINE_EXACT) {
-            const unsigned blocks = (unsigned)((count + H1_EXACT_TILE - 1) / H1_EXACT_TILE);
-            hipLaunchKernelGGL(k_h1_exact<T>, dim3(blocks), dim3(H1_EXACT_TILE), 0, st, (const H1Prob<T> *)probs_dev.p,
-                               (int)count, ui, uo, sf);
+            const unsigned blocks = (unsigned)((count + H1_EXACT_PROBS - 1) / H1_EXACT_PROBS);
+            if (lds_level)
+                hipLaunchKernelGGL((k_h1_exact<T, true>), dim3(blocks), dim3(64), (unsigned)level_bytes(), st,
+                                   (const H1Prob<T> *)probs_dev.p, (int)count, ui, uo, sf);
+            else
+                hipLaunchKernelGGL((k_h1_exact<T, false>), dim3(blocks), dim3(64), 0, st,
+                                   (const H1Prob<T> *)probs_dev.p, (int)count, ui, uo, sf);
         } else {
             switch (pm) {
             case 1: launch_wave<1>(st, ui, uo, sf); break;

@@ -49,13 +49,13 @@ __global__ void __launch_bounds__(64 * H1_WAVES) k_h1_wave(const H1Prob<T> *__re
             u[t] = in[gidx(t)];
         T ulo = in[0], uhi = in[N];  // the level's end values (used where the ends are Dirichlet)
         auto load_coeff = [&](int st) {
-            const T *cs = P.coeff + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)n;
+            const T *cs = P.coeff + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)P.ld;
 #pragma unroll
             for (int t = 0; t < C; ++t) {
                 const int g = gidx(t);
                 cA[t] = cs[g];
-                cB[t] = cs[n + g];
-                cD[t] = cs[2 * n + g];
+                cB[t] = cs[P.ld + g];
+                cD[t] = cs[2 * P.ld + g];
             }
         };
         auto store_level = [&](T *row) {

@@ -162,3 +162,90 @@ def test_invalid_descriptions_are_rejected():
     with pytest.raises(L.LssError):
         plan.run_host([np.zeros(99)])
     plan.close()
+
+
+# ---------------------------------------------------------------------------------------------
+# Every form of a described problem through the exact kernel: both sweeps, the nine end pairs, coefficients
+# and boundaries fixed or changing in time, with and without a source, lines that end anywhere in a group of
+# 16 points, problems of different forms and lengths side by side in a wavefront, levels in LDS (every line
+# of the plan at most 512 points) and in the workspace.  The oracle steps the same rows one by one; the
+# kernel keeps its order of operations, so equality is exact.
+# ---------------------------------------------------------------------------------------------
+def _descr(ctypes, fp, n, steps, tri, lo, hi, direction, tdep_c, tdep_b, source, theta, rng):
+    dt = L.np_dtype(fp)
+    cs, bs = (steps if tdep_c else 1), (steps if tdep_b else 1)
+    A = rng.uniform(0.1, 2.0, (cs, n)).astype(dt)
+    D = rng.uniform(0.1, 2.0, (cs, n)).astype(dt)
+    B = ((A + D) / dt(2) + rng.uniform(0.0, 0.2, (cs, n)).astype(dt)).astype(dt)
+    return dict(fp=fp, n=n, steps=steps, tri=tri, lo=lo, hi=hi, direction=direction, theta=theta, k=dt(0.01),
+                coeff=np.ascontiguousarray(np.stack([A, B, D], 1)), bnd=rng.uniform(-0.5, 0.5, (bs, 4)).astype(dt),
+                src=rng.uniform(-1.0, 1.0, (steps, 2, n)).astype(dt) if source else None,
+                u0=rng.uniform(-1.0, 1.0, n).astype(dt))
+
+
+def _stepped(O, q):
+    dt, n, N = L.np_dtype(q["fp"]), q["n"], q["n"] - 1
+    one, two, th, k = dt(1), dt(2), dt(q["theta"]), dt(q["k"])
+    om, h = one - th, one / dt(n - 1)
+    u, levels = q["u0"].copy(), [q["u0"]]
+    solve = O.double_sweep if q["tri"] == L.DOUBLE_SWEEP else O.thomas_lu
+    for s in range(q["steps"]):
+        A, B, D = q["coeff"][s if len(q["coeff"]) > 1 else 0]
+        ll, lv, hl, hv = q["bnd"][s if len(q["bnd"]) > 1 else 0]
+        f = np.zeros(n, dt)
+        f[1:N] = (D[1:N] * om * u[2:]) + ((one - two * B[1:N] * om) * u[1:N]) + (A[1:N] * om * u[:N - 1])
+        if q["lo"] != L.BC_DIRICHLET:
+            beta = two * h * lv
+            mid = (one - two * om * B[0]) if q["lo"] == L.BC_NEUMANN else (one - om * (two * B[0] - two * h * ll * A[0]))
+            f[0] = om * beta * A[0] + mid * u[0] + om * (A[0] + D[0]) * u[1]
+        if q["hi"] != L.BC_DIRICHLET:
+            delta = two * h * hv
+            mid = (one - two * om * B[N]) if q["hi"] == L.BC_NEUMANN else (one - om * (two * B[N] + two * h * hl * D[N]))
+            f[N] = om * (A[N] + D[N]) * u[N - 1] + mid * u[N] - om * delta * D[N]
+        if q["src"] is not None:
+            F, Fn = q["src"][s]
+            f[1:N] = f[1:N] + k * (th * Fn[1:N] + om * F[1:N])
+            for e, t in ((0, q["lo"]), (N, q["hi"])):
+                if t != L.BC_DIRICHLET:
+                    f[e] = f[e] + th * k * Fn[e] + om * k * F[e]
+        u = solve(-th * A, one + two * th * B, -th * D, f, (q["lo"], ll, lv), (q["hi"], hl, hv),
+                  "f64" if q["fp"] == L.FP64 else "f32")
+        levels.append(u)
+    return np.stack(levels if q["direction"] == L.FORWARD else levels[::-1]), u
+
+
+def _described_plan(ctypes, descr, line_solver):
+    class D(ctypes.Structure):
+        _fields_ = [*[(f, ctypes.c_int32) for f in ("fp", "tridiagonal", "line_solver", "lo_type", "hi_type", "direction")],
+                    ("n", ctypes.c_int64), ("steps", ctypes.c_int64), ("theta", ctypes.c_double), ("k", ctypes.c_double),
+                    ("coeff_sets", ctypes.c_int64), ("coeff", ctypes.c_void_p), ("bnd_sets", ctypes.c_int64),
+                    ("bnd", ctypes.c_void_p), ("source", ctypes.c_void_p)]
+    arr = (D * len(descr))(*[D(q["fp"], q["tri"], line_solver, q["lo"], q["hi"], q["direction"], q["n"], q["steps"],
+                               q["theta"], float(q["k"]), len(q["coeff"]), q["coeff"].ctypes.data, len(q["bnd"]),
+                               q["bnd"].ctypes.data, None if q["src"] is None else q["src"].ctypes.data) for q in descr])
+    h = ctypes.c_void_p()
+    lib = H._lib()
+    assert lib.lss_heat1d_plan_create(arr, ctypes.c_int64(len(descr)), ctypes.byref(h)) == 0, L.lib().lss_last_error()
+    return H.Heat1dPlan(h.value, descr[0]["fp"], len(descr))
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("sizes", [(4, 5, 15, 16, 17, 18, 31, 32, 33, 48, 49, 70), (16, 17, 600, 513, 4, 530)])
+def test_every_form_of_the_exact_kernel_equals_the_oracle(oracle, fp, sizes):
+    import ctypes
+    import itertools
+    rng = np.random.default_rng(len(sizes))
+    ends = (L.BC_DIRICHLET, L.BC_NEUMANN, L.BC_ROBIN)
+    descr = []
+    for z, (tri, lo, hi, tc, tb, src) in enumerate(itertools.product((L.THOMAS_LU, L.DOUBLE_SWEEP), ends, ends, (0, 1), (0, 1),
+                                                                     (0, 1))):
+        descr.append(_descr(ctypes, fp, sizes[(z * 5 + z // 7) % len(sizes)], 3 + z % 3, tri, lo, hi,
+                            L.FORWARD if z % 2 else L.BACKWARD, tc, tb, src, 1.0 if z % 4 == 3 else 0.5, rng))
+    plan = _described_plan(ctypes, descr, L.LINE_EXACT)
+    for _ in range(2):  # the second solve finds the first one's workspace
+        outs, surfs = plan.run_host([q["u0"] for q in descr], surfaces=True)
+        for z, q in enumerate(descr):
+            surf, out = _stepped(oracle, q)
+            assert np.array_equal(outs[z], out), (z, q["n"], q["tri"], q["lo"], q["hi"])
+            assert np.array_equal(surfs[z], surf), (z, q["n"])
+    plan.close()
