@@ -28,11 +28,9 @@
 
 namespace lssamd {
 
-template <typename T> __global__ void k_bnd_a(const Prob<T> *, const Tile *, int);
 template <typename T> __global__ void k_bnd_b(const Prob<T> *, const Tile *, int);
-template <typename T> __global__ void k_xsweep(const Prob<T> *, const Tile *, int, int);
-template <typename T> __global__ void k_vsweep(const Prob<T> *, const Tile *, int, int);
-template <typename T> __global__ void k_hv_y3(const Prob<T> *, const Tile *, int);
+template <typename T, int PAT> __global__ void k_xsweep(const Prob<T> *, const Tile *, int, int, int);
+template <typename T, int PAT> __global__ void k_vsweep(const Prob<T> *, const Tile *, int, int, int);
 template <typename T, int PAT> __global__ void k_euler(const Prob<T> *, const Tile *, int);
 template <typename T, int PAT> __global__ void k_euler_res(const Prob<T> *, const Tile *);
 template <typename T>
@@ -142,10 +140,10 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     std::vector<ProbLayout> layouts;
     dev_buffer mem;                    // all problems
     dev_buffer probs_dev, tiles_dev;
-    // tile tables: rows [0,nx), cols [0,ny), S-lines [1,ny-2], v-lines [1,nx-2], interior rows
+    // tile tables: cols [0,ny), S-lines [1,ny-2], v-lines [1,nx-2]
     // adjoint: S-line tiles of P_XTJ, v-line tiles of P_VROWS, one tile per row (all rows)
     // forward partitioned sweeps: S-line tiles of 16 (TB_X) or 8 (TB_X8), v-line tiles of 4 (TB_V) or 16 (TB_V16)
-    enum { TB_I = 0, TB_J, TB_X, TB_V, TB_R, TB_AX, TB_AV, TB_U, TB_X8, TB_V16, TB_X4, TB_E, TB_P, TB_N };
+    enum { TB_J = 0, TB_X, TB_V, TB_AX, TB_AV, TB_U, TB_X8, TB_V16, TB_X4, TB_E, TB_P, TB_N };
     std::vector<Tile> tiles[TB_N];
     size_t tile_off[TB_N] = {};
     std::vector<int> prefix[TB_N];     // prefix[tb][q] = tiles of internal problems [0, q)
@@ -186,6 +184,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     bool adj_ok = false;               // every line fits the partitioned solver (needed by the adjoint)
     bool euler = false;                // explicit Euler plan (no line sweeps)
     bool euler_res = false;            // ... whose problems all fit k_euler_res (the loop resident in LDS)
+    bool all_fields = true;            // every problem has FIELDS coefficients
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
@@ -302,6 +301,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             euler_res = euler_res && descs[q].nx >= 4 && descs[q].ny <= ERES_T &&
                         descs[q].nx * descs[q].ny <= (int64_t)ERES_T * ERES_K && descs[q].coeff_sets == 1 &&
                         descs[q].bnd_sets == 1;
+        for (int64_t q = 0; q < n; ++q)
+            all_fields = all_fields && descs[q].coeff_mode == LSS_COEFF_FIELDS;
         {
             int64_t mx = 1, my = 1;
             for (int64_t q = 0; q < n; ++q) {
@@ -344,7 +345,9 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             L.off_y1 = take(nxy);
             L.off_y2 = one_stage(d) ? 0 : take(nxy);
             L.off_y3 = one_stage(d) ? 0 : take(nxy);
-            L.off_scr = take(nxy);
+            // blocks of 16 lines x 16 points, for the S-lines and for the v-lines
+            const size_t blocks = ((size_t)d.nx + 13) / 16 * (((size_t)d.ny + 13) / 16);
+            L.off_scr = line_solver == LINE_EXACT && !euler ? take(2 * blocks * EX_ARRAYS * 256) : 0;
             L.off_colA0 = take((size_t)d.nx);
             L.off_colA1 = take((size_t)d.nx);
             L.off_coeff = take(coeff_stride(d) * (size_t)d.coeff_sets);
@@ -388,8 +391,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             p.y1 = t + L.off_y1;
             p.y2 = one_stage(d) ? nullptr : t + L.off_y2;
             p.y3 = one_stage(d) ? nullptr : t + L.off_y3;
-            p.y4 = line_solver == LINE_PARTITIONED ? p.y3 : p.y1;
-            p.scr = t + L.off_scr;
+            p.y4 = p.y3;
+            p.scr = line_solver == LINE_EXACT && !euler ? t + L.off_scr : nullptr;
             p.colA0 = t + L.off_colA0;
             p.colA1 = t + L.off_colA1;
             p.coeff = t + L.off_coeff;
@@ -443,12 +446,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 const Prob<T> &p = probs[q];
                 int lo = 0, hi = 0, step = TILE;
                 switch (tb) {
-                case TB_I: lo = 0, hi = p.nx; break;
                 case TB_J: lo = 0, hi = p.ny; break;
-                case TB_X: lo = 1, hi = p.ny - 1, step = line_solver == LINE_PARTITIONED ? P_XTJ : TILE; break;
+                case TB_X: lo = 1, hi = p.ny - 1, step = line_solver == LINE_PARTITIONED ? P_XTJ : EXL; break;
                 case TB_V:
                     lo = 1, hi = p.nx - 1;
-                    step = line_solver == LINE_PARTITIONED ? P_VROWS * vlines_per_wave(p.ny - 2, pmy) : TILE;
+                    step = line_solver == LINE_PARTITIONED ? P_VROWS * vlines_per_wave(p.ny - 2, pmy) : EXL;
                     break;
                 case TB_AX: lo = 1, hi = p.ny - 1, step = P_XTJ; break;
                 case TB_AV: lo = 1, hi = p.nx - 1, step = P_VROWS; break;
@@ -456,8 +458,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 case TB_X8: lo = 1, hi = p.ny - 1, step = 8; break;
                 case TB_X4: lo = 1, hi = p.ny - 1, step = 4; break;
                 case TB_P: lo = 0, hi = 1, step = 1; break;  // one tile per problem
-                case TB_V16: lo = 1, hi = p.nx - 1, step = 16 * vlines_per_wave(p.ny - 2, pmy); break;
-                default: lo = 1, hi = p.nx - 1, step = 1; break;
+                default: lo = 1, hi = p.nx - 1, step = 16 * vlines_per_wave(p.ny - 2, pmy); break;  // TB_V16
                 }
                 if (tb == TB_U || tb == TB_E) {  // two-dimensional tiles (adjoint gathers, explicit step)
                     const int rows = tb == TB_U ? AGR : GTR * ERPT, cols = tb == TB_U ? AGC : GTC;
@@ -465,7 +466,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                         for (int c = 0; c < p.ny; c += cols)
                             tiles[tb].push_back({(int32_t)q, r, std::min(rows, p.nx - r), c});
                 } else {
-                    for (int s = lo; s < hi; s += step) {
+                    // exact plans lay their v-line tiles out from the last row: the tile that ends there holds the
+                    // two rows that boundary stage B extrapolates from
+                    const int first = tb == TB_V && line_solver == LINE_EXACT ? (hi - lo) % step : 0;
+                    if (first)
+                        tiles[tb].push_back({(int32_t)q, lo, first, 0});
+                    for (int s = lo + first; s < hi; s += step) {
                         Tile t;
                         t.prob = (int32_t)q;
                         t.first = s;
@@ -530,13 +536,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         for (int64_t q = 0; q < na; ++q) {
             const Prob<T> &p = probs[q];
             const double nxy = (double)p.nx * p.ny;
-            const bool dr = p.scheme == SCHEME_DR, hv = p.scheme == SCHEME_HV;
+            const bool dr = p.scheme == SCHEME_DR;
             switch (k) {
-            case LSS_K_BND_A: b += 5.0 * p.nx; break;
-            case LSS_K_XSWEEP1: b += 2 * nxy + (line_solver == LINE_PARTITIONED ? 5.0 * p.nx : 0); break;
+            case LSS_K_XSWEEP1: b += 2 * nxy + 5.0 * p.nx; break;
             case LSS_K_VSWEEP1: b += 3 * nxy; break;
-            case LSS_K_HV_Y3: b += hv ? 4 * nxy : 0; break;
-            case LSS_K_XSWEEP2: b += dr ? 0 : ((hv && line_solver != LINE_PARTITIONED) ? 3 * nxy : 4 * nxy); break;
+            case LSS_K_XSWEEP2: b += dr ? 0 : 4 * nxy; break;
             case LSS_K_VSWEEP2: b += dr ? 0 : 3 * nxy; break;
             case LSS_K_EULER: b += 2 * nxy; break;
             default: b += 4.0 * p.ny; break;
@@ -665,7 +669,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 try {
                     HIPCHK(hipStreamBeginCapture(gstream[g], hipStreamCaptureModeThreadLocal));
                     for (int s = 0; s < probs[g].steps; ++s)  // group g's first problem has its most steps
-                        launch_step(s, gstream[g]);
+                        launch_step(s, s == 0, gstream[g]);
                 } catch (...) {
                     set_ = 0;
                     hipGraph_t partial = nullptr;
@@ -760,7 +764,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 for (int rep = 0; rep < 2; ++rep) {  // the first pass warms caches and code
                     HIPCHK(hipEventRecord(e0, st));
                     for (int s = 0; s < nst; ++s)
-                        launch_step(s, st);
+                        launch_step(s, s == 0, st);
                     HIPCHK(hipEventRecord(e1, st));
                 }
                 HIPCHK(hipEventSynchronize(e1));
@@ -781,18 +785,17 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     }
 
     // one loop step of every active problem; `table` replaces the plan's problem table (the adjoint's
-    // recomputation writes each step's stage outputs into their own buffers)
-    void launch_step(int s, hipStream_t st, Profiler *prof = nullptr, const Prob<T> *table = nullptr)
+    // recomputation writes each step's stage outputs into their own buffers); fresh: the first step of a loop
+    // (the exact sweeps compute the lines' gamma there)
+    void launch_step(int s, bool fresh, hipStream_t st, Profiler *prof = nullptr, const Prob<T> *table = nullptr)
     {
         const int64_t na = active(s);
         const Prob<T> *pd = table ? table : (const Prob<T> *)probs_dev.p;
         const Tile *td = (const Tile *)tiles_dev.p;
         auto grid = [&](int tb) { return (unsigned)pre(tb, na); };
-        bool any_split2 = false, any_hv = false;
-        for (int64_t q = 0; q < na; ++q) {
+        bool any_split2 = false;
+        for (int64_t q = 0; q < na; ++q)
             any_split2 |= probs[q].scheme != SCHEME_DR;
-            any_hv |= probs[q].scheme == SCHEME_HV;
-        }
         auto pre = [&](int k) {
             if (prof)
                 prof->begin(k, algo_bytes(k, na));
@@ -814,21 +817,16 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             post();
             return;
         }
-        if (line_solver == LINE_EXACT) {  // (the partitioned stage-1 S-sweep evaluates stage A itself)
-            pre(LSS_K_BND_A);
-            hipLaunchKernelGGL(k_bnd_a<T>, dim3(grid(TB_I)), dim3(TILE), 0, st, pd, td + toff(TB_I), s);
-            post();
-        }
         auto xs = [&](int stage) {
             if (line_solver == LINE_EXACT) {
-                hipLaunchKernelGGL(k_xsweep<T>, dim3(grid(TB_X)), dim3(TILE), 0, st, pd, td + toff(TB_X), s, stage);
+                launch_exact(true, grid(TB_X), st, pd, td + toff(TB_X), s, stage, fresh && stage == 1);
                 return;
             }
             launch_x(stage, s, st, pd, na);
         };
         auto vs = [&](int stage) {
             if (line_solver == LINE_EXACT) {
-                hipLaunchKernelGGL(k_vsweep<T>, dim3(grid(TB_V)), dim3(TILE), 0, st, pd, td + toff(TB_V), s, stage);
+                launch_exact(false, grid(TB_V), st, pd, td + toff(TB_V), s, stage, fresh && stage == 1);
                 return;
             }
             launch_v(stage, s, st, pd, na);
@@ -839,11 +837,6 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         pre(LSS_K_VSWEEP1);
         vs(1);
         post();
-        if (any_hv && line_solver == LINE_EXACT) {
-            pre(LSS_K_HV_Y3);
-            hipLaunchKernelGGL(k_hv_y3<T>, dim3(grid(TB_R)), dim3(TILE), 0, st, pd, td + toff(TB_R), s);
-            post();
-        }
         if (any_split2) {
             pre(LSS_K_XSWEEP2);
             xs(2);
@@ -852,6 +845,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             vs(2);
             post();
         }
+        if (line_solver == LINE_EXACT)
+            return;  // (the last v-sweep evaluated stage B)
         pre(LSS_K_BND_B);
         hipLaunchKernelGGL(k_bnd_b<T>, dim3(grid(TB_J)), dim3(TILE), 0, st, pd, td + toff(TB_J), s);
         post();
@@ -988,16 +983,16 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         for (int64_t q = 0; q < n; ++q) {
             const Prob<T> &p = probs[q];
             const size_t nxy = ((size_t)p.nx * p.ny + 63) / 64 * 64;
-            const bool dr = p.scheme == SCHEME_DR, hv = p.scheme == SCHEME_HV;
-            const size_t nys = (dr ? 1 : 3) + ((hv && line_solver == LINE_EXACT) ? 1 : 0);
+            const bool dr = p.scheme == SCHEME_DR;
+            const size_t nys = dr ? 1 : 3;
             seg_bytes += ((size_t)(K + 1) + (size_t)K * nys) * nxy * sizeof(T);
         }
         dbl = overlap_mode >= 0 ? overlap_mode == 1 : seg_bytes <= SEG2_MAX_BYTES;
         for (int64_t q = 0; q < n; ++q) {
             const Prob<T> &p = probs[q];
             const size_t nxy = (size_t)p.nx * p.ny, nx_ = (size_t)p.nx, ny_ = (size_t)p.ny;
-            const bool dr = p.scheme == SCHEME_DR, hv = p.scheme == SCHEME_HV;
-            const size_t nys = (dr ? 1 : 3) + ((hv && line_solver == LINE_EXACT) ? 1 : 0);
+            const bool dr = p.scheme == SCHEME_DR;
+            const size_t nys = dr ? 1 : 3;
             const size_t nl = dr ? 4 : 7;
             const size_t nck = ((size_t)p.steps + K - 1) / K;
             const Terms *tm = terms.empty() ? nullptr : &terms[order[q]];
@@ -1024,8 +1019,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         for (int64_t q = 0; q < n; ++q) {
             const Prob<T> &p = probs[q];
             const size_t nxy = (size_t)p.nx * p.ny, nx_ = (size_t)p.nx, ny_ = (size_t)p.ny;
-            const bool dr = p.scheme == SCHEME_DR, hv = p.scheme == SCHEME_HV;
-            const size_t nys = (dr ? 1 : 3) + ((hv && line_solver == LINE_EXACT) ? 1 : 0);
+            const bool dr = p.scheme == SCHEME_DR;
+            const size_t nys = dr ? 1 : 3;
             const size_t nck = ((size_t)p.steps + K - 1) / K;
             auto al = [](size_t k) { return (k + 63) / 64 * 64; };
             T *t = (T *)(base + off_T[q]);
@@ -1125,13 +1120,13 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                     t.b = lk;
                     t.a = lk1;
                 }
-                const bool dr = t.scheme == SCHEME_DR, hv = t.scheme == SCHEME_HV;
-                const size_t nys = (dr ? 1 : 3) + ((hv && line_solver == LINE_EXACT) ? 1 : 0);
+                const bool dr = t.scheme == SCHEME_DR;
+                const size_t nys = dr ? 1 : 3;
                 T *yb = seg_y_base[q + set * n] + (size_t)k * nys * nxy;
                 t.y1 = yb;
                 t.y2 = dr ? nullptr : yb + nxy;
                 t.y3 = dr ? nullptr : yb + 2 * nxy;
-                t.y4 = line_solver == LINE_PARTITIONED ? t.y3 : (hv ? yb + 3 * nxy : t.y1);
+                t.y4 = t.y3;
                 seg[((size_t)set * K + k) * n + q] = t;
             }
         ck_len = K;
@@ -1308,7 +1303,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         for (int s = 0; s < max_steps; ++s) {
             if (s % K == 0)
                 launch_jobs(jd + fwd_job_off[s / K], fwd_job_n[s / K], stream);
-            launch_step(s, stream);
+            launch_step(s, s == 0, stream);
         }
         HIPCHK(hipGetLastError());
         for (int64_t q = 0; q < count; ++q) {
@@ -1349,7 +1344,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             const int s0 = c * K, s1 = std::min(max_steps, s0 + K);
             launch_jobs(jd + bwd_job_off[c], bwd_job_n[c], st);
             for (int s = s0; s < s1; ++s)
-                launch_step(s, st, nullptr, seg_table(s - s0, set));
+                launch_step(s, s == s0, st, nullptr, seg_table(s - s0, set));
         };
         auto adjoint = [&](int c, int set) {
             const int s0 = c * K, s1 = std::min(max_steps, s0 + K);
@@ -1421,10 +1416,27 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         HIPCHK(hipGetLastError());
     }
 
+    // a sweep of exact lines: S-lines (x) or v-lines
+    template <int PAT>
+    void launch_exact_t(bool x, unsigned grid, hipStream_t st, const Prob<T> *pd, const Tile *td, int s, int stage, int fresh)
+    {
+        if (x)
+            hipLaunchKernelGGL((k_xsweep<T, PAT>), dim3(grid), dim3(256), 0, st, pd, td, s, stage, fresh);
+        else
+            hipLaunchKernelGGL((k_vsweep<T, PAT>), dim3(grid), dim3(256), 0, st, pd, td, s, stage, fresh);
+    }
+    void launch_exact(bool x, unsigned grid, hipStream_t st, const Prob<T> *pd, const Tile *td, int s, int stage, int fresh)
+    {
+        if (all_fields)
+            launch_exact_t<PAT_FIELDS>(x, grid, st, pd, td, s, stage, fresh);
+        else
+            launch_exact_t<PAT_GENERIC>(x, grid, st, pd, td, s, stage, fresh);
+    }
+
     void launch_loop(hipStream_t st)
     {
         for (int s = 0; s < max_steps; ++s)
-            launch_step(s, st);
+            launch_step(s, s == 0, st);
         HIPCHK(hipGetLastError());
     }
 
@@ -1439,7 +1451,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                                   stream));
         }
         for (int s = 0; s < max_steps; ++s)
-            launch_step(s, stream, &prof);
+            launch_step(s, s == 0, stream, &prof);
         HIPCHK(hipGetLastError());
         for (int64_t q = 0; q < count; ++q) {
             const Prob<T> &p = probs[q];
@@ -1492,7 +1504,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 HIPCHK(hipStreamCreateWithFlags(&cap_stream, hipStreamNonBlocking));
                 HIPCHK(hipStreamBeginCapture(cap_stream, hipStreamCaptureModeThreadLocal));
                 for (int s = 0; s < max_steps; ++s)
-                    launch_step(s, cap_stream);
+                    launch_step(s, s == 0, cap_stream);
                 HIPCHK(hipStreamEndCapture(cap_stream, &graph));
                 HIPCHK(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
             }
@@ -1592,7 +1604,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         }
         launch_jobs(jd, (int)(lv_first[1] - lv_first[0]), stream);
         for (int s = 0; s < max_steps; ++s) {
-            launch_step(s, stream);
+            launch_step(s, s == 0, stream);
             launch_jobs(jd + lv_first[s + 1], (int)(lv_first[s + 2] - lv_first[s + 1]), stream);
         }
         HIPCHK(hipGetLastError());

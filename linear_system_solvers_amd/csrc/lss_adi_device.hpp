@@ -78,8 +78,9 @@ template <typename T> struct Prob {
     // general_heston_equation_coefficients scalars (coefficients.hpp:62-73) and theta, zeta
     T theta, zeta, alpha, beta, gamma, delta, ni, rho, h1;
     T *a, *b;                  // ping-pong state: step s reads (s even ? a : b), writes the other
-    T *y1, *y2, *y3, *scr;     // intermediates and line-solver scratch (nx*ny each)
-    T *y4;                     // HV's fourth stage: Y1's buffer (exact sweeps) or Y3's (partitioned)
+    T *y1, *y2, *y3;           // intermediates (nx*ny each)
+    T *scr;                    // workspace of the exact sweeps
+    T *y4;                     // HV's fourth stage: Y3's buffer (Y3 is evaluated in place)
     T *colA0, *colA1;          // v = 0 and v = v_max columns produced by boundary stage A (nx each)
     const uint32_t *idx1;      // index_of maps (lss_grid_config.hpp:110-118)
     const uint32_t *idx2;
@@ -204,6 +205,8 @@ template <typename T> struct LineBC {
     }
 };
 
+constexpr int EXL = 16;        // lines per tile of the exact sweeps (one wavefront, four lanes per line)
+constexpr int EX_ARRAYS = 6;   // arrays of the exact sweeps' workspace
 constexpr int TRI_LONG_C = 8;  // unknowns per thread of k_tridiag_long
 
 // one device-to-device copy of n elements (checkpoint and lambda transfers)

@@ -2,55 +2,30 @@
 //
 // One time step of every scheme is the same program of launches (the reference's loop body,
 // pde_solvers/two_dimensional/heat_type/lss_2d_general_heston_equation_implicit_kernel.hpp:177-184):
-//   bnd_a   boundary stage A: v = 0 column (explicit degenerate row) and v = v_max column
+//   xsweep  stage 1: S-lines j = 1..ny-2, rhs_intermed_1 of u, implicit solve along S  -> Y1; with it boundary
+//           stage A: v = 0 column (explicit degenerate row) and v = v_max column
 //           (lss_2d_general_heston_equation_explicit_boundary.hpp:181-200, :39-84)
-//   xsweep  stage 1: S-lines j = 1..ny-2, rhs_intermed_1 of u, implicit solve along S  -> Y1
 //   vsweep  stage 1: v-lines i = 1..nx-2, v-direction rhs, implicit solve along v     -> Y2 (DR: next)
-//   hv_y3   HV only: full-grid explicit stage                                         -> Y3
-//   xsweep  stage 2: CS/MCS rhs_intermed_3 -> Y3 ; HV rhs_intermed_4 -> Y4 (stored in Y1's buffer)
+//   xsweep  stage 2: CS/MCS rhs_intermed_3 -> Y3; HV rhs_intermed_4 -> Y4, its explicit stage Y3 evaluated in place
 //   vsweep  stage 2: v-direction rhs of (u, Y3) or (Y2, Y4)                          -> next
 //   bnd_b   boundary stage B: S_min row and S_max Neumann extrapolation (explicit_boundary.hpp:202-238)
+//           (exact lines: evaluated by the step's last v-sweep)
 // The explicit Euler solver's step is one launch of k_euler (interior and both boundary stages).
 // Kernels are compiled with -ffp-contract=off and keep the reference's operand order, so with
 // FIELDS coefficients every value is rounded exactly as the reference's host code rounds it.
-//
-// Line solves (v1): one lane per line, the forward sweep keeps (gamma_t, sol_t) in HBM
-// (sol in the output array, gamma in a scratch array), the backward sweep overwrites the output.
-// Lanes of a wavefront hold adjacent S-lines, so S-line sweeps read and write whole rows.
 
 #include "lss_adi_stencil.hpp"
+#include "lss_quad.hpp"
+
+#include <type_traits>
 
 namespace lssamd {
-
-constexpr int LB = 8;  // points per batch of the exact line sweeps
-
-// -------------------------------------------------------------------------------------------------
-// Boundary stage A: colA0 = new v = 0 column, colA1 = v_max column (explicit_boundary.hpp:39-84, :181-200)
-// as a launch of its own (plans with exact lines; the partitioned stage-1 S-sweep evaluates it itself)
-// -------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(TILE) k_bnd_a(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
-                                                int step)
-{
-    const Tile tl = tiles[blockIdx.x];
-    const Prob<T> &p = probs[tl.prob];
-    if (step >= p.steps || (int)threadIdx.x >= tl.count)
-        return;
-    bnd_a_row(p, step, tl.first + (int)threadIdx.x);
-}
 
 // -------------------------------------------------------------------------------------------------
 // Boundary stage B: row 0 Dirichlet, row nx-1 Neumann extrapolation through idx2 (explicit_boundary.hpp:202-238)
 // -------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(TILE) k_bnd_b(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
-                                                int step)
+template <typename T> __device__ __forceinline__ void bnd_b_col(const Prob<T> &p, int step, int j)
 {
-    const Tile tl = tiles[blockIdx.x];
-    const Prob<T> &p = probs[tl.prob];
-    if (step >= p.steps || (int)threadIdx.x >= tl.count)
-        return;
-    const int j = tl.first + threadIdx.x;
     const int nx = p.nx, ny = p.ny;
     const gptr<T> nxt = G((step & 1) ? p.a : p.b);
     const gptr<const T> bs = bnd_set(p, step);
@@ -62,265 +37,364 @@ __global__ void __launch_bounds__(TILE) k_bnd_b(const Prob<T> *__restrict__ prob
     nxt[j] = bs[nx + j];
     nxt[(int64_t)(nx - 1) * ny + j] = e;
 }
-
-// -------------------------------------------------------------------------------------------------
-// Line solve step of the forward sweep.  Thomas LU keeps (gamma_t, sol_t); double sweep keeps
-// (L_t, K_t).  first/last fold the Dirichlet ends exactly as thomas_lu_boundary.hpp:127-135,
-// 176-183 and double_sweep_boundary.hpp:100-106 do.
-// -------------------------------------------------------------------------------------------------
 template <typename T>
-__device__ __forceinline__ void fwd_step(int tri, bool first, bool last, T low, T diag, T high, T r, T lo, T hi,
-                                         T gprev, T sprev, T &g, T &s)
-{
-    if (tri == TRI_THOMAS) {
-        if (first) {
-            const T beta = diag;
-            g = high / beta;
-            const T rr = r - low * lo;
-            s = rr / beta;
-        } else if (!last) {
-            const T beta = diag - (low * gprev);
-            g = high / beta;
-            s = (r - (low * sprev)) / beta;
-        } else {
-            const T beta = diag - (low * gprev);
-            const T rn = r - high * hi;
-            s = (rn - (low * sprev)) / beta;
-            g = (T)0;
-        }
-    } else {
-        const T mone = (T)-1.0;
-        const T Lp = first ? (T)0 : gprev;
-        const T Kp = first ? lo : sprev;
-        const T tmp = diag + (low * Lp);
-        g = mone * high / tmp;
-        s = (r - (low * Kp)) / tmp;
-    }
-}
-
-template <typename T> __device__ __forceinline__ T bwd_step(int tri, T g, T s, T xnext)
-{
-    return tri == TRI_THOMAS ? (s - (g * xnext)) : ((g * xnext) + s);
-}
-
-// -------------------------------------------------------------------------------------------------
-// S-line sweep (one lane per line j).  stage 1: rhs_intermed_1(u) -> Y1.
-// stage 2: CS/MCS rhs_intermed_3(u, Y1, Y2) -> Y3; HV rhs_intermed_4(Y2, Y3) -> Y4 (in Y1's buffer).
-// Dirichlet ends: u(0, idx2[j]), u(nx-1, idx2[j]) (implicit_kernel.hpp:86-101, old time level).
-// -------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(TILE) k_xsweep(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
-                                                 int step, int stage)
-{
-    const Tile tl = tiles[blockIdx.x];
-    const Prob<T> &p = probs[tl.prob];
-    if (step >= p.steps || (stage == 2 && p.scheme == SCHEME_DR) || (int)threadIdx.x >= tl.count)
-        return;
-    const int j = tl.first + threadIdx.x;
-    const int nx = p.nx, ny = p.ny, end = nx - 2, tri = p.tri;
-    const T *u0 = (step & 1) ? p.b : p.a;
-    const gptr<const T> u = G(u0);
-    const gptr<const T> cs = coeff_set(p, step);
-    const T one = (T)1.0, theta = p.theta;
-    const int kind = (stage == 1) ? 0 : (p.scheme == SCHEME_CS ? 1 : (p.scheme == SCHEME_MCS ? 2 : 3));
-    const gptr<const T> in = G((kind == 3) ? (const T *)p.y2 : u0);
-    const gptr<const T> inh = G((const T *)((kind == 3) ? p.y3 : p.y1));
-    const gptr<const T> inhn = G((const T *)p.y2);
-    const gptr<T> out = G((kind == 0) ? p.y1 : (kind == 3 ? p.y4 : p.y3));
-    const gptr<T> scr = G(p.scr);
-    const uint32_t jj = p.idx2[j];
-    const T lo = u[jj], hi = u[(int64_t)(nx - 1) * ny + jj];
-    auto at = [&](gptr<const T> b, int64_t q) { return PAt<gptr<const T>>{b + q, ny}; };
-    const T *sp = kind == 0 ? src_set(p, step) : nullptr;
-    const int64_t nxy = (int64_t)nx * ny;
-    // The sweeps run in batches of LB points: the loads of a batch are issued together before its
-    // stores (the arrays read and written are distinct), so a lane waits once per batch, not per point.
-    T gprev = (T)0, sprev = (T)0;
-    for (int t0 = 1; t0 <= end; t0 += LB) {
-        T lw[LB], dg[LB], hg[LB], rr[LB];
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 + k;
-            if (t > end)
-                break;
-            const int64_t q = (int64_t)t * ny + j;
-            const Stencil<T> s = stencil_at(p, cs, t, j);
-            lw[k] = (-theta * s.M);
-            dg[k] = (one + theta * s.Z);
-            hg[k] = (-theta * s.P);
-            T r;
-            if (kind == 0) {
-                r = rhs_intermed_1(p, s, at(in, q));
-                // rhs_intermed_1_source (lss_heat_douglas_rachford_method.hpp:70-104)
-                if (sp)
-                    r = r + (theta * p.rho * sp[nxy + q]) + ((one - theta) * p.rho * sp[q]);
-            } else if (kind == 1)
-                r = rhs_intermed_3<T, false>(p, s, at(in, q), at(inh, q), at(inhn, q));
-            else if (kind == 2)
-                r = rhs_intermed_3<T, true>(p, s, at(in, q), at(inh, q), at(inhn, q));
-            else
-                r = rhs_intermed_4(p, s, at(in, q), at(inh, q));
-            rr[k] = r;
-        }
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 + k;
-            if (t > end)
-                break;
-            const int64_t q = (int64_t)t * ny + j;
-            T g, sv;
-            fwd_step(tri, t == 1, t == end, lw[k], dg[k], hg[k], rr[k], lo, hi, gprev, sprev, g, sv);
-            scr[q] = g;
-            out[q] = sv;
-            gprev = g;
-            sprev = sv;
-        }
-    }
-    T x = (tri == TRI_THOMAS) ? sprev : bwd_step(tri, gprev, sprev, hi);
-    out[(int64_t)end * ny + j] = x;
-    for (int t0 = end - 1; t0 >= 1; t0 -= LB) {
-        T gg[LB], ss[LB];
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 - k;
-            if (t < 1)
-                break;
-            const int64_t q = (int64_t)t * ny + j;
-            gg[k] = scr[q];
-            ss[k] = out[q];
-        }
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 - k;
-            if (t < 1)
-                break;
-            x = bwd_step(tri, gg[k], ss[k], x);
-            out[(int64_t)t * ny + j] = x;
-        }
-    }
-    out[j] = lo;
-    out[(int64_t)(nx - 1) * ny + j] = hi;
-}
-
-// -------------------------------------------------------------------------------------------------
-// v-line sweep (one lane per line i).  stage 1: rhs_v(u, Y1) -> Y2 (DR: next).
-// stage 2: CS/MCS rhs_v(u, Y3) -> next; HV rhs_v(Y2, Y4) -> next.
-// Dirichlet ends colA0/colA1[idx1[i]]: the copy of `next` the vertical lambdas captured after
-// boundary stage A (implicit_kernel.hpp:69-84).
-// -------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(TILE) k_vsweep(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
-                                                 int step, int stage)
-{
-    const Tile tl = tiles[blockIdx.x];
-    const Prob<T> &p = probs[tl.prob];
-    if (step >= p.steps || (stage == 2 && p.scheme == SCHEME_DR) || (int)threadIdx.x >= tl.count)
-        return;
-    const int i = tl.first + threadIdx.x;
-    const int ny = p.ny, end = ny - 2, tri = p.tri;
-    const T *u = (step & 1) ? p.b : p.a;
-    T *nxt = (step & 1) ? p.a : p.b;
-    const gptr<const T> cs = coeff_set(p, step);
-    const T one = (T)1.0, theta = p.theta;
-    const T *in0, *inh0;
-    T *out0;
-    if (stage == 1) {
-        in0 = u;
-        inh0 = p.y1;
-        out0 = (p.scheme == SCHEME_DR) ? nxt : p.y2;
-    } else if (p.scheme == SCHEME_HV) {
-        in0 = p.y2;
-        inh0 = p.y4;
-        out0 = nxt;
-    } else {
-        in0 = u;
-        inh0 = p.y3;
-        out0 = nxt;
-    }
-    const int64_t row = (int64_t)i * ny;
-    const uint32_t ii = p.idx1[i];
-    const T lo = G(p.colA0)[ii], hi = G(p.colA1)[ii];
-    const gptr<T> scr = G(p.scr + row);
-    const gptr<const T> in = G(in0 + row);
-    const gptr<const T> inh = G(inh0 + row);
-    const gptr<T> out = G(out0 + row);
-    // (batches of LB points, as in k_xsweep)
-    T gprev = (T)0, sprev = (T)0;
-    for (int t0 = 1; t0 <= end; t0 += LB) {
-        T lw[LB], dg[LB], hg[LB], rr[LB];
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 + k;
-            if (t > end)
-                break;
-            const Stencil<T> s = stencil_at(p, cs, i, t);
-            lw[k] = (-theta * s.Mt);
-            dg[k] = (one + theta * s.W);
-            hg[k] = (-theta * s.Pt);
-            rr[k] = rhs_v(p, s, in + t, inh + t);
-        }
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 + k;
-            if (t > end)
-                break;
-            T g, sv;
-            fwd_step(tri, t == 1, t == end, lw[k], dg[k], hg[k], rr[k], lo, hi, gprev, sprev, g, sv);
-            scr[t] = g;
-            out[t] = sv;
-            gprev = g;
-            sprev = sv;
-        }
-    }
-    T x = (tri == TRI_THOMAS) ? sprev : bwd_step(tri, gprev, sprev, hi);
-    out[end] = x;
-    for (int t0 = end - 1; t0 >= 1; t0 -= LB) {
-        T gg[LB], ss[LB];
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 - k;
-            if (t < 1)
-                break;
-            gg[k] = scr[t];
-            ss[k] = out[t];
-        }
-#pragma unroll
-        for (int k = 0; k < LB; ++k) {
-            const int t = t0 - k;
-            if (t < 1)
-                break;
-            x = bwd_step(tri, gg[k], ss[k], x);
-            out[t] = x;
-        }
-    }
-    out[0] = lo;
-    out[ny - 1] = hi;
-}
-
-// -------------------------------------------------------------------------------------------------
-// HV full-grid explicit stage Y3 (lss_heat_hundsdorfer_verwer_method.hpp:128-172), interior only.
-// One workgroup per row r; lanes over columns.
-// -------------------------------------------------------------------------------------------------
-template <typename T>
-__global__ void __launch_bounds__(TILE) k_hv_y3(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
+__global__ void __launch_bounds__(TILE) k_bnd_b(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
                                                 int step)
 {
     const Tile tl = tiles[blockIdx.x];
     const Prob<T> &p = probs[tl.prob];
-    if (step >= p.steps || p.scheme != SCHEME_HV)
+    if (step >= p.steps || (int)threadIdx.x >= tl.count)
         return;
-    const int r = tl.first;
-    const int ny = p.ny;
-    const gptr<const T> u = G((const T *)((step & 1) ? p.b : p.a));
+    bnd_b_col(p, step, tl.first + (int)threadIdx.x);
+}
+
+// -------------------------------------------------------------------------------------------------
+// Exact line sweeps.  DIR 0: S-lines (line l = column, point t = row), DIR 1: v-lines (line = row, point =
+// column).  A tile of EXL lines is swept in phases:
+//   exact_rhs     every thread forms right-hand sides of the tile's points (independent of each other), the
+//                 Dirichlet ends folded, into the workspace;
+//   exact_factor  a, beta = b - a gamma, 1 / beta and gamma = c / beta of the tile's rows, which do not depend on
+//                 the right-hand sides: in a loop's first step (fresh) for coefficients that do not change in time,
+//                 for both stages of every step, else in every step's first stage;
+//   exact_sweep   the recurrence s = (f - a s) / beta and the back substitution x = s - gamma x, four lanes (a quad)
+//                 per line, one wavefront per tile.
+// The last two take a line through the quad in groups of 16 points, lane q holding points 4q .. 4q + 3 of the group,
+// and pass the recurrence between the lanes in the reference's order, so every value is rounded as the reference
+// rounds it.  The double sweep is the same recurrence with L = -gamma (b + a L = b - a gamma, L x + K = K - gamma x:
+// negation is exact); the two differ in the last row only.
+// A wavefront issues an instruction every four to five cycles whatever it depends on, and one wavefront sweeps a
+// tile, so what bounds a sweep is the number of instructions of the recurrence: everything else is done by other
+// wavefronts (exact_rhs) or once per loop (exact_factor), and the workspace is laid out by lane, in 16-byte pieces at
+// fixed offsets, so that a group costs no addresses.  Measured in fp64 (one lane per line with the rows formed in the
+// sweep before): 100 x 50, 100 steps DR 8.8 -> 1.96 ms (the S-sweep 58.8 -> 12, the v-sweep 24.5 -> 8 us); 512 x 256
+// HV 1134 -> 157 us a step; 256 mixed problems of up to 512 x 256 points 149 -> 40 ms.
+//
+// Workspace (Prob::scr): the S-lines' tiles, then the v-lines'; of each tile its groups, of each group EX_ARRAYS
+// arrays of 256 values as [half][lane][2]: the right-hand sides, the intermediate solution, a, beta, 1 / beta, gamma.
+// -------------------------------------------------------------------------------------------------
+constexpr int EXT = 256;  // threads per tile
+constexpr int EXU = 3;    // points a thread forms at a time
+enum { EX_F = 0, EX_S = 1, EX_A = 2, EX_BETA = 3, EX_Y = 4, EX_G = 5 };
+
+// groups of 16 points of a line and block of array `arr` of (tile, group); the S-lines' tiles number the v-lines'
+// groups and the other way round
+template <typename T, int DIR> __device__ __forceinline__ int ex_groups(const Prob<T> &p)
+{
+    return ((DIR == 0 ? p.nx : p.ny) - 2 + 15) / 16;
+}
+template <typename T, int DIR> __device__ __forceinline__ gptr<T> ex_tile(const Prob<T> &p, int tile)
+{
+    const size_t nb = (size_t)ex_groups<T, 0>(p) * (size_t)ex_groups<T, 1>(p);
+    return G(p.scr) + ((size_t)DIR * nb + (size_t)tile * ex_groups<T, DIR>(p)) * (EX_ARRAYS * 256);
+}
+// point accessor at a 32-bit offset from a scalar base
+template <typename T> struct PAt32 {
+    gptr<const T> b;
+    uint32_t q, ny;
+    __device__ __forceinline__ T operator()(int di, int dj) const
+    {
+        return ldg(b, q + (uint32_t)di * ny + (uint32_t)dj);
+    }
+};
+template <typename T> struct Pair {
+    typedef T v2 __attribute__((ext_vector_type(2)));
+};
+template <typename T> __device__ __forceinline__ void ex_load(gptr<T> b, int g, int arr, int lane, T (&v)[4])
+{
+    typedef typename Pair<T>::v2 v2;
+    const gptr<const v2> q = (gptr<const v2>)(b + (size_t)g * (EX_ARRAYS * 256) + lane * 2) + arr * 128;
+    const v2 x = q[0], y = q[64];
+    v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
+}
+template <typename T> __device__ __forceinline__ void ex_store(gptr<T> b, int g, int arr, int lane, const T (&v)[4])
+{
+    typedef typename Pair<T>::v2 v2;
+    const gptr<v2> q = (gptr<v2>)(b + (size_t)g * (EX_ARRAYS * 256) + lane * 2) + arr * 128;
+    q[0] = v2{v[0], v[1]};
+    q[64] = v2{v[2], v[3]};
+}
+
+// Right-hand sides.  KIND: 0 stage-1 S-lines (every scheme); 1 CS, 2 MCS, 3 HV stage-2 S-lines (HV evaluates its
+// explicit stage Y3 in place); 4 v-lines (of in, inh).  Dirichlet ends of line l: lo(l), hi(l).
+template <typename T, int PAT, int KIND, typename LoF, typename HiF>
+__device__ __forceinline__ void exact_rhs(const Prob<T> &p, int step, int l0, int cnt, gptr<const T> in,
+                                          gptr<const T> inh, LoF &&lo, HiF &&hi, int tid)
+{
+    constexpr int DIR = KIND == 4 ? 1 : 0;
+    const int nx = p.nx, ny = p.ny, N = (DIR ? ny : nx) - 2;
+    constexpr int RP = EXT / EXL;  // points of a line formed side by side
+    const int c = DIR ? tid / RP : tid % EXL, r = DIR ? tid % RP : tid / EXL;
+    if (c >= cnt)
+        return;
+    const int l = l0 + c;
     const gptr<const T> cs = coeff_set(p, step);
-    const gptr<const T> y1 = G((const T *)p.y1), y2 = G((const T *)p.y2);
-    const gptr<T> y3 = G(p.y3);
-    for (int c = 1 + threadIdx.x; c < ny - 1; c += blockDim.x) {
-        const int64_t q = (int64_t)r * ny + c;
-        const Stencil<T> s = stencil_at(p, cs, r, c);
-        const PAt<gptr<const T>> in{u + q, ny}, inh{y1 + q, ny}, inhn{y2 + q, ny};
-        const T val = hv_y3_at(p, s, in, inh, inhn);
-        y3[q] = val;
+    const gptr<T> ws = ex_tile<T, DIR>(p, (l0 + EXL - 2) / EXL);
+    const gptr<const T> u = G((const T *)((step & 1) ? p.b : p.a)), y1 = G((const T *)p.y1), y2 = G((const T *)p.y2);
+    const T one = (T)1.0, theta = p.theta;
+    const T *sp = KIND == 0 ? src_set(p, step) : nullptr;
+    const int64_t nxy = (int64_t)nx * ny;
+    const bool thomas = p.tri == TRI_THOMAS;
+    auto at = [&](gptr<const T> b, uint32_t q) { return PAt32<T>{b, q, (uint32_t)ny}; };
+    auto point = [&](int t) -> T {
+        const int i = DIR ? l : t, j = DIR ? t : l;
+        const uint32_t q = (uint32_t)i * (uint32_t)ny + (uint32_t)j;
+        const Stencil<T> s = stencil_at<T, PAT>(p, cs, i, j);
+        T v;
+        if constexpr (KIND == 0) {
+            v = rhs_intermed_1(p, s, at(u, q));
+            // rhs_intermed_1_source (lss_heat_douglas_rachford_method.hpp:70-104)
+            if (sp)
+                v = v + (theta * p.rho * sp[nxy + q]) + ((one - theta) * p.rho * sp[q]);
+        } else if constexpr (KIND == 1) {
+            v = rhs_intermed_3<T, false>(p, s, at(u, q), at(y1, q), at(y2, q));
+        } else if constexpr (KIND == 2) {
+            v = rhs_intermed_3<T, true>(p, s, at(u, q), at(y1, q), at(y2, q));
+        } else if constexpr (KIND == 3) {  // rhs_intermed_4 (lss_heat_hundsdorfer_verwer_method.hpp:174-194)
+            const T y3 = hv_y3_at(p, s, at(u, q), at(y1, q), at(y2, q));
+            const auto y2q = at(y2, q);
+            v = (-theta * s.M * y2q(-1, 0)) + (theta * s.Z * y2q(0, 0)) - (theta * s.P * y2q(1, 0)) + y3;
+        } else {
+            v = rhs_v(p, s, GAt<T>{in, q}, GAt<T>{inh, q});
+        }
+        // the folded ends (thomas_lu_boundary.hpp:127-135, double_sweep_boundary.hpp:100-106)
+        if (t == 1)
+            v = v - (-theta * (DIR ? s.Mt : s.M)) * lo(l);
+        if (t == N && thomas)
+            v = v - (-theta * (DIR ? s.Pt : s.P)) * hi(l);
+        return v;
+    };
+    auto put = [&](int t, T v) {
+        const int g = (t - 1) >> 4, k = (t - 1) & 15, ln = c * 4 + (k >> 2);
+        ws[(size_t)g * (EX_ARRAYS * 256) + EX_F * 256 + ((k >> 1) & 1) * 128 + ln * 2 + (k & 1)] = v;
+    };
+    // EXU points at a time, loaded before the first store
+    for (int t = 1 + r; t <= N; t += RP * EXU) {
+        T v[EXU];
+#pragma unroll
+        for (int k = 0; k < EXU; ++k)
+            v[k] = point(min(t + RP * k, N));
+#pragma unroll
+        for (int k = 0; k < EXU; ++k)
+            if (t + RP * k <= N)
+                put(t + RP * k, v[k]);
+    }
+}
+
+// a, beta, 1 / beta and gamma of the rows of a tile's lines (identity rows past a line's end and for lines past the
+// tile's count, so that the sweep needs no conditions)
+template <typename T, int PAT, int DIR> __device__ __forceinline__ void exact_factor(const Prob<T> &p, int step, int l0, int cnt)
+{
+    const int lane = (int)threadIdx.x & 63, ql = lane & 3, end = (DIR == 0 ? p.nx : p.ny) - 2, ng = (end + 15) / 16;
+    const bool live = (lane >> 2) < cnt;
+    const int l = l0 + (live ? lane >> 2 : 0);
+    const gptr<const T> cs = coeff_set(p, step);
+    const gptr<T> ws = ex_tile<T, DIR>(p, (l0 + EXL - 2) / EXL);
+    const T one = (T)1.0, theta = p.theta;
+    struct Stage {
+        T M[4], Z[4], P[4];
+    };
+    auto load = [&](int g, Stage &s) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = min(1 + 16 * g + 4 * ql + j, end);
+            const Stencil<T> st = stencil_at<T, PAT>(p, cs, DIR == 0 ? t : l, DIR == 0 ? l : t);
+            s.M[j] = DIR == 0 ? st.M : st.Mt;
+            s.Z[j] = DIR == 0 ? st.Z : st.W;
+            s.P[j] = DIR == 0 ? st.P : st.Pt;
+        }
+    };
+    T gcar = (T)0;
+    auto body = [&](int g, Stage &s) {
+        T a[4], b[4], c[4], beta[4], gm[4], y[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int t = 1 + 16 * g + 4 * ql + j;
+            const bool row = live && t <= end;
+            a[j] = (row && t > 1) ? (-theta * s.M[j]) : (T)0;  // (the first row's end is folded)
+            b[j] = row ? (one + theta * s.Z[j]) : one;
+            c[j] = row ? (-theta * s.P[j]) : (T)0;
+        }
+        gcar = quad_gamma(a, b, c, gcar, beta, gm);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+            y[j] = quick_rcp(beta[j]);
+        ex_store(ws, g, EX_A, lane, a);
+        ex_store(ws, g, EX_BETA, lane, beta);
+        ex_store(ws, g, EX_Y, lane, y);
+        ex_store(ws, g, EX_G, lane, gm);
+    };
+    quad_stages<Stage>(0, ng, 1, load, body);
+}
+
+// forward recurrence and back substitution of a tile's lines; out: the solution's array, lo and hi: the lane's line's
+// end values
+template <typename T, int DIR>
+__device__ __forceinline__ void exact_sweep(const Prob<T> &p, int l0, int cnt, gptr<T> out, T lo, T hi)
+{
+    const int lane = (int)threadIdx.x & 63, ql = lane & 3, ny = p.ny, end = (DIR == 0 ? p.nx : ny) - 2, ng = (end + 15) / 16;
+    const bool live = (lane >> 2) < cnt;
+    const gptr<T> ws = ex_tile<T, DIR>(p, (l0 + EXL - 2) / EXL);
+    const bool thomas = p.tri == TRI_THOMAS;
+    struct Stage {
+        T a[4], beta[4], y[4], f[4];
+    };
+    auto load = [&](int g, Stage &s) {
+        ex_load(ws, g, EX_A, lane, s.a);
+        ex_load(ws, g, EX_BETA, lane, s.beta);
+        ex_load(ws, g, EX_Y, lane, s.y);
+        ex_load(ws, g, EX_F, lane, s.f);
+    };
+    SeenNum seen;
+    T scar = (T)0;
+    quad_stages<Stage>(0, ng, 1, load, [&](int g, Stage &s) {
+        T x[4];
+        scar = quad_forward<true>(s.a, s.f, s.beta, s.y, scar, x, seen);
+        ex_store(ws, g, EX_S, lane, x);
+    });
+    if (__builtin_amdgcn_ballot_w64(!seen_ok(seen, scar))) {  // a numerator outside quick_div's range
+        scar = (T)0;
+#pragma unroll 1
+        for (int g = 0; g < ng; ++g) {
+            Stage s;
+            T x[4];
+            load(g, s);
+            scar = quad_forward<false>(s.a, s.f, s.beta, s.y, scar, x, seen);
+            ex_store(ws, g, EX_S, lane, x);
+        }
+    }
+    struct Back {
+        T G[4], s[4];
+    };
+    auto loadb = [&](int g, Back &b) {
+        ex_load(ws, g, EX_G, lane, b.G);
+        ex_load(ws, g, EX_S, lane, b.s);
+    };
+    const uint32_t l = (uint32_t)(l0 + (live ? lane >> 2 : 0));
+    const uint32_t base = DIR == 0 ? l : l * (uint32_t)ny, str = DIR == 0 ? (uint32_t)ny : 1u;
+    T xcar = hi;
+    quad_stages<Back>(ng - 1, ng, -1, loadb, [&](int g, Back &b) {
+        const int t0 = 1 + 16 * g + 4 * ql;
+        T x[4];
+        if (g == ng - 1) {  // the Thomas sweep's last point is s itself
+            xcar = quad_backward_ends(
+                b.G, b.s, xcar, x, [&](int j) { return t0 + j == end && thomas; }, [&](int j) { return t0 + j > end; });
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (live && t0 + j <= end)
+                    stg(out, base + (uint32_t)(t0 + j) * str, x[j]);
+        } else {
+            xcar = quad_backward(b.G, b.s, xcar, x);
+            if (live) {
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+                    stg(out, base + (uint32_t)(t0 + j) * str, x[j]);
+            }
+        }
+    });
+    if (live && ql == 0) {
+        stg(out, base, lo);
+        stg(out, base + (uint32_t)(end + 1) * str, hi);
+    }
+}
+
+// S-line sweep of tile (l0, cnt).  stage 1: rhs_intermed_1(u) -> Y1.  stage 2: CS/MCS rhs_intermed_3(u, Y1, Y2)
+// -> Y3; HV rhs_intermed_4(Y2, Y3) -> Y4.  Dirichlet ends u(0, idx2[j]), u(nx-1, idx2[j])
+// (implicit_kernel.hpp:86-101, old time level).
+template <typename T, int PAT>
+__device__ __forceinline__ void xsweep_rhs(const Prob<T> &p, int step, int stage, int l0, int cnt, int tid)
+{
+    const gptr<const T> u = G((const T *)((step & 1) ? p.b : p.a)), none = nullptr;
+    auto lo = [&](int j) { return ldg(u, p.idx2[j]); };
+    auto hi = [&](int j) { return ldg(u, (uint32_t)(p.nx - 1) * (uint32_t)p.ny + p.idx2[j]); };
+    if (stage == 1)
+        exact_rhs<T, PAT, 0>(p, step, l0, cnt, none, none, lo, hi, tid);
+    else if (p.scheme == SCHEME_CS)
+        exact_rhs<T, PAT, 1>(p, step, l0, cnt, none, none, lo, hi, tid);
+    else if (p.scheme == SCHEME_MCS)
+        exact_rhs<T, PAT, 2>(p, step, l0, cnt, none, none, lo, hi, tid);
+    else
+        exact_rhs<T, PAT, 3>(p, step, l0, cnt, none, none, lo, hi, tid);
+}
+template <typename T, int PAT>
+__device__ __forceinline__ void xsweep_solve(const Prob<T> &p, int step, int stage, bool fresh, int l0, int cnt)
+{
+    const int lane = (int)threadIdx.x & 63;
+    if (fresh)
+        exact_factor<T, PAT, 0>(p, step, l0, cnt);
+    const gptr<const T> u = G((const T *)((step & 1) ? p.b : p.a));
+    const uint32_t jj = p.idx2[l0 + min(lane >> 2, cnt - 1)];
+    exact_sweep<T, 0>(p, l0, cnt, G(stage == 1 ? p.y1 : (p.scheme == SCHEME_HV ? p.y4 : p.y3)), ldg(u, jj),
+                      ldg(u, (uint32_t)(p.nx - 1) * (uint32_t)p.ny + jj));
+}
+
+// v-line sweep of tile (l0, cnt).  stage 1: rhs_v(u, Y1) -> Y2 (DR: next).  stage 2: CS/MCS rhs_v(u, Y3) -> next;
+// HV rhs_v(Y2, Y4) -> next.  Dirichlet ends colA0/colA1[idx1[i]]: the copy of `next` the vertical lambdas
+// captured after boundary stage A (implicit_kernel.hpp:69-84).
+template <typename T, int PAT>
+__device__ __forceinline__ void vsweep_rhs(const Prob<T> &p, int step, int stage, int l0, int cnt, int tid)
+{
+    const T *u = (step & 1) ? p.b : p.a;
+    const bool hv2 = stage == 2 && p.scheme == SCHEME_HV;
+    const gptr<const T> cA = G((const T *)p.colA0), cB = G((const T *)p.colA1);
+    exact_rhs<T, PAT, 4>(p, step, l0, cnt, G(hv2 ? (const T *)p.y2 : u),
+                    G((const T *)(stage == 1 ? p.y1 : (hv2 ? p.y4 : p.y3))), [&](int i) { return ldg(cA, p.idx1[i]); },
+                    [&](int i) { return ldg(cB, p.idx1[i]); }, tid);
+}
+template <typename T, int PAT>
+__device__ __forceinline__ void vsweep_solve(const Prob<T> &p, int step, int stage, bool fresh, int l0, int cnt)
+{
+    const int lane = (int)threadIdx.x & 63;
+    if (fresh)
+        exact_factor<T, PAT, 1>(p, step, l0, cnt);
+    const uint32_t ii = p.idx1[l0 + min(lane >> 2, cnt - 1)];
+    exact_sweep<T, 1>(p, l0, cnt, G((stage == 1 && p.scheme != SCHEME_DR) ? p.y2 : ((step & 1) ? p.a : p.b)),
+                      ldg((gptr<const T>)G(p.colA0), ii), ldg((gptr<const T>)G(p.colA1), ii));
+}
+
+// One tile per workgroup: its threads form the right-hand sides, its first wavefront sweeps; in
+// stage 1 of the S-sweep the other wavefronts evaluate the tile's share of boundary stage A meanwhile (the v-sweeps
+// read it), and in the step's last v-sweep the tile that holds rows nx - 2 and nx - 3 (the plan lays v-line tiles out
+// from the last row) evaluates boundary stage B.  Workgroups of 1024 threads, for fewer rounds of loads in the
+// right-hand sides, were slower also for one small problem (100 x 50 x 100 steps: 2.29 ms against 1.96), and a loop
+// that keeps the whole problem in one workgroup was as well (2.92 ms: the loads of the right-hand sides then go
+// through one CU's L1).
+template <typename T, int PAT>
+__global__ void __launch_bounds__(EXT) k_xsweep(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
+                                               int step, int stage, int fresh)
+{
+    const Tile tl = tiles[blockIdx.x];
+    const Prob<T> &p = probs[tl.prob];
+    if (step >= p.steps || (stage == 2 && p.scheme == SCHEME_DR))
+        return;  // uniform over the workgroup
+    const int tid = (int)threadIdx.x;
+    xsweep_rhs<T, PAT>(p, step, stage, tl.first, tl.count, tid);
+    __syncthreads();
+    if (tid < 64) {
+        xsweep_solve<T, PAT>(p, step, stage, stage == 1 && (fresh || p.coeff_sets > 1), tl.first, tl.count);
+    } else if (stage == 1) {
+        const int ntl = (p.ny - 2 + EXL - 1) / EXL, k = (tl.first - 1) / EXL;
+        for (int i = k * (EXT - 64) + tid - 64; i < p.nx; i += ntl * (EXT - 64))
+            bnd_a_row(p, step, i);
+    }
+}
+
+template <typename T, int PAT>
+__global__ void __launch_bounds__(EXT) k_vsweep(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
+                                               int step, int stage, int fresh)
+{
+    const Tile tl = tiles[blockIdx.x];
+    const Prob<T> &p = probs[tl.prob];
+    if (step >= p.steps || (stage == 2 && p.scheme == SCHEME_DR))
+        return;  // uniform over the workgroup
+    const int tid = (int)threadIdx.x;
+    vsweep_rhs<T, PAT>(p, step, stage, tl.first, tl.count, tid);
+    __syncthreads();
+    if (tid < 64)
+        vsweep_solve<T, PAT>(p, step, stage, stage == 1 && (fresh || p.coeff_sets > 1), tl.first, tl.count);
+    if ((stage == 2 || p.scheme == SCHEME_DR) && tl.first + tl.count == p.nx - 1) {  // uniform
+        __syncthreads();
+        for (int j = tid; j < p.ny; j += EXT)
+            bnd_b_col(p, step, j);
     }
 }
 
@@ -587,12 +661,12 @@ __global__ void __launch_bounds__(256) k_tridiag_lane(int64_t B, int n, int stri
 // -------------------------------------------------------------------------------------------------
 // explicit instantiations
 // -------------------------------------------------------------------------------------------------
+#define LSS_INST_EX(T, PAT)                                                                                   \
+    template __global__ void k_xsweep<T, PAT>(const Prob<T> *, const Tile *, int, int, int);                  \
+    template __global__ void k_vsweep<T, PAT>(const Prob<T> *, const Tile *, int, int, int);
 #define LSS_INST(T)                                                                                           \
-    template __global__ void k_bnd_a<T>(const Prob<T> *, const Tile *, int);                                  \
     template __global__ void k_bnd_b<T>(const Prob<T> *, const Tile *, int);                                  \
-    template __global__ void k_xsweep<T>(const Prob<T> *, const Tile *, int, int);                            \
-    template __global__ void k_vsweep<T>(const Prob<T> *, const Tile *, int, int);                            \
-    template __global__ void k_hv_y3<T>(const Prob<T> *, const Tile *, int);                                  \
+    LSS_INST_EX(T, PAT_GENERIC) LSS_INST_EX(T, PAT_FIELDS)                                                    \
     template __global__ void k_euler_res<T, PAT_GENERIC>(const Prob<T> *, const Tile *);                      \
     template __global__ void k_euler_res<T, PAT_HESTON>(const Prob<T> *, const Tile *);                       \
     template __global__ void k_euler_res<T, PAT_SABR0>(const Prob<T> *, const Tile *);                        \
@@ -604,5 +678,6 @@ __global__ void __launch_bounds__(256) k_tridiag_lane(int64_t B, int n, int stri
 LSS_INST(double)
 LSS_INST(float)
 #undef LSS_INST
+#undef LSS_INST_EX
 
 }  // namespace lssamd

@@ -15,7 +15,8 @@ template <typename T> struct Stencil {
 // and 2 are the patterns of the reference models' data (Heston with r != 0, SABR with r = 0), fixed
 // at compile time so that zero and unit factors cost nothing.  The plan selects a pattern only
 // when every problem has exactly its codes.
-enum : int32_t { PAT_GENERIC = 0, PAT_HESTON = 1, PAT_SABR0 = 2, PAT_COUNT = 3 };
+enum : int32_t { PAT_GENERIC = 0, PAT_HESTON = 1, PAT_SABR0 = 2, PAT_COUNT = 3,
+                 PAT_FIELDS = 4 };  // FIELDS coefficients, known at compile time (exact sweeps)
 template <int PAT> struct FPat;
 template <> struct FPat<PAT_HESTON> {
     static constexpr int c[24] = {0, -1, -2, -1, 1, -1, 2, 3, -2, -1, -2, -1,
@@ -111,7 +112,17 @@ template <typename T, int PAT = PAT_GENERIC, typename P>
 __device__ __forceinline__ Stencil<T> stencil_at(const Prob<T> &p, P cs, int i, int j)
 {
     Stencil<T> s;
-    if (PAT == PAT_GENERIC && p.coeff_mode == COEFF_FIELDS) {
+    if constexpr (PAT == PAT_FIELDS) {  // (each field at a 32-bit offset from a scalar base)
+        const uint32_t nxy = (uint32_t)p.nx * (uint32_t)p.ny, q = (uint32_t)i * (uint32_t)p.ny + (uint32_t)j;
+        auto field = [&](int k) { return ldg(cs + (size_t)k * nxy, q); };
+        s.M = field(0);
+        s.Mt = field(1);
+        s.P = field(2);
+        s.Pt = field(3);
+        s.Z = field(4);
+        s.W = field(5);
+        s.C = field(6);
+    } else if (PAT == PAT_GENERIC && p.coeff_mode == COEFF_FIELDS) {
         const int nxy = p.nx * p.ny, q = i * p.ny + j;
         s.M = cs[q];
         s.Mt = cs[nxy + q];

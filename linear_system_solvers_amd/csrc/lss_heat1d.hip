@@ -23,27 +23,12 @@
 #include "lss_capi_common.hpp"
 #include "lss_heat1d.h"
 #include "lss_heat1d_device.hpp"
+#include "lss_quad.hpp"
 
 namespace lssamd {
 
 template <typename T, int M>
 __global__ void k_h1_wave(const H1Prob<T> *, int, const T *const *, T *const *, T *const *);
-
-// Lane i of a quad takes lane (CTRL >> 2i) & 3's value (DPP quad_perm).
-template <int CTRL> __device__ __forceinline__ int quad_mov(int v)
-{
-    return __builtin_amdgcn_update_dpp(v, v, CTRL, 0xf, 0xf, true);
-}
-template <int CTRL> __device__ __forceinline__ float quad_perm(float v)
-{
-    return __int_as_float(quad_mov<CTRL>(__float_as_int(v)));
-}
-template <int CTRL> __device__ __forceinline__ double quad_perm(double v)
-{
-    return __hiloint2double(quad_mov<CTRL>(__double2hiint(v)), quad_mov<CTRL>(__double2loint(v)));
-}
-constexpr int QUAD_UP = 0x90, QUAD_DOWN = 0xf9;                      // lane q takes lane q - 1's / q + 1's
-template <int Q> constexpr int QUAD_BCAST = Q * 0x55;                // every lane takes lane Q's
 
 template <typename T> struct H1Vec {
     typedef T v2 __attribute__((ext_vector_type(2)));
@@ -82,11 +67,11 @@ __device__ __forceinline__ void finish_end(T (&x)[4], const T (&gm)[4], const T 
 // group.  Everything that does not depend on the previous point -- the loads, the rows of the theta scheme
 // and, once gamma is known, the divisors -- is formed by the four lanes at once; the recurrence of the
 // sweep then passes from lane to lane by DPP, each lane running its four points in the reference's order.
-// That chain (a multiplication, a subtraction and an IEEE division per point) bounds a wavefront; a large
-// book is bound by the 40 bytes of A, B, D and gamma (twice) that each point of each step reads: 16384
-// problems x 256 points x 1000 steps in fp64 take 29.4 ms, 5.7 TB/s from the last-level cache.  With one
-// lane per problem, each access in a cache line of its own, they took 304 ms (1.2 us a point).  Four lanes
-// make 1024 wavefronts of that book, one per SIMD.
+// What bounds a wavefront is the number of instructions of that chain and of the rows (it issues one every four to
+// five cycles), and a large book also the 40 bytes of A, B, D and gamma (twice) that each point of each step reads
+// from the last-level cache: 16384 problems x 256 points x 1000 steps in fp64 take 26.4 ms (29.4 with an IEEE
+// division per point), 6.4 TB/s.  With one lane per problem, each access in a cache line of its own, they took 304 ms.
+// Four lanes make 1024 wavefronts of that book, one per SIMD.
 //
 // Layouts: a problem's A, B and D are padded to whole groups (16-byte aligned), so a quad reads whole
 // 128-byte lines; the level u (LDS when it fits, else the workspace) and gamma (workspace) are kept by lane,
@@ -117,68 +102,70 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
     const bool fwd = P.direction == H1_FORWARD, has_src = P.src != nullptr;
     const bool const_gamma =
         P.coeff_sets == 1 && (P.bnd_sets == 1 || (P.lo_type != BC_ROBIN && P.hi_type != BC_ROBIN));
-    T *const gbase = P.gamma, *const ubase = P.level;
-    lptr<T> ush = (lptr<T>)h1_lds;
+    const gptr<T> gbase = G(P.gamma), ubase = G(P.level);
+    lptr<v2> ush = (lptr<v2>)h1_lds;
     // four own values of group g in the lane-ordered workspace / the level
-    auto ld4 = [&](const T *b, int g, T(&v)[4]) {
-        const v2 x = *(const v2 *)(b + ((size_t)(2 * g) * 64 + lane) * 2),
-                 y = *(const v2 *)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2);
+    auto ld4 = [&](gptr<T> b, int g, T(&v)[4]) {
+        const v2 x = *(gptr<const v2>)(b + ((size_t)(2 * g) * 64 + lane) * 2),
+                 y = *(gptr<const v2>)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2);
         v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
     };
-    auto st4 = [&](T *b, int g, const T(&v)[4]) {
-        *(v2 *)(b + ((size_t)(2 * g) * 64 + lane) * 2) = v2{v[0], v[1]};
-        *(v2 *)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2) = v2{v[2], v[3]};
+    auto st4 = [&](gptr<T> b, int g, const T(&v)[4]) {
+        *(gptr<v2>)(b + ((size_t)(2 * g) * 64 + lane) * 2) = v2{v[0], v[1]};
+        *(gptr<v2>)(b + ((size_t)(2 * g + 1) * 64 + lane) * 2) = v2{v[2], v[3]};
     };
     auto uget = [&](int g, T(&v)[4]) {
         if constexpr (LDSU) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                v[j] = ush[(4 * g + j) * 64 + lane];
+            const v2 p0 = ush[(2 * g) * 64 + lane], p1 = ush[(2 * g + 1) * 64 + lane];
+            v[0] = p0.x, v[1] = p0.y, v[2] = p1.x, v[3] = p1.y;
         } else {
             ld4(ubase, g, v);
         }
     };
     auto uput = [&](int g, const T(&v)[4]) {
         if constexpr (LDSU) {
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-                ush[(4 * g + j) * 64 + lane] = v[j];
+            ush[(2 * g) * 64 + lane] = v2{v[0], v[1]};
+            ush[(2 * g + 1) * 64 + lane] = v2{v[2], v[3]};
         } else {
             st4(ubase, g, v);
         }
     };
-    auto store_level = [&](T *row, int g, const T(&v)[4]) {
+    auto store_level = [&](gptr<T> row, int g, const T(&v)[4]) {
 #pragma unroll
         for (int j = 0; j < 4; ++j)
             if (16 * g + 4 * ql + j < n)
                 row[16 * g + 4 * ql + j] = v[j];
     };
-    T *sf = surf ? surf[p] : nullptr, *out = uout[p];
+    T *const sf0 = surf ? surf[p] : nullptr;
+    const gptr<T> sf = G(sf0), out = G(uout[p]);
     {
-        const T *in = uin[p];
+        const gptr<const T> in = G(uin[p]);
         for (int g = 0; g < ng; ++g) {
             T v[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j)
                 v[j] = in[min(16 * g + 4 * ql + j, N)];
             uput(g, v);
-            if (sf)
+            if (sf0)
                 store_level(sf + (size_t)(fwd ? 0 : steps) * n, g, v);
         }
     }
     struct Stage {
-        T A[4], B[4], D[4], G[4];
+        T A[4], B[4], D[4], G[4], u[4];
+    };
+    struct Back {
+        T G[4], s[4];
     };
     for (int st = 0; st < steps; ++st) {
-        const T *cs = P.coeff + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)ld;
-        const T *bs = P.bnd + (P.bnd_sets > 1 ? st : 0) * 4;
+        const gptr<const T> cs = G(P.coeff) + (size_t)(P.coeff_sets > 1 ? st : 0) * 3 * (size_t)ld;
+        const gptr<const T> bs = G(P.bnd) + (P.bnd_sets > 1 ? st : 0) * 4;
         const T lo_lin = bs[0], lo_val = bs[1], hi_lin = bs[2], hi_val = bs[3];
-        const T *src = has_src ? P.src + (size_t)st * 2 * (size_t)n : nullptr;
+        const gptr<const T> src = G(P.src) + (size_t)st * 2 * (size_t)n;
         const bool reuse = const_gamma && st > 0;  // gamma of this problem is in the workspace
         auto load = [&](int g, Stage &s) {
             const int o = 16 * g + 4 * ql;
-            auto two_of = [&](const T *b, T(&v)[4]) {
-                const v2 x = *(const v2 *)(b + o), y = *(const v2 *)(b + o + 2);
+            auto two_of = [&](gptr<const T> b, T(&v)[4]) {
+                const v2 x = *(gptr<const v2>)(b + o), y = *(gptr<const v2>)(b + o + 2);
                 v[0] = x.x, v[1] = x.y, v[2] = y.x, v[3] = y.y;
             };
             two_of(cs, s.A);
@@ -186,19 +173,14 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
             two_of(cs + 2 * ld, s.D);
             if (reuse)
                 ld4(gbase, g, s.G);
+            uget(g, s.u);
         };
         // ---- forward sweep: rows (a, b, c, f), gamma and the intermediate solution, which replaces the level
-        Stage s0, s1;
-        load(0, s0);
-        load(min(1, ng - 1), s1);
-        T uc[4], ulast = (T)0, glast = (T)0, gcar = (T)0, scar = (T)0;
-        uget(0, uc);
-        for (int g = 0; g < ng; ++g) {
-            Stage s2;
-            load(min(g + 2, ng - 1), s2);
+        T ulast = (T)0, glast = (T)0, scar = (T)0;
+        auto forward = [&](int g, Stage &s0) {
             T un[4];
             uget(min(g + 1, ng - 1), un);
-            T left = quad_perm<QUAD_UP>(uc[3]), right = quad_perm<QUAD_DOWN>(uc[0]);
+            T left = quad_perm<QUAD_UP>(s0.u[3]), right = quad_perm<QUAD_DOWN>(s0.u[0]);
             const T nfirst = quad_perm<QUAD_BCAST<0>>(un[0]);
             left = ql == 0 ? ulast : left;
             right = ql == 3 ? nfirst : right;
@@ -206,13 +188,13 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const T A = s0.A[j], B = s0.B[j], D = s0.D[j];
-                const T um = j > 0 ? uc[j - 1] : left, up = j < 3 ? uc[j + 1] : right;
+                const T um = j > 0 ? s0.u[j - 1] : left, up = j < 3 ? s0.u[j + 1] : right;
                 // rows of split (:200-210): low = -theta A, diag = 1 + 2 theta B, high = -theta D; interior
                 // right-hand side (:88-94)
                 a[j] = (-theta * A);
                 b[j] = (one + two * theta * B);
                 c[j] = (-theta * D);
-                f[j] = (D * omt * up) + ((one - two * B * omt) * uc[j]) + (A * omt * um);
+                f[j] = (D * omt * up) + ((one - two * B * omt) * s0.u[j]) + (A * omt * um);
             }
             const bool edge = g == 0 || 16 * g + 16 >= N;  // holds row 0, N - 1, N or points past the line
             if (edge || has_src) {
@@ -220,7 +202,7 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
                 for (int j = 0; j < 4; ++j) {
                     const int t = 16 * g + 4 * ql + j;
                     const T A = s0.A[j], B = s0.B[j], D = s0.D[j];
-                    const T um = j > 0 ? uc[j - 1] : left, up = j < 3 ? uc[j + 1] : right;
+                    const T um = j > 0 ? s0.u[j - 1] : left, up = j < 3 ? s0.u[j + 1] : right;
                     const T sr = has_src ? src[min(t, N)] : (T)0, srn = has_src ? src[n + min(t, N)] : (T)0;
                     if (t == 0) {
                         if (dlo) {  // the end value; row 1 then folds it as f - a lo
@@ -231,10 +213,10 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
                             const T beta = two * h * lo_val;
                             T r;
                             if (P.lo_type == BC_NEUMANN) {
-                                r = omt * beta * A + (one - two * omt * B) * uc[j] + omt * (A + D) * up;
+                                r = omt * beta * A + (one - two * omt * B) * s0.u[j] + omt * (A + D) * up;
                             } else {
                                 const T alpha = two * h * lo_lin;
-                                r = omt * beta * A + (one - omt * (two * B - alpha * A)) * uc[j] + omt * (A + D) * up;
+                                r = omt * beta * A + (one - omt * (two * B - alpha * A)) * s0.u[j] + omt * (A + D) * up;
                             }
                             if (has_src)
                                 r = r + theta * k * srn + omt * k * sr;
@@ -259,10 +241,10 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
                             const T delta = two * h * hi_val;
                             T r;
                             if (P.hi_type == BC_NEUMANN) {
-                                r = omt * (A + D) * um + (one - two * omt * B) * uc[j] - omt * delta * D;
+                                r = omt * (A + D) * um + (one - two * omt * B) * s0.u[j] - omt * delta * D;
                             } else {
                                 const T gamma = two * h * hi_lin;
-                                r = omt * (A + D) * um + (one - omt * (two * B + gamma * D)) * uc[j] -
+                                r = omt * (A + D) * um + (one - omt * (two * B + gamma * D)) * s0.u[j] -
                                     omt * delta * D;
                             }
                             if (has_src)
@@ -287,136 +269,70 @@ __global__ void __launch_bounds__(64) k_h1_exact(const H1Prob<T> *__restrict__ p
                     }
                 }
             }
-            // the chain: s = (f - a s) / (b - a gamma), gamma = c / (b - a gamma)
+            // gamma = c / beta and beta = b - a gamma, then the chain s = (f - a s) / beta
+            T beta[4], gm[4], y[4];
             if (reuse) {
                 const T gup = quad_perm<QUAD_UP>(s0.G[3]);
-                T beta[4];
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
-                    gp[j] = j > 0 ? s0.G[j - 1] : (ql == 0 ? glast : gup);
+                    gm[j] = s0.G[j];
+                    gp[j] = j > 0 ? s0.G[j > 0 ? j - 1 : 0] : (ql == 0 ? glast : gup);
                     beta[j] = b[j] - (a[j] * gp[j]);
-                }
-                auto run = [&](auto qq) {
-                    constexpr int Q = decltype(qq)::value;
-                    if (ql == Q) {
-                        T sv = scar;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j)
-                            x[j] = sv = (f[j] - (a[j] * sv)) / beta[j];
-                    }
-                    scar = quad_perm<QUAD_BCAST<Q>>(x[3]);
-                };
-                const T sprev = scar;
-                x[0] = x[1] = x[2] = x[3] = sprev;
-                run(std::integral_constant<int, 0>{});
-                run(std::integral_constant<int, 1>{});
-                run(std::integral_constant<int, 2>{});
-                run(std::integral_constant<int, 3>{});
-                if (edge) {
-                    const T xup = quad_perm<QUAD_UP>(x[3]);
-                    finish_end(x, s0.G, gp, ql == 0 ? sprev : xup, 16 * g + 4 * ql, N, dhi, dsweep, P.hi_type, h, hi_lin,
-                               hi_val);
                 }
                 glast = quad_perm<QUAD_BCAST<3>>(s0.G[3]);
             } else {
-                T gm[4];
-                const T sprev = scar;
-                x[0] = x[1] = x[2] = x[3] = sprev;
-                gm[0] = gm[1] = gm[2] = gm[3] = gcar;
-                gp[0] = gp[1] = gp[2] = gp[3] = gcar;
-                auto run = [&](auto qq) {
-                    constexpr int Q = decltype(qq)::value;
-                    if (ql == Q) {
-                        T sv = scar, gv = gcar;
+                const T gnext = quad_gamma(a, b, c, glast, beta, gm);
+                const T gup = quad_perm<QUAD_UP>(gm[3]);
 #pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            gp[j] = gv;
-                            const T beta = b[j] - (a[j] * gv);
-                            gm[j] = gv = c[j] / beta;
-                            x[j] = sv = (f[j] - (a[j] * sv)) / beta;
-                        }
-                    }
-                    scar = quad_perm<QUAD_BCAST<Q>>(x[3]);
-                    gcar = quad_perm<QUAD_BCAST<Q>>(gm[3]);
-                };
-                run(std::integral_constant<int, 0>{});
-                run(std::integral_constant<int, 1>{});
-                run(std::integral_constant<int, 2>{});
-                run(std::integral_constant<int, 3>{});
+                for (int j = 0; j < 4; ++j)
+                    gp[j] = j > 0 ? gm[j > 0 ? j - 1 : 0] : (ql == 0 ? glast : gup);
+                glast = gnext;
                 st4(gbase, g, gm);
-                if (edge) {
-                    const T xup = quad_perm<QUAD_UP>(x[3]);
-                    finish_end(x, gm, gp, ql == 0 ? sprev : xup, 16 * g + 4 * ql, N, dhi, dsweep, P.hi_type, h, hi_lin,
-                               hi_val);
-                }
             }
-            uput(g, x);
-            ulast = quad_perm<QUAD_BCAST<3>>(uc[3]);
 #pragma unroll
             for (int j = 0; j < 4; ++j)
-                uc[j] = un[j];
-            s0 = s1;
-            s1 = s2;
-        }
-        // ---- back substitution x = s - gamma x, from the last group down
-        T *lv = sf ? sf + (size_t)(fwd ? st + 1 : steps - 1 - st) * n : nullptr;
-        T g0[4], g1[4], sc[4], xcar = (T)0;
-        ld4(gbase, ng - 1, g0);
-        ld4(gbase, max(ng - 2, 0), g1);
-        uget(ng - 1, sc);
-        for (int g = ng - 1; g >= 0; --g) {
-            T g2[4], sn[4], x[4];
-            ld4(gbase, max(g - 2, 0), g2);
-            uget(max(g - 1, 0), sn);
-            x[0] = x[1] = x[2] = x[3] = xcar;
-            if (g == 0 || 16 * g + 16 >= N) {
-                auto run = [&](auto qq) {
-                    constexpr int Q = decltype(qq)::value;
-                    if (ql == Q) {
-                        T xv = xcar;
-#pragma unroll
-                        for (int j = 3; j >= 0; --j) {
-                            const int t = 16 * g + 4 * ql + j;
-                            // the forward sweep left the value itself at row N, at a Dirichlet row 0 and at
-                            // the Thomas sweep's last row before a Dirichlet end
-                            const bool own = t >= N || (t == 0 && dlo) || (t == N - 1 && dhi && !dsweep);
-                            x[j] = xv = own ? sc[j] : (sc[j] - (g0[j] * xv));
-                        }
-                    }
-                    xcar = quad_perm<QUAD_BCAST<Q>>(x[0]);
-                };
-                run(std::integral_constant<int, 3>{});
-                run(std::integral_constant<int, 2>{});
-                run(std::integral_constant<int, 1>{});
-                run(std::integral_constant<int, 0>{});
-            } else {
-                auto run = [&](auto qq) {
-                    constexpr int Q = decltype(qq)::value;
-                    if (ql == Q) {
-                        T xv = xcar;
-#pragma unroll
-                        for (int j = 3; j >= 0; --j)
-                            x[j] = xv = sc[j] - (g0[j] * xv);
-                    }
-                    xcar = quad_perm<QUAD_BCAST<Q>>(x[0]);
-                };
-                run(std::integral_constant<int, 3>{});
-                run(std::integral_constant<int, 2>{});
-                run(std::integral_constant<int, 1>{});
-                run(std::integral_constant<int, 0>{});
+                y[j] = quick_rcp(beta[j]);
+            const T sprev = scar;
+            SeenNum seen;
+            scar = quad_forward<true>(a, f, beta, y, sprev, x, seen);
+            if (__builtin_amdgcn_ballot_w64(!seen_ok(seen, sprev)))
+                scar = quad_forward<false>(a, f, beta, y, sprev, x, seen);
+            if (edge) {
+                const T xup = quad_perm<QUAD_UP>(x[3]);
+                finish_end(x, gm, gp, ql == 0 ? sprev : xup, 16 * g + 4 * ql, N, dhi, dsweep, P.hi_type, h, hi_lin, hi_val);
             }
             uput(g, x);
-            if (lv)
+            ulast = quad_perm<QUAD_BCAST<3>>(s0.u[3]);
+        };
+        quad_stages<Stage>(0, ng, 1, load, forward);
+        // ---- back substitution x = s - gamma x, from the last group down
+        const gptr<T> lv = sf + (size_t)(fwd ? st + 1 : steps - 1 - st) * n;
+        T xcar = (T)0;
+        auto loadb = [&](int g, Back &b) {
+            ld4(gbase, g, b.G);
+            uget(g, b.s);
+        };
+        auto backward = [&](int g, Back &b) {
+            T x[4];
+            if (g == 0 || 16 * g + 16 >= N)
+                // the forward sweep left the value itself at row N, at a Dirichlet row 0 and at the Thomas sweep's
+                // last row before a Dirichlet end
+                xcar = quad_backward_ends(
+                    b.G, b.s, xcar, x,
+                    [&](int j) {
+                        const int t = 16 * g + 4 * ql + j;
+                        return t >= N || (t == 0 && dlo) || (t == N - 1 && dhi && !dsweep);
+                    },
+                    [](int) { return false; });
+            else
+                xcar = quad_backward(b.G, b.s, xcar, x);
+            uput(g, x);
+            if (sf0)
                 store_level(lv, g, x);
             if (st == steps - 1)
                 store_level(out, g, x);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                g0[j] = g1[j];
-                g1[j] = g2[j];
-                sc[j] = sn[j];
-            }
-        }
+        };
+        quad_stages<Back>(ng - 1, ng, -1, loadb, backward);
     }
 }
 

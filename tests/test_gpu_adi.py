@@ -331,3 +331,44 @@ def test_graph_groups_of_a_large_plan_equal_direct_launches(oracle):
         c = oracle_solve(oracle, models[q])
         assert _normwise(res[1][q], c) <= 1e-12
     plan.close()
+
+
+# ---------------------------------------------------------------------------------------------
+# The exact sweeps take lines in groups of 16 points and tiles of 16 lines, and divide by known divisors
+# without an IEEE division where the exponents allow it.  Sizes around those edges, both operation orders, both
+# coefficient forms side by side, and initial surfaces whose values are huge, tiny, negative zero or subnormal:
+# every bit (signs of zeros included) must be the oracle's.
+# ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("nx,ny", [(4, 4), (17, 18), (18, 19), (19, 34), (34, 35), (50, 17), (35, 66)])
+def test_exact_sweeps_equal_the_oracle_at_their_edges(oracle, fp, nx, ny):
+    ofp = "f64" if fp == L.FP64 else "f32"
+    models = [config0(nx=nx, ny=ny, nt=5, splitting=s, tridiagonal=tri, implicit_scheme=L.THETA_80, weighting=0.3)
+              for s in range(4) for tri in (L.THOMAS_LU, L.DOUBLE_SWEEP)]
+    plan = L.Plan.from_models(models, fp)
+    outs = plan.run_host()
+    for m, g in zip(models, outs):
+        c = oracle_solve(oracle, m, ofp)
+        assert np.array_equal(g, c) and np.array_equal(np.signbit(g), np.signbit(c)), (m.splitting, m.tridiagonal)
+    plan.close()
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("scale", [1.0, 0.0, -0.0, 1e-30, 1e-300, 1e-310, 1e30, 1e300])
+def test_exact_sweeps_keep_the_rounding_at_any_magnitude(oracle, fp, scale):
+    # the two operation orders and two tile positions of the same problem step the same surface: the loop is linear
+    # and its coefficients do not see the scale, so the sweeps of both halves of the book must agree with a plan that
+    # forms gamma anew (fresh) in every step, i.e. one step per run, bit for bit
+    dt = L.np_dtype(fp)
+    m = config0(nx=37, ny=21, nt=4, splitting=L.CRAIG_SNEYD)
+    one = config0(nx=37, ny=21, nt=2, splitting=L.CRAIG_SNEYD, t_hi=1.0 / 3.0, maturity=1.0)
+    plan, single = L.Plan.from_models([m], fp), L.Plan.from_models([one], fp)
+    rng = np.random.default_rng(3)
+    with np.errstate(over="ignore", under="ignore"):
+        u = (rng.standard_normal((37, 21)) * scale).astype(dt)
+    levels = plan.run_levels_host([u])[0]
+    for s in range(3):
+        nxt = single.run_host([levels[s]])[0]
+        assert np.array_equal(nxt, levels[s + 1], equal_nan=True)
+    plan.close()
+    single.close()

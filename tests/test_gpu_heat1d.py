@@ -249,3 +249,28 @@ def test_every_form_of_the_exact_kernel_equals_the_oracle(oracle, fp, sizes):
             assert np.array_equal(outs[z], out), (z, q["n"], q["tri"], q["lo"], q["hi"])
             assert np.array_equal(surfs[z], surf), (z, q["n"])
     plan.close()
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("scale", [0.0, -0.0, 1e-25, 1e-42, 1e-280, 1e-305, 1e-318, 1e30, 1e295])
+def test_exact_kernel_rounds_like_the_oracle_at_any_magnitude(oracle, fp, scale):
+    # the sweep divides by known divisors without an IEEE division where the exponents allow it; zeros of either
+    # sign, subnormal, tiny and huge levels (each also mixed with ordinary values) take every way out of that
+    import ctypes
+    rng = np.random.default_rng(17)
+    dt, descr = L.np_dtype(fp), []
+    for z in range(24):
+        q = _descr(ctypes, fp, 20 + 3 * z, 3, (L.THOMAS_LU, L.DOUBLE_SWEEP)[z % 2], z % 3, (z // 3) % 3, L.FORWARD, 0, 0, 0,
+                   0.5, rng)
+        with np.errstate(over="ignore", under="ignore"):
+            keep = rng.uniform(size=q["n"]) < (0.0 if z % 4 else 0.3)
+            q["u0"] = np.where(keep, q["u0"], (q["u0"].astype(np.float64) * scale).astype(dt)).astype(dt)
+            q["bnd"] = (q["bnd"].astype(np.float64) * (scale if z % 5 else 1.0)).astype(dt)
+        descr.append(q)
+    plan = _described_plan(ctypes, descr, L.LINE_EXACT)
+    outs = plan.run_host([q["u0"] for q in descr])
+    for z, q in enumerate(descr):
+        with np.errstate(all="ignore"):
+            out = _stepped(oracle, q)[1]
+        assert np.array_equal(outs[z], out, equal_nan=True), (z, q["n"])
+    plan.close()
