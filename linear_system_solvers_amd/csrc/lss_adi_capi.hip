@@ -32,7 +32,7 @@ template <typename T> __global__ void k_bnd_b(const Prob<T> *, const Tile *, int
 template <typename T, int PAT> __global__ void k_xsweep(const Prob<T> *, const Tile *, int, int, int);
 template <typename T, int PAT> __global__ void k_vsweep(const Prob<T> *, const Tile *, int, int, int);
 template <typename T, int PAT> __global__ void k_euler(const Prob<T> *, const Tile *, int);
-template <typename T, int PAT> __global__ void k_euler_res(const Prob<T> *, const Tile *);
+template <typename T, int PAT, int K> __global__ void k_euler_res(const Prob<T> *, const Tile *);
 template <typename T>
 __global__ void k_tridiag_lane(int64_t, int, int, const T *, const T *, const T *, const T *, T *, T *, LineBC<T>);
 template <typename T, int M, int STAGE, int W, int PAT, int NC>
@@ -183,6 +183,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     bool tuned = false;                // the autotuner has chosen xw and vr
     bool adj_ok = false;               // every line fits the partitioned solver (needed by the adjoint)
     bool euler = false;                // explicit Euler plan (no line sweeps)
+    int eres_rows = 10;                // rows per strip of k_euler_res
     bool euler_res = false;            // ... whose problems all fit k_euler_res (the loop resident in LDS)
     bool all_fields = true;            // every problem has FIELDS coefficients
     hipStream_t cap_stream = nullptr;
@@ -299,8 +300,17 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         euler_res = euler;
         for (int64_t q = 0; q < n; ++q)
             euler_res = euler_res && descs[q].nx >= 4 && descs[q].ny <= ERES_T &&
-                        descs[q].nx * descs[q].ny <= (int64_t)ERES_T * ERES_K && descs[q].coeff_sets == 1 &&
+                        descs[q].nx * descs[q].ny <= (int64_t)ERES_POINTS && descs[q].coeff_sets == 1 &&
                         descs[q].bnd_sets == 1;
+        // rows per strip: the least for which every problem's strips have a thread each (10 always does within
+        // ERES_POINTS points: the columns of more than 128 interior points have at most 9 rows)
+        for (int k : {10, 8, 6}) {
+            bool fits = true;
+            for (int64_t q = 0; q < n && euler_res; ++q)
+                fits = fits && (descs[q].nx - 2 + k - 1) / k * (descs[q].ny - 2) <= ERES_T;
+            if (fits)
+                eres_rows = k;
+        }
         for (int64_t q = 0; q < n; ++q)
             all_fields = all_fields && descs[q].coeff_mode == LSS_COEFF_FIELDS;
         {
@@ -1400,6 +1410,15 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         }
     }
 
+    template <int K> void launch_euler_res_k(dim3 g, dim3 b, hipStream_t st, const Prob<T> *pd, const Tile *tp)
+    {
+        if (fpat == PAT_HESTON)
+            hipLaunchKernelGGL((k_euler_res<T, PAT_HESTON, K>), g, b, 0, st, pd, tp);
+        else if (fpat == PAT_SABR0)
+            hipLaunchKernelGGL((k_euler_res<T, PAT_SABR0, K>), g, b, 0, st, pd, tp);
+        else
+            hipLaunchKernelGGL((k_euler_res<T, PAT_GENERIC, K>), g, b, 0, st, pd, tp);
+    }
     // every step of every problem of a plan of small explicit Euler problems (euler_res), the levels
     // resident in LDS; the result is where the step-by-step loop leaves it
     void launch_euler_res(hipStream_t st)
@@ -1407,12 +1426,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         const Prob<T> *pd = (const Prob<T> *)probs_dev.p;
         const Tile *tp = (const Tile *)tiles_dev.p + tile_off[TB_P];
         const dim3 g((unsigned)count), b(ERES_T);
-        if (fpat == PAT_HESTON)
-            hipLaunchKernelGGL((k_euler_res<T, PAT_HESTON>), g, b, 0, st, pd, tp);
-        else if (fpat == PAT_SABR0)
-            hipLaunchKernelGGL((k_euler_res<T, PAT_SABR0>), g, b, 0, st, pd, tp);
+        if (eres_rows == 6)
+            launch_euler_res_k<6>(g, b, st, pd, tp);
+        else if (eres_rows == 8)
+            launch_euler_res_k<8>(g, b, st, pd, tp);
         else
-            hipLaunchKernelGGL((k_euler_res<T, PAT_GENERIC>), g, b, 0, st, pd, tp);
+            launch_euler_res_k<10>(g, b, st, pd, tp);
         HIPCHK(hipGetLastError());
     }
 

@@ -129,7 +129,7 @@ constexpr int GTR = 8, GTC = 32;  // explicit step: GTR x GTC threads, each ERPT
 // (AGT = (AGR + 2) x (AGC + 2) = 512), so that every equation point is formed in one pass
 constexpr int AGR = 14, AGC = 30, AGT = (AGR + 2) * (AGC + 2);
 constexpr int ERPT = 8;           // rows per thread of the explicit step (its tiles: GTR * ERPT rows)
-constexpr int ERES_T = 256, ERES_K = 6;  // threads and points per thread of the resident explicit loop
+constexpr int ERES_T = 256, ERES_POINTS = 1536;  // threads and points of the resident explicit loop
 
 // v-lines per wavefront of the partitioned v-sweep for lines of N interior points and the plan's
 // chunk bound M: 2 when the line fits 32 chunks of at most M <= 4 points, else 1 (the plan's v-line

@@ -495,112 +495,134 @@ __global__ void __launch_bounds__(GTR *GTC) k_euler(const Prob<T> *__restrict__ 
 // time levels resident in LDS (lss_heston_euler_solver_scheme.hpp:63-67, 78-83).  Per step: the
 // interior and boundary stage A from the old level into the new one; a barrier; boundary stage B (row 0,
 // and row nx - 1 extrapolated from rows nx - 2 and nx - 3 of the new level, as the reference reads
-// them); a barrier.  Every value takes the arithmetic of k_euler in the same order.  The thread's
-// points are numbered interior first, then the v = 0 column, then the v_max column, so that the
-// wavefronts mostly take one branch; their stencil weights and boundary values are formed once (the
-// problems have one coefficient set and one boundary set).  For problems of at most ERES_T * ERES_K
-// points with nx >= 4 and ny <= ERES_T; HBM is read once and written once.
+// them); a barrier.  Every value takes the arithmetic of k_euler in the same order.
+//
+// A thread holds a strip of K consecutive rows of one column: its stencil weights, formed once (one coefficient
+// set and one boundary set), and its column's values stay in registers, so that per strip and step it reads
+// 2 K + 6 values from LDS and writes K (K = 6: 4 accesses a point; a thread per point, scattered, takes 10, which
+// bound the loop by LDS bandwidth: 1024 problems 50 x 30, 7999 steps in fp64 19.0 ms at 52 TB/s against 11.0 ms at 36
+// with strips; the v = 0 weights in LDS instead of registers: 11.4 ms).  Strips of columns
+// with at least K interior rows overlap at the bottom instead of ending early (both compute the same values);
+// shorter columns mask.  Values that do not change from step to step (row 0, column ny - 1) are written in the
+// first two steps only.  For problems of at most ERES_POINTS points with nx >= 4 and ny <= ERES_T: then some K of 6,
+// 8 and 10 gives every strip a thread.  HBM is read once and written once.
 // -------------------------------------------------------------------------------------------------
-template <typename T, int PAT>
-__global__ void __launch_bounds__(ERES_T) __attribute__((amdgpu_waves_per_eu(4)))
+template <typename T, int PAT, int K>
+__global__ void __launch_bounds__(ERES_T) __attribute__((amdgpu_waves_per_eu(K <= 6 ? 4 : 2)))
 k_euler_res(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles)
 {
-    __shared__ T lv[2][ERES_T * ERES_K];
+    __shared__ T lv[2][ERES_POINTS];
     const Tile tl = tiles[blockIdx.x];
     const Prob<T> &p = probs[tl.prob];
     const int nx = p.nx, ny = p.ny, n = nx * ny, steps = p.steps, tid = (int)threadIdx.x;
-    const int ni_ = (nx - 2) * (ny - 2), na = ni_ + (nx - 2);  // interior points, then the v = 0 column
     const T one = (T)1.0, two = (T)2.0, three = (T)3.0, four = (T)4.0;
     {
         const gptr<const T> a = G((const T *)p.a);
         for (int q = tid; q < n; q += ERES_T)
             lv[0][q] = a[q];
     }
-    // the thread's points: pt = kind << 16 | (r * ny + c); kind 1 interior, 2 v = 0, 3 v_max, 0 none
-    int pt[ERES_K];
+    const gptr<const T> cs = coeff_set(p, 0);
+    const gptr<const T> bs = bnd_set(p, 0);
+    // the thread's strip: rows r0 .. r0 + nv - 1 of column c
+    const int cols = ny - 2, rows = nx - 2, nst = (rows + K - 1) / K;
+    const bool strip = tid < nst * cols;
+    const int c = strip ? 1 + tid % cols : 1, sr = strip ? tid / cols : 0;
+    const int nv = min(K, rows), r0 = 1 + min(sr * K, rows - nv), o0 = r0 * ny + c;
+    T wt[K][6];  // C, M, M~, 1 - Z - W, P~, P (C = gamma c)
 #pragma unroll
-    for (int k = 0; k < ERES_K; ++k) {
-        const int e = tid + k * ERES_T;
-        int r = 0, c = 0, kd = 0;
-        if (e < ni_) {
-            r = 1 + e / (ny - 2);
-            c = 1 + e % (ny - 2);
-            kd = 1;
-        } else if (e < na) {
-            r = 1 + (e - ni_);
-            kd = 2;
-        } else if (e < na + (nx - 2)) {
-            r = 1 + (e - na);
-            c = ny - 1;
-            kd = 3;
-        }
-        pt[k] = kd << 16 | (r * ny + c);
+    for (int j = 0; j < K; ++j) {
+        const Stencil<T> st = stencil_at<T, PAT>(p, cs, min(r0 + j, nx - 2), c);
+        wt[j][0] = p.gamma * st.C;
+        wt[j][1] = st.M;
+        wt[j][2] = st.Mt;
+        wt[j][3] = one - st.Z - st.W;
+        wt[j][4] = st.Pt;
+        wt[j][5] = st.P;
     }
-    // interior: C, M, M~, 1 - Z - W, P~, P (C = gamma c); v = 0: -delta D, 1 - 3 ni E + rho F, delta D,
-    // ni E, 4 ni E; v_max: the boundary value
-    T wt[ERES_K][6];
+    // the v = 0 points of rows 1 + k, from the last thread down: -delta D, 1 - 3 ni E + rho F, delta D, ni E, 4 ni E
+    constexpr int NV0 = (ERES_POINTS / 4 + ERES_T - 1) / ERES_T;
+    T w0[NV0][5];
+#pragma unroll
+    for (int k = 0; k < NV0; ++k) {
+        T D, E, F;
+        def_row0<T, PAT>(p, cs, min(1 + ERES_T - 1 - tid + k * ERES_T, nx - 2), D, E, F);
+        const T delta = p.delta, ni = p.ni, rho = p.rho;
+        w0[k][0] = -delta * D;
+        w0[k][1] = one - three * ni * E + rho * F;
+        w0[k][2] = delta * D;
+        w0[k][3] = ni * E;
+        w0[k][4] = four * ni * E;
+    }
     T lo_j = (T)0, hup_j = (T)0;  // boundary stage B of column tid: h_lower and 2 h_1 h_upper X'(1)
     int jj = 0;
-    {
-        const gptr<const T> cs = coeff_set(p, 0);
-        const gptr<const T> bs = bnd_set(p, 0);
-#pragma unroll
-        for (int k = 0; k < ERES_K; ++k) {
-            const int kd = pt[k] >> 16, o = pt[k] & 0xffff, r = o / ny, c = o - r * ny;
-            if (kd == 1) {
-                const Stencil<T> st = stencil_at<T, PAT>(p, cs, r, c);
-                wt[k][0] = p.gamma * st.C;
-                wt[k][1] = st.M;
-                wt[k][2] = st.Mt;
-                wt[k][3] = one - st.Z - st.W;
-                wt[k][4] = st.Pt;
-                wt[k][5] = st.P;
-            } else if (kd == 2) {
-                T D, E, F;
-                def_row0<T, PAT>(p, cs, r, D, E, F);
-                const T delta = p.delta, ni = p.ni, rho = p.rho;
-                wt[k][0] = -delta * D;
-                wt[k][1] = one - three * ni * E + rho * F;
-                wt[k][2] = delta * D;
-                wt[k][3] = ni * E;
-                wt[k][4] = four * ni * E;
-            } else if (kd == 3) {
-                wt[k][0] = bs[r];  // v_upper(t, X(zeta_r))
-            }
-        }
-        if (tid < ny) {
-            lo_j = bs[nx + tid];  // h_lower(t, Y(eta_j))
-            hup_j = two * p.h1 * bs[nx + ny + tid];
-            jj = (int)p.idx2[tid];
-        }
+    if (tid < ny) {
+        lo_j = bs[nx + tid];  // h_lower(t, Y(eta_j))
+        hup_j = two * p.h1 * bs[nx + ny + tid];
+        jj = (int)p.idx2[tid];
     }
     __syncthreads();
-    for (int s = 0; s < steps; ++s) {
-        const T *u = lv[s & 1];
-        T *w = lv[(s & 1) ^ 1];
+    T own[K];
 #pragma unroll
-        for (int k = 0; k < ERES_K; ++k) {
-            const int kd = pt[k] >> 16, o = pt[k] & 0xffff;
-            if (kd == 1) {
-                const T C = wt[k][0];
-                w[o] = C * u[o - ny - 1] + wt[k][1] * u[o - ny] - C * u[o - ny + 1] + wt[k][2] * u[o - 1] +
-                       wt[k][3] * u[o] + wt[k][4] * u[o + 1] - C * u[o + ny - 1] + wt[k][5] * u[o + ny] +
-                       C * u[o + ny + 1];
-            } else if (kd == 2) {
-                w[o] = (wt[k][0] * u[o - ny]) + (wt[k][1] * u[o]) + (wt[k][2] * u[o + ny]) - (wt[k][3] * u[o + 2]) +
-                       (wt[k][4] * u[o + 1]);
-            } else if (kd == 3) {
-                w[o] = wt[k][0];
+    for (int j = 0; j < K; ++j)
+        own[j] = lv[0][o0 + min(j, nv - 1) * ny];
+    auto loop = [&](auto full) {
+        constexpr bool FULL = decltype(full)::value;  // the strip has K rows
+        for (int s = 0; s < steps; ++s) {
+            const T *u = lv[s & 1];
+            T *w = lv[(s & 1) ^ 1];
+            if (strip) {
+                const T *q = u + o0;
+                const T bot = q[nv * ny];
+                // column above, at and below the current row, and its neighbours' values
+                T um = q[-ny], lm = q[-ny - 1], rm = q[-ny + 1], l0 = q[-1], r0v = q[1];
+                T nw[K];
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    const int jd = FULL ? j + 1 : min(j + 1, nv);
+                    const T lp = q[jd * ny - 1], rp = q[jd * ny + 1];
+                    const T up = FULL ? (j + 1 < K ? own[j + 1 < K ? j + 1 : 0] : bot)
+                                      : (j + 1 < nv ? own[j + 1 < K ? j + 1 : 0] : bot);
+                    const T C = wt[j][0];
+                    nw[j] = C * lm + wt[j][1] * um - C * rm + wt[j][2] * l0 + wt[j][3] * own[j] + wt[j][4] * r0v - C * lp +
+                            wt[j][5] * up + C * rp;
+                    um = own[j];
+                    lm = l0;
+                    rm = r0v;
+                    l0 = lp;
+                    r0v = rp;
+                }
+#pragma unroll
+                for (int j = 0; j < K; ++j) {
+                    if (FULL || j < nv)
+                        w[o0 + j * ny] = nw[j];
+                    own[j] = nw[j];
+                }
             }
+#pragma unroll
+            for (int k = 0; k < NV0; ++k) {
+                const int r = 1 + ERES_T - 1 - tid + k * ERES_T;
+                if (r <= nx - 2) {
+                    const T *q = u + r * ny;
+                    w[r * ny] = (w0[k][0] * q[-ny]) + (w0[k][1] * q[0]) + (w0[k][2] * q[ny]) - (w0[k][3] * q[2]) +
+                                (w0[k][4] * q[1]);
+                }
+            }
+            if (s < 2) {
+                for (int r = 1 + tid; r <= nx - 2; r += ERES_T)
+                    w[r * ny + ny - 1] = bs[r];  // v_upper(t, X(zeta_r))
+                if (tid < ny)
+                    w[tid] = lo_j;
+            }
+            __syncthreads();
+            if (tid < ny)
+                w[(nx - 1) * ny + tid] = (((four * w[(nx - 2) * ny + jj]) - w[(nx - 3) * ny + jj] - hup_j) / three);
+            __syncthreads();
         }
-        __syncthreads();
-        if (tid < ny) {
-            const T e = (((four * w[(nx - 2) * ny + jj]) - w[(nx - 3) * ny + jj] - hup_j) / three);
-            w[tid] = lo_j;
-            w[(nx - 1) * ny + tid] = e;
-        }
-        __syncthreads();
-    }
+    };
+    if (rows >= K)
+        loop(std::true_type{});
+    else
+        loop(std::false_type{});
     const gptr<T> out = G((steps & 1) ? p.b : p.a);
     for (int q = tid; q < n; q += ERES_T)
         out[q] = lv[steps & 1][q];
@@ -664,12 +686,14 @@ __global__ void __launch_bounds__(256) k_tridiag_lane(int64_t B, int n, int stri
 #define LSS_INST_EX(T, PAT)                                                                                   \
     template __global__ void k_xsweep<T, PAT>(const Prob<T> *, const Tile *, int, int, int);                  \
     template __global__ void k_vsweep<T, PAT>(const Prob<T> *, const Tile *, int, int, int);
+#define LSS_INST_ERES(T, PAT)                                                                                 \
+    template __global__ void k_euler_res<T, PAT, 6>(const Prob<T> *, const Tile *);                           \
+    template __global__ void k_euler_res<T, PAT, 8>(const Prob<T> *, const Tile *);                           \
+    template __global__ void k_euler_res<T, PAT, 10>(const Prob<T> *, const Tile *);
 #define LSS_INST(T)                                                                                           \
     template __global__ void k_bnd_b<T>(const Prob<T> *, const Tile *, int);                                  \
     LSS_INST_EX(T, PAT_GENERIC) LSS_INST_EX(T, PAT_FIELDS)                                                    \
-    template __global__ void k_euler_res<T, PAT_GENERIC>(const Prob<T> *, const Tile *);                      \
-    template __global__ void k_euler_res<T, PAT_HESTON>(const Prob<T> *, const Tile *);                       \
-    template __global__ void k_euler_res<T, PAT_SABR0>(const Prob<T> *, const Tile *);                        \
+    LSS_INST_ERES(T, PAT_GENERIC) LSS_INST_ERES(T, PAT_HESTON) LSS_INST_ERES(T, PAT_SABR0)                    \
     template __global__ void k_euler<T, PAT_GENERIC>(const Prob<T> *, const Tile *, int);                     \
     template __global__ void k_euler<T, PAT_HESTON>(const Prob<T> *, const Tile *, int);                      \
     template __global__ void k_euler<T, PAT_SABR0>(const Prob<T> *, const Tile *, int);                       \
@@ -679,5 +703,6 @@ LSS_INST(double)
 LSS_INST(float)
 #undef LSS_INST
 #undef LSS_INST_EX
+#undef LSS_INST_ERES
 
 }  // namespace lssamd

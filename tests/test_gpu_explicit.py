@@ -133,3 +133,22 @@ def test_plans_outside_the_residency_limits_step_launch_by_launch(oracle):
         g = plan.run_host()[0]
         plan.close()
         assert np.array_equal(g, oracle_solve(oracle, m))
+
+
+# shapes around the strips of the resident loop: columns shorter than a strip, strips that overlap at the bottom, the
+# most columns, the most rows, shapes that need 8 and 10 rows per strip, and several of them in one plan
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("shapes", [[(4, 4)], [(5, 30), (8, 9), (9, 9)], [(50, 30)], [(6, 256)], [(384, 4)], [(11, 139)],
+                                    [(16, 96)], [(13, 7), (50, 30), (11, 130), (200, 7)]])
+def test_resident_strips_equal_the_oracle(oracle, fp, shapes):
+    models = []
+    for q, (nx, ny) in enumerate(shapes):
+        m = model_from_case(EXPLICIT[0])
+        steps = 9 + q  # (odd and even: the result ends in either level)
+        m.nx, m.ny, m.nt, m.t_hi = nx, ny, steps + 1, m.t_hi * steps / (m.nt - 1)
+        models.append(m)
+    plan = L.Plan.from_models(models, fp)
+    assert plan.kernel_config()["explicit_resident"] == 1
+    for m, g in zip(models, plan.run_host()):
+        assert np.array_equal(g, oracle_solve(oracle, m, "f64" if fp == L.FP64 else "f32")), (m.nx, m.ny)
+    plan.close()
