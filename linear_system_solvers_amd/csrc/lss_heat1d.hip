@@ -29,6 +29,8 @@ namespace lssamd {
 
 template <typename T, int M>
 __global__ void k_h1_wave(const H1Prob<T> *, int, const T *const *, T *const *, T *const *);
+template <typename T, int M>
+__global__ void k_h1_wave_fixed(const H1Prob<T> *, int, const T *const *, T *const *, T *const *);
 
 template <typename T> struct H1Vec {
     typedef T v2 __attribute__((ext_vector_type(2)));
@@ -367,6 +369,7 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
     int ngmax = 0;           // groups of 16 points of the longest line
     bool lds_level = false;  // the level of every problem stays in LDS
     int pm = 1;  // chunk bound of the partitioned kernel
+    bool fixed = true;  // no problem's matrix changes in time
     std::vector<const void *> table;  // u_in, u_out, surfaces pointers of the last device run
     bool table_valid = false;
 
@@ -409,6 +412,8 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
             const int64_t nu = d[q].n - (d[q].lo_type == LSS_BC_DIRICHLET) - (d[q].hi_type == LSS_BC_DIRICHLET);
             while (pm * 64 < nu && pm < 16)
                 pm *= 2;
+            const bool robin = d[q].lo_type == LSS_BC_ROBIN || d[q].hi_type == LSS_BC_ROBIN;
+            fixed = fixed && d[q].coeff_sets == 1 && (d[q].bnd_sets == 1 || !robin);
         }
         mem.alloc(total * sizeof(T));
         probs.resize(cnt);
@@ -479,6 +484,11 @@ template <typename T> struct H1Plan final : lss_heat1d_plan {
     template <int M> void launch_wave(hipStream_t st, const T *const *ui, T *const *uo, T *const *sf)
     {
         const unsigned blocks = (unsigned)((count + H1_WAVES - 1) / H1_WAVES);
+        if (fixed) {
+            hipLaunchKernelGGL((k_h1_wave_fixed<T, M>), dim3(blocks), dim3(64 * H1_WAVES), 0, st,
+                               (const H1Prob<T> *)probs_dev.p, (int)count, ui, uo, sf);
+            return;
+        }
         hipLaunchKernelGGL((k_h1_wave<T, M>), dim3(blocks), dim3(64 * H1_WAVES), 0, st,
                            (const H1Prob<T> *)probs_dev.p, (int)count, ui, uo, sf);
     }

@@ -274,3 +274,28 @@ def test_exact_kernel_rounds_like_the_oracle_at_any_magnitude(oracle, fp, scale)
             out = _stepped(oracle, q)[1]
         assert np.array_equal(outs[z], out, equal_nan=True), (z, q["n"])
     plan.close()
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("n", [4, 20, 65, 66, 67, 130, 190, 258, 390, 514, 600, 1024])
+def test_every_form_of_the_partitioned_kernels(oracle, fp, n):
+    # the nine end pairs, with and without a source, boundaries fixed or changing in time, the matrix fixed (one plan)
+    # or changing in time (another): 1..16 points per lane, lines that end on a lane's last point and before it.
+    # Tolerance: the rows dominate by at least 1 of at most 5 (b = 1 + theta 2 B, |a| + |c| = theta (A + D) <= theta 2 B),
+    # so a step's few tens of roundings grow at most fivefold; 256 eps a step covers both sides.
+    import ctypes
+    import itertools
+    rng = np.random.default_rng(n)
+    ends = (L.BC_DIRICHLET, L.BC_NEUMANN, L.BC_ROBIN)
+    for tc in (0, 1):
+        descr = [_descr(ctypes, fp, n, 6, L.THOMAS_LU, lo, hi, L.FORWARD if src else L.BACKWARD, tc,
+                        tb and (tc or L.BC_ROBIN not in (lo, hi)), src, 0.5, rng)
+                 for lo, hi, src, tb in itertools.product(ends, ends, (0, 1), (0, 1))]
+        plan = _described_plan(ctypes, descr, L.LINE_PARTITIONED)
+        outs, surfs = plan.run_host([q["u0"] for q in descr], surfaces=True)
+        for z, q in enumerate(descr):
+            surf, out = _stepped(oracle, q)
+            tol = 256 * q["steps"] * np.finfo(L.np_dtype(fp)).eps
+            e, es = _normwise(outs[z], out), _normwise(surfs[z], surf)
+            assert e <= tol and es <= tol, (tc, z, q["lo"], q["hi"], e, es)
+        plan.close()
