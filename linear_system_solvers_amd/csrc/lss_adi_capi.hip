@@ -163,9 +163,43 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     hipGraphExec_t gexec[GROUPS] = {};
     hipEvent_t gfork = nullptr, gjoin[GROUPS] = {};
 
-    // launch grid of tile table tb over the na problems still stepping, and the first tile, in the
-    // current tile set
-    int pre(int tb, int64_t na) const
+    // Slices.  A loop over problems whose state exceeds the last-level cache reads it from HBM in every stage; run
+    // as consecutive slices of problems (internal order: similar step counts) whose state about fits, the stages of a
+    // slice find most of it cached.  Smaller slices leave CUs idle and pay more launches.  Measured in fp64 (ms a
+    // solve by the bytes of a slice, MB): 1024 mixed Heston problems of up to 512 x 256, 50..500 steps: 130: 376, 160:
+    // 348, 200: 329, 260: 313, 320: 335, 450: 379, one slice: 377; 256 MCS problems of 512 x 256, 60 steps: 260: 46,
+    // 320: 54, 550: 62, one slice: 62.  So as many slices as bring each nearest to the cache's 256 MB.
+    // A sliced loop is launched directly: its kernels last longer than their launches take the host (312.6 ms against
+    // 313.8 ms as a graph), and capturing its hundred thousand launches would cost a first solve 0.3 s.
+    static constexpr double SLICE_BYTES = 256e6;
+    std::vector<int64_t> slices;       // slice k: internal problems slices[k] .. slices[k + 1] - 1
+    int64_t slice_q0 = 0, slice_q1 = 0;  // problems of the launches (default: all)
+    void all_problems()
+    {
+        slice_q0 = 0;
+        slice_q1 = count;
+    }
+    void make_slices()
+    {
+        double total = 0;
+        auto bytes = [&](const Prob<T> &p) { return (p.y2 ? 5.0 : 3.0) * p.nx * p.ny * sizeof(T); };
+        for (const Prob<T> &p : probs)
+            total += bytes(p);
+        const int64_t want = std::max<int64_t>(1, (int64_t)std::llround(total / SLICE_BYTES));
+        slices.assign(1, 0);
+        double at = 0;
+        for (int64_t q = 0; q < count; ++q) {
+            if ((int64_t)slices.size() < want && at >= total * (double)slices.size() / (double)want)
+                slices.push_back(q);
+            at += bytes(probs[q]);
+        }
+        slices.push_back(count);
+        all_problems();
+    }
+
+    // launch grid of tile table tb over the slice's problems among the na still stepping, and the first tile, in
+    // the current tile set
+    int pre_all(int tb, int64_t na) const
     {
         if (set_ == 0)
             return prefix[tb][na];
@@ -173,7 +207,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         const int64_t k = na > g ? (na - g + ngroups - 1) / ngroups : 0;
         return gprefix[g][tb][k];
     }
-    size_t toff(int tb) const { return set_ == 0 ? tile_off[tb] : gtile_off[set_ - 1][tb]; }
+    int pre(int tb, int64_t na) const { return pre_all(tb, std::max(na, slice_q0)) - pre_all(tb, slice_q0); }
+    size_t toff(int tb) const
+    {
+        return (set_ == 0 ? tile_off[tb] : gtile_off[set_ - 1][tb]) + (size_t)pre_all(tb, slice_q0);
+    }
     int max_steps = 0;
     int line_solver = LINE_EXACT;
     int pmx = 1, pmy = 1;              // points per chunk bound (template M) of S-lines and v-lines
@@ -520,6 +558,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             for (int tb = 0; tb < TB_N; ++tb)
                 HIPCHK(hipMemcpy((Tile *)tiles_dev.p + gtile_off[g][tb], gtiles[g][tb].data(),
                                  gtiles[g][tb].size() * sizeof(Tile), hipMemcpyHostToDevice));
+        make_slices();
         probs_dev.alloc(n * sizeof(Prob<T>));
         HIPCHK(hipMemcpy(probs_dev.p, probs.data(), n * sizeof(Prob<T>), hipMemcpyHostToDevice));
     }
@@ -543,7 +582,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     double algo_bytes(int k, int64_t na) const
     {
         double b = 0;
-        for (int64_t q = 0; q < na; ++q) {
+        for (int64_t q = slice_q0; q < na; ++q) {
             const Prob<T> &p = probs[q];
             const double nxy = (double)p.nx * p.ny;
             const bool dr = p.scheme == SCHEME_DR;
@@ -663,25 +702,27 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     }
 
     // the time loop as ngroups graphs (captured once), run concurrently after the work queued on
-    // `stream` and joined back into it
-    void run_groups(hipStream_t stream)
+    // `stream` and joined back into it; direct: the same launches without a graph
+    void run_groups(hipStream_t stream, bool direct)
     {
-        if (!gexec[0]) {
-            if (!gfork) {
-                HIPCHK(hipEventCreateWithFlags(&gfork, hipEventDisableTiming));
-                for (int g = 0; g < ngroups; ++g) {
+        if (!gfork) {
+            for (int g = 0; g < ngroups; ++g) {
+                if (!gstream[g])
                     HIPCHK(hipStreamCreateWithFlags(&gstream[g], hipStreamNonBlocking));
+                if (!gjoin[g])
                     HIPCHK(hipEventCreateWithFlags(&gjoin[g], hipEventDisableTiming));
-                }
             }
+            HIPCHK(hipEventCreateWithFlags(&gfork, hipEventDisableTiming));
+        }
+        if (!direct && !gexec[0]) {
             for (int g = 0; g < ngroups; ++g) {
                 set_ = g + 1;
                 try {
                     HIPCHK(hipStreamBeginCapture(gstream[g], hipStreamCaptureModeThreadLocal));
-                    for (int s = 0; s < probs[g].steps; ++s)  // group g's first problem has its most steps
-                        launch_step(s, s == 0, gstream[g]);
+                    launch_loop(gstream[g]);
                 } catch (...) {
                     set_ = 0;
+                    all_problems();
                     hipGraph_t partial = nullptr;
                     if (hipStreamEndCapture(gstream[g], &partial) == hipSuccess && partial)
                         (void)hipGraphDestroy(partial);
@@ -694,11 +735,23 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             }
         }
         HIPCHK(hipEventRecord(gfork, stream));
-        for (int g = 0; g < ngroups; ++g) {
+        for (int g = 0; g < ngroups; ++g)
             HIPCHK(hipStreamWaitEvent(gstream[g], gfork, 0));
-            HIPCHK(hipGraphLaunch(gexec[g], gstream[g]));
-            HIPCHK(hipEventRecord(gjoin[g], gstream[g]));
+        if (direct) {
+            try {
+                launch_loops();
+            } catch (...) {
+                set_ = 0;
+                all_problems();
+                throw;
+            }
+            set_ = 0;
+        } else {
+            for (int g = 0; g < ngroups; ++g)
+                HIPCHK(hipGraphLaunch(gexec[g], gstream[g]));
         }
+        for (int g = 0; g < ngroups; ++g)
+            HIPCHK(hipEventRecord(gjoin[g], gstream[g]));
         for (int g = 0; g < ngroups; ++g)
             HIPCHK(hipStreamWaitEvent(stream, gjoin[g], 0));
     }
@@ -750,7 +803,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         tuned = true;
     }
 
-    // Autotuner: times every (xw, vr) mapping on the first steps of the loop (at most 8, from the
+    // Autotuner: times every (xw, vr) mapping on the first steps of the first slice's loop (at most 8, from the
     // plan's current state) and keeps the fastest.  The mappings give identical results.
     void autotune(hipStream_t st)
     {
@@ -758,6 +811,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         if (line_solver != LINE_PARTITIONED || euler)
             return;
         const int nst = std::min(max_steps, 8);
+        slice_q1 = slices[1];  // (the first slice stands for the others)
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));
@@ -789,6 +843,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             }
         (void)hipEventDestroy(e0);
         (void)hipEventDestroy(e1);
+        all_problems();
         xw = bx;
         vr = bv;
         swz = bs;
@@ -799,12 +854,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     // (the exact sweeps compute the lines' gamma there)
     void launch_step(int s, bool fresh, hipStream_t st, Profiler *prof = nullptr, const Prob<T> *table = nullptr)
     {
-        const int64_t na = active(s);
+        const int64_t na = std::min(active(s), slice_q1);
         const Prob<T> *pd = table ? table : (const Prob<T> *)probs_dev.p;
         const Tile *td = (const Tile *)tiles_dev.p;
         auto grid = [&](int tb) { return (unsigned)pre(tb, na); };
         bool any_split2 = false;
-        for (int64_t q = 0; q < na; ++q)
+        for (int64_t q = slice_q0; q < na; ++q)
             any_split2 |= probs[q].scheme != SCHEME_DR;
         auto pre = [&](int k) {
             if (prof)
@@ -1452,11 +1507,39 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             launch_exact_t<PAT_GENERIC>(x, grid, st, pd, td, s, stage, fresh);
     }
 
+    bool sliced() const { return slices.size() > 2; }
+    // calls step(s) for every step of every slice (the slice's first problem has its most steps)
+    template <typename F> void each_slice_step(F &&step)
+    {
+        for (size_t k = 0; k + 1 < slices.size(); ++k) {
+            slice_q0 = slices[k];
+            slice_q1 = slices[k + 1];
+            for (int s = 0; s < probs[slice_q0].steps; ++s)
+                step(s);
+        }
+        all_problems();
+        HIPCHK(hipGetLastError());
+    }
+    // one step of the current slice and tile set, if it has problems that still step
+    void slice_step(int s, hipStream_t st)
+    {
+        if (pre(TB_P, std::min(active(s), slice_q1)) > 0)
+            launch_step(s, s == 0, st);
+    }
+    // the loop of the current tile set, slice by slice
     void launch_loop(hipStream_t st)
     {
-        for (int s = 0; s < max_steps; ++s)
-            launch_step(s, s == 0, st);
-        HIPCHK(hipGetLastError());
+        each_slice_step([&](int s) { slice_step(s, st); });
+    }
+    // the loops of all groups, each on its stream
+    void launch_loops()
+    {
+        each_slice_step([&](int s) {
+            for (int g = 0; g < ngroups; ++g) {
+                set_ = g + 1;
+                slice_step(s, gstream[g]);
+            }
+        });
     }
 
     void profile(const void *const *u_in, void *const *u_out, hipStream_t stream, double *ms, double *bytes,
@@ -1517,13 +1600,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         if (euler_res) {  // the whole loop in one launch, one workgroup per problem
             launch_euler_res(stream);
         } else if (use_graph && ngroups > 1) {
-            run_groups(stream);
-        } else if (use_graph) {
+            run_groups(stream, sliced());
+        } else if (use_graph && !sliced()) {
             if (!graph_exec) {
                 HIPCHK(hipStreamCreateWithFlags(&cap_stream, hipStreamNonBlocking));
                 HIPCHK(hipStreamBeginCapture(cap_stream, hipStreamCaptureModeThreadLocal));
-                for (int s = 0; s < max_steps; ++s)
-                    launch_step(s, s == 0, cap_stream);
+                launch_loop(cap_stream);
                 HIPCHK(hipStreamEndCapture(cap_stream, &graph));
                 HIPCHK(hipGraphInstantiate(&graph_exec, graph, nullptr, nullptr, 0));
             }

@@ -372,3 +372,30 @@ def test_exact_sweeps_keep_the_rounding_at_any_magnitude(oracle, fp, scale):
         assert np.array_equal(nxt, levels[s + 1], equal_nan=True)
     plan.close()
     single.close()
+
+
+# A book whose state exceeds the last-level cache is stepped as consecutive slices of problems (3 here: 210 problems
+# of about 3.0 or 1.8 MB), each slice ending at its own most steps.  Every problem takes the arithmetic of its own
+# plan: no tolerance.
+@pytest.mark.parametrize("line", [L.LINE_EXACT, L.LINE_PARTITIONED])
+def test_a_book_larger_than_the_cache_equals_its_problems_solved_alone(line):
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(41)
+    models = [_stable(int(rng.integers(290, 311)), int(rng.integers(240, 261)), steps=int(rng.integers(1, 9)),
+                      splitting=q % 4, strike=float(rng.uniform(60, 140)), coeff_mode=L.COEFF_SEPARABLE,
+                      line_solver=line)
+              for q in range(210)]
+    plan = L.Plan.from_models(models)
+    ins = [torch.from_numpy(plan.initial(p)).cuda() for p in range(plan.count)]
+    st = torch.cuda.current_stream().cuda_stream
+    res = []
+    for graph in (False, True, True):
+        outs = [torch.full_like(u, float("nan")) for u in ins]
+        plan.run_dev([u.data_ptr() for u in ins], [o.data_ptr() for o in outs], st, graph=graph)
+        res.append([(o * 1.0).cpu().numpy() for o in outs])
+        torch.cuda.synchronize()
+    plan.close()
+    for k in (1, 2):
+        assert all(np.array_equal(a, b) for a, b in zip(res[0], res[k]))
+    for q in range(0, 210, 13):
+        assert np.array_equal(_solve(models[q]), res[0][q]), q
