@@ -33,6 +33,8 @@ template <typename T, int PAT> __global__ void k_xsweep(const Prob<T> *, const T
 template <typename T, int PAT> __global__ void k_vsweep(const Prob<T> *, const Tile *, int, int, int);
 template <typename T, int PAT> __global__ void k_euler(const Prob<T> *, const Tile *, int);
 template <typename T, int PAT, int K> __global__ void k_euler_res(const Prob<T> *, const Tile *);
+template <typename T, int PAT, bool TWO>
+__global__ void k_adi_res(const Prob<T> *, const Tile *, const CopyJob *, int, const CopyJob *);
 template <typename T>
 __global__ void k_tridiag_lane(int64_t, int, int, const T *, const T *, const T *, const T *, T *, T *, LineBC<T>);
 template <typename T, int M, int STAGE, int W, int PAT, int NC>
@@ -223,6 +225,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     bool euler = false;                // explicit Euler plan (no line sweeps)
     int eres_rows = 10;                // rows per strip of k_euler_res
     bool euler_res = false;            // ... whose problems all fit k_euler_res (the loop resident in LDS)
+    bool adi_res = false;              // partitioned plan whose problems all fit k_adi_res
     bool all_fields = true;            // every problem has FIELDS coefficients
     hipStream_t cap_stream = nullptr;
     hipGraph_t graph = nullptr;
@@ -320,6 +323,20 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 code[blk * 12 + slot] = c;
             }
         }
+    }
+
+    // The resident loop (k_adi_res) takes a plan whose problems all have lines of at most 16 ARES_C interior points and
+    // fit LDS.  A step takes it the same time for 1 to 256 problems, in proportion to their points; the step-by-step
+    // loop, which spreads a problem over the GPU, takes 10.6 us for one problem of any such size in fp64, 18.5 us for
+    // 64.  Measured (DR steps, us, fp64: 1 and 64 problems step by step against resident): 100 x 50: 10.6, 18.5, 8.7;
+    // 100 x 64: 10.5, 18.7, 10.9; 130 x 66: 10.9, 19.8, 16.8; fp32: 100 x 90: 10.0, 16.6, 8.3; 130 x 100: 10.2, 17.3,
+    // 13.1; HV: fp64 100 x 50: 19.4, 33.7, 19.6; fp32 100 x 90: 18.1, 29.6, 17.8.  So larger problems need a book.
+    static constexpr int64_t RES_POINTS = sizeof(T) == 8 ? 5000 : 9000, RES_BOOK = 64;
+    static bool resident_ok(const Prob<T> &p, int64_t problems)
+    {
+        return ares_chunk(p.nx) <= ARES_C && ares_chunk(p.ny) <= ARES_C && !p.src_sets &&
+               (problems >= RES_BOOK || (int64_t)p.nx * p.ny <= RES_POINTS) &&
+               ares_values(p.nx, p.ny, p.scheme != SCHEME_DR) * (int64_t)sizeof(T) <= ARES_BYTES;
     }
 
     void build(const lss_adi_desc *descs, int64_t n)
@@ -487,6 +504,9 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 break;
             }
         }
+        adi_res = line_solver == LINE_PARTITIONED && !euler && fpat != PAT_GENERIC;
+        for (int64_t q = 0; q < n && adi_res; ++q)
+            adi_res = resident_ok(probs[q], n);
         // tile tables
         for (int tb = 0; tb < TB_N; ++tb) {
             prefix[tb].assign(n + 1, 0);
@@ -923,7 +943,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     // ---------------------------------------------------------------------------------------------
     int ck = 0;                                   // checkpoint interval of the adjoint allocation
     bool fwd_done = false;
-    dev_buffer adj_mem, adj_dev, seg_dev, slots_dev, jobs_dev, lam_jobs_dev;
+    dev_buffer adj_mem, adj_dev, seg_dev, slots_dev, jobs_dev, lam_jobs_dev, ckpt_jobs_dev;
     std::vector<Adj<T>> adjs;                     // host copy (device pointers inside)
     std::vector<T *> ckpt_base, seg_lv_base;      // per internal problem
     std::vector<size_t> fwd_job_off, bwd_job_off; // per checkpoint: first job in jobs_dev
@@ -1354,8 +1374,17 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         require(u_in && u_out, "null pointer array");
         for (int64_t c = 0; c < count; ++c)
             require(u_in[c] && u_out[c], "null surface pointer");
-        if (ck != K)
+        if (ck != K) {
+            if (adi_res && !ckpt_jobs_dev.p)
+                ckpt_jobs_dev.alloc(count * sizeof(CopyJob));
             adj_setup(K);
+            if (adi_res) {  // the resident loop writes the checkpoints
+                std::vector<CopyJob> cj;
+                for (int64_t q = 0; q < count; ++q)
+                    cj.push_back({nullptr, ckpt_base[q], 0});
+                HIPCHK(hipMemcpy(ckpt_jobs_dev.p, cj.data(), cj.size() * sizeof(CopyJob), hipMemcpyHostToDevice));
+            }
+        }
         if (!tuned)
             autotune(stream);
         fwd_done = false;
@@ -1365,10 +1394,14 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                                   stream));
         }
         const CopyJob *jd = (const CopyJob *)jobs_dev.p;
-        for (int s = 0; s < max_steps; ++s) {
-            if (s % K == 0)
-                launch_jobs(jd + fwd_job_off[s / K], fwd_job_n[s / K], stream);
-            launch_step(s, s == 0, stream);
+        if (adi_res) {
+            launch_adi_res(stream, (const CopyJob *)ckpt_jobs_dev.p, K, nullptr);
+        } else {
+            for (int s = 0; s < max_steps; ++s) {
+                if (s % K == 0)
+                    launch_jobs(jd + fwd_job_off[s / K], fwd_job_n[s / K], stream);
+                launch_step(s, s == 0, stream);
+            }
         }
         HIPCHK(hipGetLastError());
         for (int64_t q = 0; q < count; ++q) {
@@ -1490,6 +1523,26 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         HIPCHK(hipGetLastError());
     }
 
+    // the loops of a plan of small ADI problems (adi_res); levels, every, out: see k_adi_res
+    void launch_adi_res(hipStream_t st, const CopyJob *levels, int every, const CopyJob *out)
+    {
+        const Prob<T> *pd = (const Prob<T> *)probs_dev.p;
+        const Tile *tp = (const Tile *)tiles_dev.p + tile_off[TB_P];
+        const dim3 g((unsigned)count), b(ARES_T);
+        bool two = false;
+        for (const Prob<T> &p : probs)
+            two |= p.scheme != SCHEME_DR;
+        if (fpat == PAT_HESTON && two)
+            hipLaunchKernelGGL((k_adi_res<T, PAT_HESTON, true>), g, b, 0, st, pd, tp, levels, every, out);
+        else if (fpat == PAT_HESTON)
+            hipLaunchKernelGGL((k_adi_res<T, PAT_HESTON, false>), g, b, 0, st, pd, tp, levels, every, out);
+        else if (two)
+            hipLaunchKernelGGL((k_adi_res<T, PAT_SABR0, true>), g, b, 0, st, pd, tp, levels, every, out);
+        else
+            hipLaunchKernelGGL((k_adi_res<T, PAT_SABR0, false>), g, b, 0, st, pd, tp, levels, every, out);
+        HIPCHK(hipGetLastError());
+    }
+
     // a sweep of exact lines: S-lines (x) or v-lines
     template <int PAT>
     void launch_exact_t(bool x, unsigned grid, hipStream_t st, const Prob<T> *pd, const Tile *td, int s, int stage, int fresh)
@@ -1583,13 +1636,13 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             require(u_in[c] && u_out[c], "null surface pointer");
         const hipMemcpyKind kin = host ? hipMemcpyHostToDevice : hipMemcpyDeviceToDevice;
         const hipMemcpyKind kout = host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
-        if (!tuned)
+        if (!tuned && !adi_res)
             autotune(stream);
         // device surfaces of a plan of many problems: two batched copy launches instead of one copy
         // per problem and direction
         const bool batched_io = !host && count >= IO_BATCH_MIN;
         if (batched_io) {
-            io_jobs(u_in, u_out, stream);
+            io_jobs(u_in, u_out, stream, io_jobs_dev, io_last);
             launch_jobs((const CopyJob *)io_jobs_dev.p, (int)count, stream);
         } else {
             for (int64_t q = 0; q < count; ++q) {
@@ -1597,7 +1650,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 HIPCHK(hipMemcpyAsync(p.a, u_in[order[q]], sizeof(T) * (size_t)p.nx * p.ny, kin, stream));
             }
         }
-        if (euler_res) {  // the whole loop in one launch, one workgroup per problem
+        if (adi_res) {  // the whole loop in one launch, one workgroup per problem
+            const CopyJob *out = batched_io ? (const CopyJob *)io_jobs_dev.p + count : nullptr;
+            launch_adi_res(stream, nullptr, 1, out);
+            if (out)
+                return;
+        } else if (euler_res) {
             launch_euler_res(stream);
         } else if (use_graph && ngroups > 1) {
             run_groups(stream, sliced());
@@ -1666,7 +1724,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         require(u_in && levels, "null pointer array");
         for (int64_t c = 0; c < count; ++c)
             require(u_in[c] && levels[c], "null surface pointer");
-        if (!tuned)
+        if (!tuned && !adi_res)
             autotune(stream);
         if (host) {  // stage inputs and levels through one device allocation
             std::vector<size_t> off(count);
@@ -1696,6 +1754,13 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             }
             return;
         }
+        if (adi_res) {
+            io_jobs(u_in, levels, stream, lv_jobs_dev, lv_last);
+            const CopyJob *io = (const CopyJob *)lv_jobs_dev.p;
+            launch_jobs(io, (int)count, stream);
+            launch_adi_res(stream, io + count, 1, nullptr);
+            return;
+        }
         level_jobs(u_in, levels, stream);
         const CopyJob *jd = (const CopyJob *)lv_jobs_dev.p;
         for (int64_t q = 0; q < count; ++q) {
@@ -1716,11 +1781,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     static constexpr int64_t IO_BATCH_MIN = 8;
     dev_buffer io_jobs_dev;
     std::vector<const void *> io_last;
-    void io_jobs(const void *const *u_in, void *const *u_out, hipStream_t stream)
+    void io_jobs(const void *const *u_in, void *const *u_out, hipStream_t stream, dev_buffer &dev,
+                 std::vector<const void *> &last)
     {
         std::vector<const void *> key(u_in, u_in + count);
         key.insert(key.end(), u_out, u_out + count);
-        if (key == io_last)
+        if (key == last)
             return;
         std::vector<CopyJob> jobs(2 * count);
         for (int64_t q = 0; q < count; ++q) {
@@ -1729,11 +1795,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             jobs[q] = {u_in[order[q]], p.a, n};
             jobs[count + q] = {(p.steps & 1) ? p.b : p.a, u_out[order[q]], n};
         }
-        if (!io_jobs_dev.p)
-            io_jobs_dev.alloc(jobs.size() * sizeof(CopyJob));
+        if (!dev.p)
+            dev.alloc(jobs.size() * sizeof(CopyJob));
         HIPCHK(hipStreamSynchronize(stream));  // an earlier run may still read the old table
-        HIPCHK(hipMemcpy(io_jobs_dev.p, jobs.data(), jobs.size() * sizeof(CopyJob), hipMemcpyHostToDevice));
-        io_last = std::move(key);
+        HIPCHK(hipMemcpy(dev.p, jobs.data(), jobs.size() * sizeof(CopyJob), hipMemcpyHostToDevice));
+        last = std::move(key);
     }
 };
 

@@ -209,6 +209,21 @@ constexpr int EXL = 16;        // lines per tile of the exact sweeps (one wavefr
 constexpr int EX_ARRAYS = 6;   // arrays of the exact sweeps' workspace
 constexpr int TRI_LONG_C = 8;  // unknowns per thread of k_tridiag_long
 
+// The resident ADI loop (k_adi_res): threads, points per chunk at most (16 chunks per line), LDS, and per problem the
+// chunk length of lines of n points, the row stride and the LDS values it takes.  The stride spreads the accesses of an
+// S-sweep, 16 chunks of 4 adjacent lines, over the LDS banks: chunk length times stride is 4 modulo 8 where it can be.
+constexpr int ARES_T = 1024, ARES_C = 7, ARES_BYTES = 160 * 1024;
+__host__ __device__ constexpr int ares_chunk(int n) { return (n - 2 + 15) / 16; }
+__host__ __device__ constexpr int ares_ld(int nx, int ny)
+{
+    const int c = ares_chunk(nx), mod = c % 2 ? 8 : c % 4 ? 4 : 2, want = mod / 2;  // (c <= 7)
+    return ny + (want - ny % mod + mod) % mod;
+}
+__host__ __device__ constexpr int64_t ares_values(int nx, int ny, bool two)
+{
+    return (int64_t)(two ? 3 : 2) * nx * ares_ld(nx, ny) + 8 * nx + 9 * ny;
+}
+
 // one device-to-device copy of n elements (checkpoint and lambda transfers)
 struct CopyJob {
     const void *src;

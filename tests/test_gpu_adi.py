@@ -399,3 +399,51 @@ def test_a_book_larger_than_the_cache_equals_its_problems_solved_alone(line):
         assert all(np.array_equal(a, b) for a, b in zip(res[0], res[k]))
     for q in range(0, 210, 13):
         assert np.array_equal(_solve(models[q]), res[0][q]), q
+
+
+# ---------------------------------------------------------------------------------------------
+# Plans of small problems run their whole loop in one launch, a workgroup per problem, 16 chunks of 1 to 7 points per
+# line: sizes around the chunk lengths' edges, the smallest and the longest lines, the sizes that only a book of 64
+# takes.  Every scheme against the oracle (1e-12 of its largest value, the partitioned solver's tolerance above; fp32
+# 1e-5, as above); every level and the checkpointing forward equal the plain run, which runs the same loop.
+# ---------------------------------------------------------------------------------------------
+def _sabr_small(nx, ny, steps, splitting):
+    K = 0.03
+    return L.Model(kind=L.MODEL_SABR, strike=K, rate=0.0, sig_sig=0.5, rho=-0.3, beta=0.6, maturity=1.0,
+                   x_lo=0.0, x_hi=5 * K, y_lo=0.0, y_hi=0.25, nx=nx, ny=ny, nt=steps + 1, t_hi=0.002 * steps,
+                   accumulation_point=K, alpha_scale=10.0, beta_scale=50.0, grid=L.NONUNIFORM, splitting=splitting,
+                   weighting=0.5, coeff_mode=L.COEFF_SEPARABLE, line_solver=L.LINE_PARTITIONED)
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("model", ["heston", "sabr"])
+@pytest.mark.parametrize("nx,ny,count", [(4, 4, 4), (18, 19, 4), (19, 18, 4), (35, 51, 4), (66, 67, 4), (114, 43, 4),
+                                         (43, 114, 4), (101, 60, 64)])
+def test_resident_loop_matches_the_oracle(oracle, fp, model, nx, ny, count):
+    torch = pytest.importorskip("torch")
+    if model == "heston":
+        models = [_stable(nx, ny, steps=5 + q % 3, splitting=q % 4, coeff_mode=L.COEFF_SEPARABLE,
+                          line_solver=L.LINE_PARTITIONED) for q in range(count)]
+    else:
+        models = [_sabr_small(nx, ny, 5 + q % 3, q % 4) for q in range(count)]
+    plan = L.Plan.from_models(models, fp)
+    assert plan.kernel_config()["factor_pattern"] > 0
+    ins = [torch.from_numpy(plan.initial(p)).cuda() for p in range(count)]
+    pin = [u.data_ptr() for u in ins]
+    outs, fwd = ([torch.full_like(u, float("nan")) for u in ins] for _ in range(2))
+    levels = [torch.full((plan.shape(p)[2] + 1, nx, ny), float("nan"), dtype=ins[p].dtype, device="cuda")
+              for p in range(count)]
+    plan.run_dev(pin, [o.data_ptr() for o in outs])
+    plan.run_levels_dev(pin, [v.data_ptr() for v in levels])
+    plan.forward(pin, [o.data_ptr() for o in fwd], 2)
+    torch.cuda.synchronize()
+    tol = 1e-12 if fp == L.FP64 else 1e-5
+    for p in range(count):
+        assert torch.equal(outs[p], levels[p][-1]) and torch.equal(outs[p], fwd[p])
+        assert torch.equal(levels[p][0], ins[p])
+        if p < 4:
+            c = oracle_solve(oracle, models[p], "f64" if fp == L.FP64 else "f32").astype(np.float64)
+            assert _normwise(outs[p].cpu().numpy().astype(np.float64), c) <= tol
+            short = L.Plan.from_models([models[p]], fp).run_levels_host([plan.initial(p)])[0]
+            assert _normwise(levels[p].cpu().numpy().astype(np.float64), short.astype(np.float64)) <= tol
+    plan.close()
