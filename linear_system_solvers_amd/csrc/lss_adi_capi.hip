@@ -330,7 +330,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     // loop, which spreads a problem over the GPU, takes 10.6 us for one problem of any such size in fp64, 18.5 us for
     // 64.  Measured (DR steps, us, fp64: 1 and 64 problems step by step against resident): 100 x 50: 10.6, 18.5, 8.7;
     // 100 x 64: 10.5, 18.7, 10.9; 130 x 66: 10.9, 19.8, 16.8; fp32: 100 x 90: 10.0, 16.6, 8.3; 130 x 100: 10.2, 17.3,
-    // 13.1; HV: fp64 100 x 50: 19.4, 33.7, 19.6; fp32 100 x 90: 18.1, 29.6, 17.8.  So larger problems need a book.
+    // 13.1; HV: fp64 100 x 50: 19.4, 33.7, 19.6; fp32 100 x 90: 18.1, 29.6, 17.8.  So larger problems need a book.  (Resident times before the
+    // v-lines' matrix was eliminated once; they are 0.85 of these since.)
     static constexpr int64_t RES_POINTS = sizeof(T) == 8 ? 5000 : 9000, RES_BOOK = 64;
     static bool resident_ok(const Prob<T> &p, int64_t problems)
     {

@@ -212,6 +212,7 @@ constexpr int TRI_LONG_C = 8;  // unknowns per thread of k_tridiag_long
 // The resident ADI loop (k_adi_res): threads, points per chunk at most (16 chunks per line), LDS, and per problem the
 // chunk length of lines of n points, the row stride and the LDS values it takes.  The stride spreads the accesses of an
 // S-sweep, 16 chunks of 4 adjacent lines, over the LDS banks: chunk length times stride is 4 modulo 8 where it can be.
+constexpr int ARES_VT = 6, ARES_VC = 13;  // values per point and per chunk of the eliminated v-lines
 constexpr int ARES_T = 1024, ARES_C = 7, ARES_BYTES = 160 * 1024;
 __host__ __device__ constexpr int ares_chunk(int n) { return (n - 2 + 15) / 16; }
 __host__ __device__ constexpr int ares_ld(int nx, int ny)
@@ -221,7 +222,7 @@ __host__ __device__ constexpr int ares_ld(int nx, int ny)
 }
 __host__ __device__ constexpr int64_t ares_values(int nx, int ny, bool two)
 {
-    return (int64_t)(two ? 3 : 2) * nx * ares_ld(nx, ny) + 8 * nx + 9 * ny;
+    return (int64_t)(two ? 3 : 2) * nx * ares_ld(nx, ny) + 8 * nx + 9 * ny + ARES_VT * 16 * ares_chunk(ny) + ARES_VC * 16;
 }
 
 // one device-to-device copy of n elements (checkpoint and lambda transfers)

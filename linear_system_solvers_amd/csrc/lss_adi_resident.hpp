@@ -2,10 +2,10 @@
 // levels and intermediates resident in LDS.
 //
 // Step by step, such a plan is bound by its launches: 64 problems of 100 x 50 in fp64 take 18.5 us a DR step for 1 us of
-// traffic, 22 us when every level is copied out.  Here a stage ends at a barrier of its workgroup: 8.7 us a step (9.4
+// traffic, 22 us when every level is copied out.  Here a stage ends at a barrier of its workgroup: 7.4 us a step (8.3
 // with the levels, which the S-sweep's phase stores while it reads them), for 1 to 256 problems; 1024 problems 11.8 ->
-// 3.5 ms for 100 steps, one problem 1.08 -> 0.85 ms, 200 MCS problems of 40 x 20 2.84 -> 0.83 ms; fp32 64 problems 1.58
-// -> 0.58 ms.
+// 3.0 ms for 100 steps, one problem 1.08 -> 0.74 ms, 200 MCS problems of 40 x 20 2.84 -> 0.79 ms; fp32 64 problems 1.58
+// -> 0.53 ms.
 // What bounds a step is the issue of its instructions (a point's equation is formed and eliminated in about 75, and a
 // SIMD has four wavefronts), so the partition wastes few of them: a line takes 16 lanes, whose chunks are as short as
 // its length allows (any length up to ARES_C, not only those of wave_solve), and the 16 interface equations are
@@ -236,6 +236,176 @@ __device__ __forceinline__ void res_vsweep(const Prob<T> *__restrict__ probs, in
     }
 }
 
+// The v-lines' matrix, eliminated once: with the compile-time patterns b, e and f have no X factor, so it is the same
+// for every line, and for every step when the coefficients do not change in time.  vt: per point the equation (a, b - 1,
+// c) and rb = 1 / b', zq and g of Chunk; vc: per chunk a, c and 1 / b of the interface row before each reduction step, and
+// the last 1 / b.  (Per step a v-sweep then costs its right-hand sides: 100 x 50 in fp64
+// 8.7 -> 7.4 us a DR step.)
+template <typename T, int PAT> constexpr bool res_same_vlines()
+{
+    if constexpr (PAT == PAT_GENERIC) {
+        return false;
+    } else {
+        bool same = true;
+        for (int q : {1, 4, 5})
+            same = same && FPat<PAT>::c[2 * q] < 0 && FPat<PAT>::c[2 * q + 1] < 0;
+        return same;
+    }
+}
+template <typename T> struct VTab {
+    lptr<T> vt, vc;
+    int n;  // points: 16 chunks
+    __device__ __forceinline__ lptr<T> at(int arr, int q) const { return vt + arr * n + q; }
+    __device__ __forceinline__ lptr<T> level(int k, int ll) const { return vc + k * 16 + ll; }
+};
+template <typename T, int D> __device__ __forceinline__ Eq<T> res_vlevel(const VTab<T> &v, int k, int ll, bool st, const Eq<T> &e)
+{
+    if (st) {
+        *v.level(3 * k, ll) = e.a;
+        *v.level(3 * k + 1, ll) = e.c;
+        *v.level(3 * k + 2, ll) = fast_rcp(e.b);
+    }
+    return row_pcr<D>(e);
+}
+// by the first wavefront
+template <typename T, int PAT, int C>
+__device__ __forceinline__ void res_vtable(const Prob<T> *__restrict__ probs, int prob, const ResMem<T> &m, const VTab<T> &v)
+{
+    const Prob<T> &p = probs[opaque_uniform(prob)];
+    const int tid = opaque_lane((int)threadIdx.x), ll = tid & 15, N = p.ny - 2, s = 1 + ll * C;
+    if (tid >= 64)
+        return;
+    const bool st = tid < 16;  // (the four rows of lanes do the same)
+    const T one = (T)1.0, theta = p.theta;
+    T g[C], zq[C], ae = (T)0, be = one, ce = (T)0;
+#pragma unroll
+    for (int t = 0; t < C; ++t) {
+        const Stencil<T> sc = res_stencil<T, PAT>(p, m, 0, min(s + t, N + 1));
+        T a = (-theta * sc.Mt), b = theta * sc.W, c = (-theta * sc.Pt);
+        if (st) {
+            *v.at(0, s - 1 + t) = a;
+            *v.at(1, s - 1 + t) = b;
+            *v.at(2, s - 1 + t) = c;
+        }
+        b = one + b;
+        if (s > N)  // a chunk wholly past the end: identity rows
+            a = c = (T)0, b = one;
+        a = s + t == 1 ? (T)0 : a;
+        c = s + t >= N ? (T)0 : c;
+        if (t == C - 1) {
+            ae = a, be = b, ce = c;
+        } else {
+            const T rb = fast_rcp(t == 0 ? b : b - a * g[t > 0 ? t - 1 : 0]);
+            g[t] = c * rb;
+            zq[t] = (t == 0 ? -a : -a * zq[t > 0 ? t - 1 : 0]) * rb;
+            if (st)
+                *v.at(3, s - 1 + t) = rb;
+        }
+    }
+    T ql = one, rl = (T)0, QF = (T)0, RF = one;
+    if constexpr (C >= 2) {
+        g[C - 2] = -g[C - 2];
+#pragma unroll
+        for (int u = C - 3; u >= 0; --u) {
+            const T gu = g[u];
+            g[u] = -gu * g[u + 1];
+            zq[u] = zq[u] - gu * zq[u + 1];
+        }
+        ql = zq[C - 2], rl = g[C - 2], QF = zq[0], RF = g[0];
+        if (st) {
+#pragma unroll
+            for (int t = 0; t < C - 1; ++t) {
+                *v.at(4, s - 1 + t) = zq[t];
+                *v.at(5, s - 1 + t) = g[t];
+            }
+        }
+    }
+    Eq<T> e{ae * ql, (T)0, (T)0, (T)0};
+    const T nQF = row_down<1>(QF), nRF = row_down<1>(RF);
+    e.b = ae * rl + be + ce * nQF;
+    e.c = ce * nRF;
+    e = res_vlevel<T, 1>(v, 0, ll, st, e);
+    e = res_vlevel<T, 2>(v, 1, ll, st, e);
+    e = res_vlevel<T, 4>(v, 2, ll, st, e);
+    e = res_vlevel<T, 8>(v, 3, ll, st, e);
+    if (st)
+        *v.level(12, ll) = fast_rcp(e.b);
+}
+template <typename T, int D> __device__ __forceinline__ T res_vreduce(const VTab<T> &v, int k, int ll, T r)
+{
+    const T a = *v.level(3 * k, ll), c = *v.level(3 * k + 1, ll), n = r * *v.level(3 * k + 2, ll);
+    return r - a * row_up<D>(n) - c * row_down<D>(n);
+}
+// res_vsweep with the eliminated matrix
+template <typename T, int C>
+__device__ __forceinline__ void res_vsweep_tab(const Prob<T> *__restrict__ probs, int prob, const ResMem<T> &m, const VTab<T> &v,
+                                               lptr<const T> in, lptr<T> out)
+{
+    const Prob<T> &p = probs[opaque_uniform(prob)];
+    const int tid = opaque_lane((int)threadIdx.x), wave = opaque_uniform(tid >> 6), sub = (tid & 63) >> 4, ll = tid & 15;
+    const int N = p.ny - 2, lines = p.nx - 2, s = 1 + ll * C, jmax = N + 1, ld = m.ld;
+    for (int g = 4 * wave; g < lines; g += ARES_T / 16) {
+        const int i = 1 + min(g + sub, lines - 1);
+        const bool own = g + sub < lines;
+        const int ii = m.idx1[i];
+        const T lo = m.cA0[ii], hi = m.cA1[ii];
+        const int o1 = (int)(m.y1 - in);
+        T zp[C], re = (T)0, ae = (T)0, ce = (T)0;
+        if (s <= N) {
+            lptr<const T> q = in + (i * ld + s - 1);
+            T left = q[0], mid = q[min(1, jmax - (s - 1))];
+            T g0[C];
+#pragma unroll
+            for (int t = 0; t < C; ++t) {
+                const int k = s + t;
+                const T right = q[min(t + 2, jmax - (s - 1))];
+                const T a = *v.at(0, k - 1), c = *v.at(2, k - 1);
+                T r = (a * left) + (*v.at(1, k - 1) * mid) + (c * right) + q[o1 + min(t + 1, jmax - (s - 1))];
+                if (k == 1)
+                    r = r - a * lo;
+                if (k >= N)
+                    r = r - c * hi;
+                const T cf = k >= N ? (T)0 : c;
+                if (t == C - 1) {
+                    re = r, ae = a, ce = cf;
+                } else {
+                    const T rb = *v.at(3, k - 1);
+                    g0[t] = cf * rb;
+                    zp[t] = (t == 0 ? r : r - a * zp[t > 0 ? t - 1 : 0]) * rb;
+                }
+                left = mid;
+                mid = right;
+            }
+#pragma unroll
+            for (int u = C - 3; u >= 0; --u)
+                zp[u] = zp[u] - g0[u] * zp[u + 1];
+        } else {
+#pragma unroll
+            for (int t = 0; t < C; ++t)
+                zp[t] = (T)0;
+        }
+        const T pl = C >= 2 ? zp[C >= 2 ? C - 2 : 0] : (T)0, PF = C >= 2 ? zp[0] : (T)0;
+        T r = re - ae * pl - ce * row_down<1>(PF);
+        r = res_vreduce<T, 1>(v, 0, ll, r);
+        r = res_vreduce<T, 2>(v, 1, ll, r);
+        r = res_vreduce<T, 4>(v, 2, ll, r);
+        r = res_vreduce<T, 8>(v, 3, ll, r);
+        const T xi = r * *v.level(12, ll);
+        const T xl = row_up<1>(xi);
+        lptr<T> o = out + (i * ld + s);
+        if (own) {
+#pragma unroll
+            for (int t = 0; t < C; ++t)
+                if (s + t <= N)
+                    o[t] = t == C - 1 ? xi : zp[t] + *v.at(4, s - 1 + t) * xl + *v.at(5, s - 1 + t) * xi;
+            if (ll == 0) {
+                out[i * ld] = lo;
+                out[i * ld + N + 1] = hi;
+            }
+        }
+    }
+}
+
 // the surface in LDS to or from HBM, a wavefront per row
 template <typename T> __device__ __forceinline__ void res_store(gptr<T> dst, lptr<const T> u, int nx, int ny, int ld)
 {
@@ -275,6 +445,7 @@ __global__ void __launch_bounds__(ARES_T) k_adi_res(const Prob<T> *__restrict__ 
     m.cA0 = take(nx);
     m.cA1 = take(nx);
     m.bn = take(nx + 2 * ny);
+    const VTab<T> v{take(ARES_VT * 16 * ares_chunk(ny)), take(ARES_VC * 16), 16 * ares_chunk(ny)};
     const lptr<int> ix = (lptr<int>)at;
     m.idx1 = ix;
     m.idx2 = ix + nx;
@@ -294,6 +465,12 @@ __global__ void __launch_bounds__(ARES_T) k_adi_res(const Prob<T> *__restrict__ 
             m.y1[q] = (T)0;
     }
     const gptr<T> lv = levels ? G((T *)levels[tl.prob].dst) : nullptr;
+    auto vsweep = [&](lptr<const T> in, lptr<T> o) {
+        if (res_same_vlines<T, PAT>() && p.coeff_sets == 1)
+            with_length(cv, [&](auto c) { res_vsweep_tab<T, decltype(c)::value>(probs, tl.prob, m, v, in, o); });
+        else
+            with_length(cv, [&](auto c) { res_vsweep<T, PAT, decltype(c)::value>(probs, tl.prob, m, in, o); });
+    };
     const T two_ = (T)2.0, three = (T)3.0, four = (T)4.0;
     for (int s = 0; s < steps; ++s) {
         m.cs = GArr<T>{coeff_set(p, s)};
@@ -306,6 +483,10 @@ __global__ void __launch_bounds__(ARES_T) k_adi_res(const Prob<T> *__restrict__ 
             for (int q = tid; q < nx + 2 * ny; q += ARES_T)
                 m.bn[q] = bs[q];
             __syncthreads();
+            if constexpr (res_same_vlines<T, PAT>()) {  // (read after the S-sweep's barrier)
+                if (s == 0 && p.coeff_sets == 1)
+                    with_length(cv, [&](auto c) { res_vtable<T, PAT, decltype(c)::value>(probs, tl.prob, m, v); });
+            }
         }
         with_length(cx, [&](auto c) { res_xsweep<T, 0, PAT, decltype(c)::value>(probs, tl.prob, m); });
         {  // boundary stage A, from the last thread down
@@ -328,7 +509,7 @@ __global__ void __launch_bounds__(ARES_T) k_adi_res(const Prob<T> *__restrict__ 
         if (lv && s % every == 0)
             res_store<T>(lv + (size_t)(s / every) * n, m.u, nx, ny, ld);
         __syncthreads();
-        with_length(cv, [&](auto c) { res_vsweep<T, PAT, decltype(c)::value>(probs, tl.prob, m, m.u, two ? m.y2 : m.y1); });
+        vsweep(m.u, two ? m.y2 : m.y1);
         __syncthreads();
         if constexpr (TWO) {
             if (two) {
@@ -341,9 +522,7 @@ __global__ void __launch_bounds__(ARES_T) k_adi_res(const Prob<T> *__restrict__ 
                         res_xsweep<T, 3, PAT, decltype(c)::value>(probs, tl.prob, m);
                 });
                 __syncthreads();
-                with_length(cv, [&](auto c) {
-                    res_vsweep<T, PAT, decltype(c)::value>(probs, tl.prob, m, p.scheme == SCHEME_HV ? m.y2 : m.u, m.y1);
-                });
+                vsweep(p.scheme == SCHEME_HV ? m.y2 : m.u, m.y1);
                 __syncthreads();
             }
         }
