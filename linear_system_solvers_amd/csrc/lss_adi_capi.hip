@@ -944,6 +944,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     // ---------------------------------------------------------------------------------------------
     int ck = 0;                                   // checkpoint interval of the adjoint allocation
     bool fwd_done = false;
+    bool last_stored = false;                     // the last segment's storage set holds its stages
     dev_buffer adj_mem, adj_dev, seg_dev, slots_dev, jobs_dev, lam_jobs_dev, ckpt_jobs_dev;
     std::vector<Adj<T>> adjs;                     // host copy (device pointers inside)
     std::vector<T *> ckpt_base, seg_lv_base;      // per internal problem
@@ -1388,7 +1389,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         }
         if (!tuned)
             autotune(stream);
-        fwd_done = false;
+        fwd_done = last_stored = false;
+        const int cl = (max_steps - 1) / K, s0 = cl * K, set = dbl ? cl & 1 : 0;
         for (int64_t q = 0; q < count; ++q) {
             const Prob<T> &p = probs[q];
             HIPCHK(hipMemcpyAsync(p.a, u_in[order[q]], sizeof(T) * (size_t)p.nx * p.ny, hipMemcpyDeviceToDevice,
@@ -1398,20 +1400,26 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         if (adi_res) {
             launch_adi_res(stream, (const CopyJob *)ckpt_jobs_dev.p, K, nullptr);
         } else {
+            // the last segment is stepped in its storage set, as the backward pass would recompute it first
             for (int s = 0; s < max_steps; ++s) {
                 if (s % K == 0)
                     launch_jobs(jd + fwd_job_off[s / K], fwd_job_n[s / K], stream);
-                launch_step(s, s == 0, stream);
+                if (s == s0)
+                    launch_jobs(jd + bwd_job_off[cl], bwd_job_n[cl], stream);
+                launch_step(s, s == 0, stream, nullptr, s >= s0 ? seg_table(s - s0, set) : nullptr);
             }
         }
         HIPCHK(hipGetLastError());
         for (int64_t q = 0; q < count; ++q) {
             const Prob<T> &p = probs[q];
             const T *res = (p.steps & 1) ? p.b : p.a;
+            if (!adi_res && p.steps > s0)
+                res = seg_lv_base[q + set * count] + (size_t)(p.steps - s0) * p.nx * p.ny;
             HIPCHK(hipMemcpyAsync(u_out[order[q]], res, sizeof(T) * (size_t)p.nx * p.ny, hipMemcpyDeviceToDevice,
                                   stream));
         }
         fwd_done = true;
+        last_stored = !adi_res;
     }
 
     void backward(const void *const *lam_out, void *const *lam_in, double *dparams, hipStream_t stream) override
@@ -1450,9 +1458,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             for (int s = s1 - 1; s >= s0; --s)
                 launch_adj_step(s, seg_table(s - s0, set), stream);
         };
+        const bool have_last = last_stored;
+        last_stored = false;
         if (!dbl) {
             for (int c = nseg - 1; c >= 0; --c) {
-                recompute(c, 0, stream);
+                if (c < nseg - 1 || !have_last)
+                    recompute(c, 0, stream);
                 adjoint(c, 0);
             }
         } else {
@@ -1468,7 +1479,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             }
             HIPCHK(hipEventRecord(ev_fork, stream));
             HIPCHK(hipStreamWaitEvent(aux_stream, ev_fork, 0));
-            recompute(nseg - 1, (nseg - 1) & 1, aux_stream);
+            if (!have_last)
+                recompute(nseg - 1, (nseg - 1) & 1, aux_stream);
             HIPCHK(hipEventRecord(ev_ready[(nseg - 1) & 1], aux_stream));
             for (int c = nseg - 1; c >= 0; --c) {
                 if (c >= 1) {

@@ -269,3 +269,34 @@ def test_overlapped_backward_matches_the_single_stream_one():
     assert plan.kernel_config()["adjoint_overlap"] == 1
     with pytest.raises(L.LssError):
         plan.set_adjoint_overlap(2)
+
+
+@pytest.mark.parametrize("solver", [L.LINE_PARTITIONED, L.LINE_EXACT])
+@pytest.mark.parametrize("overlap", [0, 1])
+@pytest.mark.parametrize("steps", [(7,), (8,), (9, 3, 12, 8)])
+def test_a_second_backward_of_one_forward_gives_the_same_gradients(solver, overlap, steps):
+    """The forward pass leaves the last segment's stages for the first backward pass; a second one recomputes them
+    from the checkpoint.  The same kernels on the same values: no tolerance.  Steps around the segment length (4),
+    problems that end in earlier segments, and sizes that no resident loop takes."""
+    mode = L.COEFF_SEPARABLE if solver == L.LINE_PARTITIONED else L.COEFF_FIELDS
+    models = [_heston((2 + q) % 4, nx=150 + q, ny=40 + q, steps=n, coeff_mode=mode, line_solver=solver)
+              for q, n in enumerate(steps)]
+    plan = L.Plan.from_models(models)
+    plan.set_adjoint_overlap(overlap)
+    u0s = [plan.initial(p) for p in range(plan.count)]
+    ins = [_dev(u) for u in u0s]
+    outs = [torch.empty_like(d) for d in ins]
+    plan.forward([d.data_ptr() for d in ins], [o.data_ptr() for o in outs], ckpt_every=4)
+    lo = [_dev(np.random.default_rng(7 + p).standard_normal(u.shape)) for p, u in enumerate(u0s)]
+    res = []
+    for _ in range(2):
+        li = [torch.empty_like(d) for d in ins]
+        dp = plan.backward([d.data_ptr() for d in lo], [d.data_ptr() for d in li])
+        torch.cuda.synchronize()
+        res.append((dp, [g.cpu().numpy() for g in li]))
+    np.testing.assert_array_equal(res[0][0], res[1][0])
+    for a, b in zip(res[0][1], res[1][1]):
+        np.testing.assert_array_equal(a, b)
+    for o, u in zip(outs, _run(plan, u0s)):
+        np.testing.assert_array_equal(o.cpu().numpy(), u)
+    plan.close()
