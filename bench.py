@@ -485,7 +485,7 @@ def explicit_models(count=1024, seed=5, coeff_mode=L.COEFF_SEPARABLE):
 def bench_heat1d(torch, log, count=16384, n=256, nt=1001, oracle_check=2):
     """1-D Black-Scholes book (the reference's one-dimensional implicit solver): count calls with the
     strike, volatility and rate drawn per problem, n-point uniform grids, nt - 1 Crank-Nicolson steps,
-    each problem's whole loop in one launch.  Exact order (one lane per problem) and partitioned (one
+    each problem's whole loop in one launch.  Exact order (four lanes per problem) and partitioned (one
     wavefront per problem, the loop in registers); the exact path is checked against the oracle, the
     partitioned against the exact path."""
     from oracle import oracle as O
@@ -558,7 +558,7 @@ def bench_levels(torch, log, count=64):
     level_bytes = count * (st + 1) * nx * ny * es
     plan.close()
     log(f"every level: {count} problems {nx}x{ny}x{st}, levels {t_levels * 1e3:.2f} ms against final level only "
-        f"{t_final * 1e3:.2f} ms (launch by launch); {level_bytes / 1e9:.2f} GB of levels at "
+        f"{t_final * 1e3:.2f} ms; {level_bytes / 1e9:.2f} GB of levels at "
         f"{level_bytes / t_levels / 1e9:.0f} GB/s of solve time; last level equals the final-level solve: {same}")
     return {"workload": f"heston_dr_{count}x{nx}x{ny}x{st}_every_level", "levels_ms": round(t_levels * 1e3, 3),
             "final_level_ms": round(t_final * 1e3, 3), "level_bytes": level_bytes,
@@ -607,9 +607,8 @@ def bench_explicit(torch, log, count=1024, oracle_check=2):
     prof = L.run_profiled(plan, pin, pout, stream)  # (launch by launch)
     e_ms, e_bytes, e_n = prof["euler"]
     gbs = e_bytes / (e_ms / 1e3) / 1e9
-    # the resident loop reads 9 neighbours and writes 1 value per interior point-step in LDS (an upper
-    # figure: boundary points read fewer)
-    lds_gbs = 10 * 8 * ps / secs / 1e9
+    # the resident loop's strips of 6 rows read 2 x 6 + 6 values and write 6 in LDS per step
+    lds_gbs = 4 * 8 * ps / secs / 1e9
     worst = 0.0
     for q in range(oracle_check):
         c = oracle_solve(O, models[q])

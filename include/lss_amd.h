@@ -50,7 +50,7 @@ enum {
 };
 /* line solver of the implicit sweeps */
 enum {
-    LSS_LINE_EXACT = 0,       /* one lane per line in the reference's Thomas / double-sweep order   */
+    LSS_LINE_EXACT = 0,       /* the reference's Thomas / double-sweep order, operation by operation */
     LSS_LINE_PARTITIONED = 1  /* register-resident chunks + cyclic reduction of the chunk interfaces */
 };
 /* batched tridiagonal layouts */
@@ -146,8 +146,13 @@ int lss_adi_set_adjoint_overlap(lss_adi_plan *plan, int32_t mode);
  * concurrent groups a graph replay of lss_adi_run_dev runs the problems in (2 for plans of two or
  * more problems, else 1), and whether lss_adi_run_dev / lss_adi_run_host step an explicit Euler plan in
  * one launch with the time levels resident in LDS (1: every problem has at most 1536 points, nx >= 4,
- * ny <= 256, one coefficient set and one boundary set; lss_adi_run_levels always steps launch by
- * launch). */
+ * ny <= 256, one coefficient set and one boundary set; lss_adi_run_levels steps such a plan launch by
+ * launch).  Partitioned plans whose problems are all small run resident in LDS too, in every run (their
+ * lines have at most 112 interior points, their arrays fit the 160 KiB of a CU, the coefficients have a
+ * compile-time factor pattern and there is no heat source; fewer than 64 problems: at most 5000 points
+ * each in fp64, 9000 in fp32); the mapping does not matter to them and the autotuner does not run for
+ * them.  Larger books whose state exceeds the last-level cache are stepped in slices, launched directly
+ * (use_graph then only selects the two groups). */
 enum { LSS_KERNEL_CONFIG_LEN = 13 };
 int lss_plan_kernel_config(const lss_adi_plan *plan, int32_t *config);
 int lss_adi_run_host(lss_adi_plan *plan, const void *const *u_in, void *const *u_out);
