@@ -40,6 +40,7 @@ __global__ void k_tridiag_lane(int64_t, int, int, const T *, const T *, const T 
 template <typename T, int M, int STAGE, int W, int PAT, int NC>
 __global__ void k_xsweep_p(const Prob<T> *, const Tile *, int, int);
 template <typename T, int M, int VR, int PAT> __global__ void k_vsweep_p(const Prob<T> *, const Tile *, int, int, int);
+template <typename T, int M, int VR, int PAT> __global__ void k_vsweep_b(const Prob<T> *, const Tile *, int, int, int);
 template <typename T, int M, int PAT>
 __global__ void k_adj_v(const Prob<T> *, const Adj<T> *, const Tile *, int, int, double *);
 template <typename T, int M, int W, int PAT, int STAGE, int NC>
@@ -225,6 +226,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     bool euler = false;                // explicit Euler plan (no line sweeps)
     int eres_rows = 10;                // rows per strip of k_euler_res
     bool euler_res = false;            // ... whose problems all fit k_euler_res (the loop resident in LDS)
+    bool fold_b = false;               // boundary stage B in the last v-sweep (see build)
+    bool bnd_in_v = false;             // ... of the launches of a v-sweep
     bool adi_res = false;              // partitioned plan whose problems all fit k_adi_res
     bool all_fields = true;            // every problem has FIELDS coefficients
     hipStream_t cap_stream = nullptr;
@@ -325,6 +328,12 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         }
     }
 
+    // Partitioned plans of at most this many points evaluate boundary stage B in the step's last v-sweep (k_vsweep_b): a
+    // launch less per step.  Measured in fp64 (ms, a launch of its own against folded): one problem of 300 x 150, 100
+    // steps DR 1.35, 1.18, HV 2.68, 2.49; 64 of them DR 4.61, 4.19; 16 of mixed schemes 3.92, 3.78; 1024 x 512 MCS 5.42,
+    // 5.22; but 32 MCS problems of 512 x 256 6.24, 6.31, fp32 64 HV ones 7.81, 7.82, and the sweeps of a large book are
+    // a tenth slower.
+    static constexpr int64_t FOLD_POINTS = 3000000;
     // The resident loop (k_adi_res) takes a plan whose problems all have lines of at most 16 ARES_C interior points and
     // fit LDS.  A step takes it the same time for 1 to 256 problems, in proportion to their points; the step-by-step
     // loop, which spreads a problem over the GPU, takes 10.6 us for one problem of any such size in fp64, 18.5 us for
@@ -505,6 +514,10 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                 break;
             }
         }
+        int64_t points = 0;
+        for (int64_t q = 0; q < n; ++q)
+            points += (int64_t)probs[q].nx * probs[q].ny;
+        fold_b = points <= FOLD_POINTS;
         adi_res = line_solver == LINE_PARTITIONED && !euler && fpat != PAT_GENERIC;
         for (int64_t q = 0; q < n && adi_res; ++q)
             adi_res = resident_ok(probs[q], n);
@@ -535,9 +548,9 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
                         for (int c = 0; c < p.ny; c += cols)
                             tiles[tb].push_back({(int32_t)q, r, std::min(rows, p.nx - r), c});
                 } else {
-                    // exact plans lay their v-line tiles out from the last row: the tile that ends there holds the
-                    // two rows that boundary stage B extrapolates from
-                    const int first = tb == TB_V && line_solver == LINE_EXACT ? (hi - lo) % step : 0;
+                    // the v-line tiles are laid out from the last row: the tile that ends there holds the two rows
+                    // that boundary stage B extrapolates from
+                    const int first = tb == TB_V || tb == TB_V16 ? (hi - lo) % step : 0;
                     if (first)
                         tiles[tb].push_back({(int32_t)q, lo, first, 0});
                     for (int s = lo + first; s < hi; s += step) {
@@ -676,8 +689,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     {
         const int tb = VR == 4 ? TB_V : TB_V16;
         const dim3 g((unsigned)pre(tb, na)), b(64 * VR);
-        hipLaunchKernelGGL((k_vsweep_p<T, M, VR, PAT>), g, b, 0, st, pd, (const Tile *)tiles_dev.p + toff(tb),
-                           s, stage, swz);
+        const Tile *tp = (const Tile *)tiles_dev.p + toff(tb);
+        if (bnd_in_v)
+            hipLaunchKernelGGL((k_vsweep_b<T, M, VR, PAT>), g, b, 0, st, pd, tp, s, stage, swz);
+        else
+            hipLaunchKernelGGL((k_vsweep_p<T, M, VR, PAT>), g, b, 0, st, pd, tp, s, stage, swz);
     }
     template <int M, int VR> void launch_v_m(int stage, int s, hipStream_t st, const Prob<T> *pd, int64_t na)
     {
@@ -879,9 +895,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         const Prob<T> *pd = table ? table : (const Prob<T> *)probs_dev.p;
         const Tile *td = (const Tile *)tiles_dev.p;
         auto grid = [&](int tb) { return (unsigned)pre(tb, na); };
-        bool any_split2 = false;
-        for (int64_t q = slice_q0; q < na; ++q)
+        bool any_split2 = false, any_dr = false;
+        for (int64_t q = slice_q0; q < na; ++q) {
             any_split2 |= probs[q].scheme != SCHEME_DR;
+            any_dr |= probs[q].scheme == SCHEME_DR;
+        }
         auto pre = [&](int k) {
             if (prof)
                 prof->begin(k, algo_bytes(k, na));
@@ -920,9 +938,13 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         pre(LSS_K_XSWEEP1);
         xs(1);
         post();
+        // (a profiled run keeps stage B's launch of its own, and so its time)
+        const bool fold = fold_b && !prof && line_solver == LINE_PARTITIONED;
+        bnd_in_v = fold && any_dr;
         pre(LSS_K_VSWEEP1);
         vs(1);
         post();
+        bnd_in_v = fold;
         if (any_split2) {
             pre(LSS_K_XSWEEP2);
             xs(2);
@@ -931,7 +953,8 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             vs(2);
             post();
         }
-        if (line_solver == LINE_EXACT)
+        bnd_in_v = false;
+        if (line_solver == LINE_EXACT || fold)
             return;  // (the last v-sweep evaluated stage B)
         pre(LSS_K_BND_B);
         hipLaunchKernelGGL(k_bnd_b<T>, dim3(grid(TB_J)), dim3(TILE), 0, st, pd, td + toff(TB_J), s);

@@ -21,22 +21,6 @@
 
 namespace lssamd {
 
-// -------------------------------------------------------------------------------------------------
-// Boundary stage B: row 0 Dirichlet, row nx-1 Neumann extrapolation through idx2 (explicit_boundary.hpp:202-238)
-// -------------------------------------------------------------------------------------------------
-template <typename T> __device__ __forceinline__ void bnd_b_col(const Prob<T> &p, int step, int j)
-{
-    const int nx = p.nx, ny = p.ny;
-    const gptr<T> nxt = G((step & 1) ? p.a : p.b);
-    const gptr<const T> bs = bnd_set(p, step);
-    const T two = (T)2.0, three = (T)3.0, four = (T)4.0;
-    const uint32_t jj = p.idx2[j];
-    const T e = (((four * nxt[(int64_t)(nx - 2) * ny + jj]) - nxt[(int64_t)(nx - 3) * ny + jj] -
-                  (two * p.h1 * bs[nx + ny + j])) /
-                 three);
-    nxt[j] = bs[nx + j];
-    nxt[(int64_t)(nx - 1) * ny + j] = e;
-}
 template <typename T>
 __global__ void __launch_bounds__(TILE) k_bnd_b(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles,
                                                 int step)

@@ -123,6 +123,34 @@ k_vsweep_p(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles, in
     vsweep_lines<T, M, VR, PAT, 1>(p, tl, step, stage);
 }
 
+// The last v-sweep of a step with boundary stage B: the tile that ends at row nx - 2, which holds row nx - 3 too (the
+// plan lays its v-line tiles out from the last row), goes on to rows 0 and nx - 1 after a barrier.  A kernel of its own,
+// for the plans that are bound by their launches (PlanImpl::fold_b): in k_vsweep_p the added code slowed the
+// sweeps of large books by a tenth.
+template <typename T, int M, int VR, int PAT>
+__global__ void __launch_bounds__(64 * VR) __attribute__((amdgpu_waves_per_eu(M <= 4 ? 8 : 1)))
+k_vsweep_b(const Prob<T> *__restrict__ probs, const Tile *__restrict__ tiles, int step, int stage, int swz)
+{
+    const Tile tl = tiles[swz ? xcd_tile(blockIdx.x, gridDim.x) : blockIdx.x];
+    const Prob<T> &p = probs[tl.prob];
+    if (step >= p.steps || (stage == 2 && p.scheme == SCHEME_DR))
+        return;  // uniform over the workgroup
+    bool done = false;
+    if constexpr (M <= 4) {
+        if (vlines_per_wave(p.ny - 2, M) == 2) {
+            vsweep_lines<T, M, VR, PAT, 2>(p, tl, step, stage);
+            done = true;
+        }
+    }
+    if (!done)
+        vsweep_lines<T, M, VR, PAT, 1>(p, tl, step, stage);
+    if ((stage == 2 || p.scheme == SCHEME_DR) && tl.first + tl.count == p.nx - 1) {
+        __syncthreads();
+        for (int j = (int)threadIdx.x; j < p.ny; j += 64 * VR)
+            bnd_b_col(p, step, j);
+    }
+}
+
 // -------------------------------------------------------------------------------------------------
 // S-line sweep.  STAGE 1: rhs_intermed_1(u) -> Y1.  STAGE 2: CS/MCS rhs_intermed_3(u, Y1, Y2) -> Y3;
 // HV rhs_intermed_4(Y2, Y3) with Y3 evaluated in place from (u, Y1, Y2) -> Y4 (= y4).
@@ -265,6 +293,8 @@ __global__ void __launch_bounds__(W *NC) k_xsweep_p(const Prob<T> *__restrict__ 
 #define LSS_INST_X(T, M, S, W, PAT, NC) \
     template __global__ void k_xsweep_p<T, M, S, W, PAT, NC>(const Prob<T> *, const Tile *, int, int);
 #define LSS_INST_P(T, M, PAT)                                                                                  \
+    template __global__ void k_vsweep_b<T, M, 4, PAT>(const Prob<T> *, const Tile *, int, int, int);            \
+    template __global__ void k_vsweep_b<T, M, 16, PAT>(const Prob<T> *, const Tile *, int, int, int);           \
     template __global__ void k_vsweep_p<T, M, 4, PAT>(const Prob<T> *, const Tile *, int, int, int);            \
     template __global__ void k_vsweep_p<T, M, 16, PAT>(const Prob<T> *, const Tile *, int, int, int);           \
     LSS_INST_X(T, M, 1, 16, PAT, 64) LSS_INST_X(T, M, 2, 16, PAT, 64) LSS_INST_X(T, M, 1, 8, PAT, 64)          \

@@ -198,6 +198,24 @@ template <typename T, int PAT = PAT_GENERIC> __device__ __forceinline__ void bnd
     G(p.colA1)[i] = bs[i];  // v_upper(t, X(zeta_i))
 }
 
+// -------------------------------------------------------------------------------------------------
+// Boundary stage B: row 0 Dirichlet, row nx-1 Neumann extrapolation through idx2 (explicit_boundary.hpp:202-238)
+// -------------------------------------------------------------------------------------------------
+template <typename T> __device__ __forceinline__ void bnd_b_col(const Prob<T> &p, int step, int j)
+{
+#pragma clang fp contract(off)
+    const int nx = p.nx, ny = p.ny;
+    const gptr<T> nxt = G((step & 1) ? p.a : p.b);
+    const gptr<const T> bs = bnd_set(p, step);
+    const T two = (T)2.0, three = (T)3.0, four = (T)4.0;
+    const uint32_t jj = p.idx2[j];
+    const T e = (((four * nxt[(int64_t)(nx - 2) * ny + jj]) - nxt[(int64_t)(nx - 3) * ny + jj] -
+                  (two * p.h1 * bs[nx + ny + j])) /
+                 three);
+    nxt[j] = bs[nx + j];
+    nxt[(int64_t)(nx - 1) * ny + j] = e;
+}
+
 // Two-dimensional point accessors: in(di, dj) is the value at (i + di, j + dj) of the point (i, j).
 // PAt: a pointer at the point and the row stride.  GRC: a global base, the point's row k and column
 // j; every access forms the offset of its row, min(k + di, kmax) * ny, so that neighbouring points

@@ -447,3 +447,25 @@ def test_resident_loop_matches_the_oracle(oracle, fp, model, nx, ny, count):
             short = L.Plan.from_models([models[p]], fp).run_levels_host([plan.initial(p)])[0]
             assert _normwise(levels[p].cpu().numpy().astype(np.float64), short.astype(np.float64)) <= tol
     plan.close()
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("nx,ny", [(4, 4), (5, 70), (6, 130), (19, 34), (131, 66), (150, 260)])
+def test_boundary_stage_in_the_last_v_sweep_equals_its_own_launch(fp, nx, ny):
+    """Plans of few points evaluate boundary stage B in the step's last v-sweep; a profiled run keeps its launch.  The
+    same kernels otherwise: within the partitioned solver's tolerance (1e-12, fp32 1e-5 of the largest value).  The
+    150 x 40 problem keeps the plan off the resident loop."""
+    torch = pytest.importorskip("torch")
+    models = [_stable(nx, ny, steps=3 + q, splitting=q % 4, coeff_mode=L.COEFF_SEPARABLE, line_solver=L.LINE_PARTITIONED)
+              for q in range(4)] + [_stable(150, 40, steps=4, coeff_mode=L.COEFF_SEPARABLE, line_solver=L.LINE_PARTITIONED)]
+    plan = L.Plan.from_models(models, fp)
+    ins = [torch.from_numpy(plan.initial(p)).cuda() for p in range(plan.count)]
+    outs, own = ([torch.full_like(u, float("nan")) for u in ins] for _ in range(2))
+    pin = [u.data_ptr() for u in ins]
+    plan.run_dev(pin, [o.data_ptr() for o in outs])
+    L.run_profiled(plan, pin, [o.data_ptr() for o in own], torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    tol = 1e-12 if fp == L.FP64 else 1e-5
+    for a, b in zip(outs, own):
+        assert _normwise(a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)) <= tol
+    plan.close()
