@@ -85,8 +85,11 @@ __device__ __forceinline__ void quad_stages(int g0, int ng, int dg, Load &&load,
 }
 
 // s_t = (f_t - a_t s_{t-1}) / beta_t, y = RN(1 / beta) (NaN for a divisor outside quick_div's range), carry = the s
-// before the group; returns the group's last s.  `seen` gathers the numerators: while seen.ok() every value is the
-// correctly rounded quotient, otherwise the sweep has to run again with QUICK = false (divisions).
+// before the group; returns the group's last s.  `seen` gathers the numerators and each lane's last quotient: while
+// seen_ok() every value is the correctly rounded quotient, otherwise the sweep has to run again with QUICK = false
+// (divisions) from a carry that was found good.  A divisor outside the range makes its own quotient NaN; inside a lane
+// the next point's numerator shows that, and the lane's last quotient has to be looked at itself (the group's last one
+// meets no other numerator of the group).
 struct SeenNum {
     uint32_t lo = 0xffffffffu, hi = 0;  // range of the high words without their sign (a zero counts in neither)
     int32_t sg = 0;                     // smallest high word as an integer: INT32_MIN means -0
@@ -102,6 +105,9 @@ struct SeenNum {
         hi = max(hi, m + 1u);
         sg = min(sg, (int32_t)w);
     }
+    // a quotient: only NaN counts (and what lies far above the numerators' range)
+    __device__ __forceinline__ void add_quotient(double v) { hi = max(hi, (uint32_t)__double2hiint(v) & 0x7fffffffu); }
+    __device__ __forceinline__ void add_quotient(float v) { hi = max(hi, __float_as_uint(v) & 0x7fffffffu); }
 };
 __device__ __forceinline__ bool seen_ok(const SeenNum &s, double)
 {
@@ -137,6 +143,7 @@ __device__ __forceinline__ T quad_forward(const T (&a)[4], const T (&f)[4], cons
 #pragma unroll
                 for (int j = 0; j < 4; ++j)
                     seen.add(num[j]);
+                seen.add_quotient(x[3]);
             }
         }
     } else {

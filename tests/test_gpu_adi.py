@@ -469,3 +469,51 @@ def test_boundary_stage_in_the_last_v_sweep_equals_its_own_launch(fp, nx, ny):
     for a, b in zip(outs, own):
         assert _normwise(a.cpu().numpy().astype(np.float64), b.cpu().numpy().astype(np.float64)) <= tol
     plan.close()
+
+
+# ---------------------------------------------------------------------------------------------
+# The exact sweeps against the oracle where they divide by a known divisor and where they must not.
+# ---------------------------------------------------------------------------------------------
+def _divisors(m, direction, line):
+    """Divisors of S-line (0) or v-line (1) `line` of a Heston plan on a uniform grid, for one Euler step, in double."""
+    k, h1, h2 = (m.t_hi - m.t_lo) / (m.nt - 1), 1.0 / (m.nx - 1), 1.0 / (m.ny - 1)
+    span, y, pt = m.x_hi - m.x_lo, m.y_hi - m.y_lo, m.accumulation_point
+    w = np.arcsinh(1.0) * (np.arange(1, m.ny - 1) if direction else line) * h2
+    v, dv, ddv = m.y_lo + y * np.sinh(w), y * np.arcsinh(1.0) * np.cosh(w), y * np.arcsinh(1.0) ** 2 * np.sinh(w)
+    if direction == 0:
+        z = np.arange(1, m.nx - 1) * h1
+        c0, c1 = np.arcsinh((m.x_hi - pt) / span), np.arcsinh((m.x_lo - pt) / span)
+        w = c0 * z + c1 * (1 - z)
+        x, dx, ddx = pt + span * np.sinh(w), span * (c0 - c1) * np.cosh(w), span * (c0 - c1) ** 2 * np.sinh(w)
+        diff = 0.5 * v * x * x
+        second, first = k / h1 ** 2 * diff / dx ** 2, k / (2 * h1) * (m.rate * x / dx - diff * ddx / dx ** 3)
+    else:
+        diff = 0.5 * m.sig_sig ** 2 * v
+        second = k / h2 ** 2 * diff / dv ** 2
+        first = k / (2 * h2) * (m.sig_kappa * (m.sig_theta - v) / dv - diff * ddv / dv ** 3)
+    a, b, c = -(second - first), 1.0 + 2.0 * second + 0.5 * k * m.rate, -(second + first)
+    beta = [b[0]]
+    for t in range(1, len(b)):
+        beta.append(b[t] - a[t] * c[t - 1] / beta[-1])
+    return np.array(beta)
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("direction", [0, 1])
+@pytest.mark.parametrize("splitting", range(4))
+def test_a_divisor_out_of_range_in_the_last_row_of_a_line(oracle, fp, direction, splitting):
+    # lines of 16 k interior points whose divisors grow past 2^21 (fp64: 2^101) at the last row only; the S-line with
+    # the largest v, and every v-line
+    ofp, limit = ("f64", 2.0 ** 101) if fp == L.FP64 else ("f32", 2.0 ** 21)
+    over = dict(nx=18, ny=34, nt=3 if splitting == 0 else 2, splitting=splitting, implicit_scheme=L.EULER)
+    line = 32 if direction == 0 else 8
+    ref = _divisors(config0(**over, t_hi=1e12), direction, line)
+    t_hi = 1e12 * limit / np.sqrt(ref[-1] * ref[-2])  # (the divisors grow in proportion to the step)
+    for tri in (L.THOMAS_LU, L.DOUBLE_SWEEP):
+        m = config0(**over, t_hi=t_hi, tridiagonal=tri)
+        beta = _divisors(m, direction, line)
+        assert beta[-1] > limit * 1.003 and (beta[:-1] < limit * 0.997).all()
+        c = oracle_solve(oracle, m, ofp)
+        g = _solve(m, fp)
+        assert np.isfinite(c).all()
+        assert np.array_equal(g, c) and np.array_equal(np.signbit(g), np.signbit(c))

@@ -299,3 +299,53 @@ def test_every_form_of_the_partitioned_kernels(oracle, fp, n):
             e, es = _normwise(outs[z], out), _normwise(surfs[z], surf)
             assert e <= tol and es <= tol, (tc, z, q["lo"], q["hi"], e, es)
         plan.close()
+
+
+# ---------------------------------------------------------------------------------------------
+# Divisors outside the range in which the exact kernel divides by a known divisor (2^-20 .. 2^21 in fp32, 2^-100 ..
+# 2^101 in fp64): one such row in a line, at each of the 16 positions of a group, or in the line's last row.  A
+# wavefront holds 16 problems and takes the division as soon as one of them asks for it, so the 16 problems of a block
+# have their row at the same position.  The oracle divides every row; equality is exact, signs of zeros included.
+# ---------------------------------------------------------------------------------------------
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("tdep", [0, 1])
+@pytest.mark.parametrize("kind", ["large", "small"])
+def test_one_divisor_out_of_range_at_every_position(oracle, fp, kind, tdep):
+    import ctypes
+    rng = np.random.default_rng(23)
+    dt, descr = L.np_dtype(fp), []
+    bits = 22 if fp == L.FP32 else 102
+    for row in [*range(16, 32), -1]:
+        for z in range(16):
+            lo, hi = z % 3, (z // 3) % 3
+            if row < 0 and hi == L.BC_DIRICHLET:
+                hi = L.BC_ROBIN  # (the last row has a divisor of its own)
+            q = _descr(ctypes, fp, 48 if row < 0 else 33 + 2 * z, 3, (L.THOMAS_LU, L.DOUBLE_SWEEP)[z % 2], lo, hi,
+                       L.FORWARD, tdep, 0, 0, 0.5, rng)
+            A, B, D = q["coeff"][:, 0], q["coeff"][:, 1], q["coeff"][:, 2]
+            if kind == "large":  # diagonal 1 + B
+                B[:, row] = 2.0 ** bits
+            else:  # diagonal 0: the divisor is what elimination leaves
+                B[:, row] = -1.0
+                A[:, row] *= dt(2.0 ** -bits)
+                if row < 0:
+                    D[:, row] = 0.0
+                    q["bnd"][:, 2] = 0.0
+            descr.append(q)
+    plan = _described_plan(ctypes, descr, L.LINE_EXACT)
+    outs = plan.run_host([q["u0"] for q in descr])
+    for z, q in enumerate(descr):
+        out = _stepped(oracle, q)[1]
+        assert np.isfinite(out).all()
+        assert np.array_equal(outs[z], out) and np.array_equal(np.signbit(outs[z]), np.signbit(out)), (z // 16, z % 16)
+    plan.close()
+
+
+@pytest.mark.parametrize("n,sig", [(8001, 0.41), (10000, 0.46)])
+def test_a_fine_fp32_line_whose_diagonal_grows_past_the_range(oracle, n, sig):
+    m = H.BsModel(n=n, nt=2, rate=0.05, sig=sig, implicit_scheme=L.EULER)
+    plan = H.Heat1dPlan.from_bs_models([m], L.FP32)
+    out = plan.run_host()[0]
+    plan.close()
+    assert np.isfinite(out).all()
+    assert np.array_equal(out, _oracle(oracle, m, "f32"))
