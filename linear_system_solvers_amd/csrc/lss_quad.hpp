@@ -32,14 +32,17 @@ template <int Q> constexpr int QUAD_BCAST = Q * 0x55;      // every lane takes l
 // 1990: q' = RN(q + r y) with r = a - b q is the correctly rounded quotient when q is faithful and
 // y = RN(1 / b)).  Four dependent operations instead of the ten of an IEEE division.  It holds while no
 // intermediate value leaves the normal range: the exponents of a and b are bounded so that 1 / b, the quotients
-// and the residuals (multiples of ulp(b) ulp(q)) are normal or exact.  A numerator of +0 gives the right signed
-// zero; everything else takes the division.
+// and the residuals (multiples of ulp(b) ulp(q)) are normal or exact.  A numerator of +0 gives +0, which is right for
+// positive divisors (a y = +0, and +0 + a z = +0 for either sign of z); for negative ones it would depend on the sign
+// of z, so they take the division, as everything else does.
 // -------------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t exponent_of(double x) { return (uint32_t)__double2hiint(x) >> 20 & 0x7ffu; }
-__device__ __forceinline__ uint32_t exponent_of(float x) { return __float_as_uint(x) >> 23 & 0xffu; }
-// divisors 2^-100 .. 2^100 (fp32: 2^-20 .. 2^20), numerators 2^-900 .. 2^900 (2^-90 .. 2^90) or +0
-__device__ __forceinline__ bool quick_div_ok(double b) { return exponent_of(b) - (1023u - 100u) <= 200u; }
-__device__ __forceinline__ bool quick_div_ok(float b) { return exponent_of(b) - (127u - 20u) <= 40u; }
+// sign and exponent (a negative number lies above every positive one)
+__device__ __forceinline__ uint32_t sign_exponent(double x) { return (uint32_t)__double2hiint(x) >> 20; }
+__device__ __forceinline__ uint32_t sign_exponent(float x) { return __float_as_uint(x) >> 23; }
+// divisors from 2^-100 to below 2^101 (fp32: 2^-20 to below 2^21), numerators from +-2^-900 to below 2^900 (2^-90, 2^90)
+// or +0
+__device__ __forceinline__ bool quick_div_ok(double b) { return sign_exponent(b) - (1023u - 100u) <= 200u; }
+__device__ __forceinline__ bool quick_div_ok(float b) { return sign_exponent(b) - (127u - 20u) <= 40u; }
 // y = RN(1 / b) and its correction z = y (1 - b y)
 __device__ __forceinline__ double quick_div(double a, double b, double y, double z)
 {

@@ -349,3 +349,27 @@ def test_a_fine_fp32_line_whose_diagonal_grows_past_the_range(oracle, n, sig):
     plan.close()
     assert np.isfinite(out).all()
     assert np.array_equal(out, _oracle(oracle, m, "f32"))
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+def test_negative_divisors_keep_the_sign_of_zero(oracle, fp):
+    # zero levels and negative diagonals: the quotients are zeros whose signs are the divisors'
+    import ctypes
+    rng = np.random.default_rng(29)
+    dt, descr = L.np_dtype(fp), []
+    for z in range(64):
+        q = _descr(ctypes, fp, 17 + z, 3, (L.THOMAS_LU, L.DOUBLE_SWEEP)[z % 2], z % 3, (z // 3) % 3, L.FORWARD, 0, 0, 0, 1.0,
+                   rng)
+        q["coeff"][:, 1] = -rng.uniform(1.1, 4.0, q["coeff"][:, 1].shape).astype(dt)  # diagonal 1 + 2 B < 0
+        q["coeff"][:, (0, 2)] *= dt(0.1)
+        keep = rng.uniform(size=q["n"]) < 0.2 * (z % 2)
+        q["u0"] = np.where(keep, q["u0"], dt(0.0)).astype(dt)
+        q["bnd"][:] = 0.0
+        descr.append(q)
+    plan = _described_plan(ctypes, descr, L.LINE_EXACT)
+    outs, surfs = plan.run_host([q["u0"] for q in descr], surfaces=True)
+    for z, q in enumerate(descr):
+        surf, out = _stepped(oracle, q)
+        assert np.array_equal(outs[z], out) and np.array_equal(surfs[z], surf)
+        assert np.array_equal(np.signbit(surfs[z]), np.signbit(surf)), (z, q["n"])
+    plan.close()
