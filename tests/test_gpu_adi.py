@@ -517,3 +517,27 @@ def test_a_divisor_out_of_range_in_the_last_row_of_a_line(oracle, fp, direction,
         g = _solve(m, fp)
         assert np.isfinite(c).all()
         assert np.array_equal(g, c) and np.array_equal(np.signbit(g), np.signbit(c))
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("rate", [0.02, -9.0])
+@pytest.mark.parametrize("scale", [1.0, 0.0, -0.0, 1e-25, 1e-30, 1e-42, 1e-280, 1e-310, 1e25, 1e30, 1e290])
+def test_exact_sweeps_round_like_the_oracle_at_any_magnitude(oracle, fp, rate, scale):
+    # one step of surfaces whose values are huge, tiny, subnormal or zeros of either sign, also mixed with ordinary
+    # values (rate -9: negative diagonals too); every bit must be the oracle's
+    from tests.helpers import oracle_cfg, oracle_pde
+    dt, ofp = L.np_dtype(fp), "f64" if fp == L.FP64 else "f32"
+    rng = np.random.default_rng(3)
+    for z in range(8):
+        m = config0(nx=37, ny=21, nt=2, rate=rate, splitting=z % 4, tridiagonal=(L.THOMAS_LU, L.DOUBLE_SWEEP)[z // 4],
+                    implicit_scheme=L.EULER if z % 2 else L.THETA_80, weighting=0.3)
+        with np.errstate(over="ignore", under="ignore"):
+            u = (rng.standard_normal((37, 21)) * scale).astype(dt)
+            if z % 3 == 0:
+                u = np.where(rng.uniform(size=u.shape) < 0.3, rng.standard_normal(u.shape).astype(dt), u)
+        plan = L.Plan.from_models([m], fp)
+        g = plan.run_host([u])[0]
+        plan.close()
+        with np.errstate(all="ignore"):
+            c = oracle.step(oracle_pde(oracle, m), oracle_cfg(oracle, m), u, 0.0, ofp)  # (its data do not see the time)
+        assert np.array_equal(g, c, equal_nan=True) and np.array_equal(np.signbit(g[g == 0]), np.signbit(c[c == 0])), z
