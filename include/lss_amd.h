@@ -214,6 +214,12 @@ int lss_plan_problem_shape(const lss_adi_plan *plan, int64_t p, int64_t *nx, int
  * partitioned elimination with no scratch; longer ones one lane per system, with B*n values of scratch
  * allocated on `stream` (stream-ordered, hipMallocAsync) and freed on it after the solve, so that calls on
  * different streams never share scratch.
+ * The partitioned elimination starts at the first row of every chunk of a system and takes reciprocals in the
+ * normal range: it is sound for rows that dominate, |a_i| + |c_i| <= |b_i| once the ends are folded.  Longer
+ * systems (contiguous: more than 512 unknowns in fp64, 1024 in fp32; strided: more than 1024) are looked at row
+ * by row, and those that do not dominate, or whose |b_i| leave 2^-900..2^900 (fp32 2^-100..2^100), are swept in
+ * the reference's order with divisions, rounding for rounding, several times slower.  Shorter systems are not
+ * looked at: there the chunks' first diagonals must not vanish.
  */
 int lss_tridiag_batched(int32_t fp, int32_t layout, int64_t B, int64_t n, const void *a, const void *b,
                         const void *c, const void *d, void *x, void *stream);

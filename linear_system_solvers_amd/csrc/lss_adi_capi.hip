@@ -52,6 +52,8 @@ template <typename T, int M>
 __global__ void k_tridiag_rows(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
 template <typename T, int M, int W, int NC>
 __global__ void k_tridiag_cols(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
+template <typename T, int C, int W, int NC>
+__global__ void k_tridiag_cols_long(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
 template <typename T, int NTMAX>
 __global__ void k_tridiag_long(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
 constexpr int P_NCH = 64, P_XTJ = 16, P_VROWS = 4;
@@ -2162,6 +2164,11 @@ template <int M, int W, int NC, typename T> void tridiag_cols(const TriArgs<T> &
     hipLaunchKernelGGL((k_tridiag_cols<T, M, W, NC>), dim3((unsigned)((t.B + W - 1) / W)), dim3(W * NC), 0, t.st, t.B,
                        t.n, t.a, t.b, t.c, t.d, t.x, t.bc);
 }
+template <int C, int W, int NC, typename T> void tridiag_cols_long(const TriArgs<T> &t)
+{
+    hipLaunchKernelGGL((k_tridiag_cols_long<T, C, W, NC>), dim3((unsigned)((t.B + W - 1) / W)), dim3(W * NC), 0, t.st,
+                       t.B, t.n, t.a, t.b, t.c, t.d, t.x, t.bc);
+}
 
 // Threads of k_tridiag_long for nf unknowns (TRI_LONG_C each, whole wavefronts), or 0 when the system does
 // not fit a workgroup or its one staged array does not fit 64 KiB of LDS (more than 7168 unknowns in fp64,
@@ -2229,7 +2236,7 @@ template <typename T> bool tridiag_part_cols(const TriArgs<T> &t, int64_t nf)
         else if (nf <= 1024)
             tridiag_cols<16, 16, 64>(t);
         else if (nf <= 2048)
-            tridiag_cols<16, 8, 128>(t);
+            tridiag_cols_long<16, 8, 128>(t);
         else
             return false;
     } else {
@@ -2244,7 +2251,7 @@ template <typename T> bool tridiag_part_cols(const TriArgs<T> &t, int64_t nf)
         else if (nf <= 1024)
             tridiag_cols<8, 8, 128>(t);
         else if (nf <= 2048)
-            tridiag_cols<16, 4, 128>(t);
+            tridiag_cols_long<16, 4, 128>(t);
         else
             return false;
     }

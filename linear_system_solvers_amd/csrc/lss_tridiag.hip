@@ -11,11 +11,12 @@
 //   k_tridiag_long  contiguous systems too long for one wavefront: one workgroup per system.
 //   k_tridiag_cols  strided layout x[i*B + k]: W systems x NC chunks per workgroup, so that each access
 //                   reads W consecutive systems of one row.
+//   k_tridiag_cols_long  the same for more than 1024 unknowns.
 //
-// Memory bounds all three (5 values moved per unknown).  Measured on one MI355X, where a 4 + 4 GiB copy
-// reaches 4.8 TB/s: rows 65536 x 256 fp64 5.4 TB/s; long 1000 x 2000 fp64 16.3 us (4.9 TB/s; one lane per
-// system took 3380 us), 8388 x 2000 5.5 TB/s; cols 12289 x 509 fp32 38 us (3.3 TB/s; 53 us in launch
-// order).
+// Memory bounds them (5 values moved per unknown), the long ones also the registers of their last pass.  Measured on
+// one MI355X, where a 4 + 4 GiB copy reaches 4.8 TB/s: rows 65536 x 256 fp64 5.4 TB/s; long 1000 x 2000 fp64 19.2 us
+// (4.2 TB/s; one lane per system took 3380 us), 8388 x 2000 131 us (5.1 TB/s); cols 12289 x 509 fp32 38 us (3.3 TB/s;
+// 53 us in launch order).
 
 // The fast path may fuse multiply-adds (the library is built with -ffp-contract=off so that the exact
 // line solver keeps the reference's rounding; this translation unit opts back in).
@@ -111,15 +112,167 @@ __global__ void __launch_bounds__(W *NC) k_tridiag_cols(int64_t B, int n, const 
     }
 }
 
-// Contiguous systems too long for one wavefront: one workgroup per system, a thread holds TRI_LONG_C
-// consecutive unknowns.  All loads of the four arrays are coalesced rows of the workgroup, issued together;
-// each array then passes through LDS once to reach the thread that owns its points (positions padded by one
-// per chunk, so that neither side meets a bank conflict), so LDS holds one array and not four.  The interface
-// system (one equation per thread) is reduced by cyclic reduction in the same LDS.
+// -------------------------------------------------------------------------------------------------
+// Long systems: a workgroup holds W systems, position pos of a system (np of them) the C consecutive unknowns from
+// pos * C on.  The chunks are eliminated and their interface system (one equation per position) is reduced by cyclic
+// reduction in LDS.
+//
+// All this is sound while the rows dominate, |a| + |c| <= |b|: then so do the rows that any elimination leaves, in
+// whatever order, and no multiplier exceeds 1.  A system with a row that does not
+// dominate, or whose diagonal leaves the range that fast_rcp and a few sums need, is swept as the reference sweeps it
+// instead, with divisions, position after position (the result of one lane per system, bit for bit).  The threads
+// still share the loads and the other systems' work: 1000 systems of 2000 unknowns in fp64 take 0.50 ms, 8388 of them
+// 3.2 ms (one lane per system: 3.5 and 3.7), interleaved 0.27 and 2.1 ms (1.6 and 2.05).
+// -------------------------------------------------------------------------------------------------
+__device__ __forceinline__ bool dominates(double a, double b, double c)
+{
+    const double m = fabs(b);
+    return (fabs(a) + fabs(c) <= m * (1 + 0x1p-49)) & (m >= 0x1p-900) & (m <= 0x1p900);
+}
+__device__ __forceinline__ bool dominates(float a, float b, float c)
+{
+    const float m = fabsf(b);
+    return (fabsf(a) + fabsf(c) <= m * (1 + 0x1p-20f)) & (m >= 0x1p-100f) & (m <= 0x1p100f);
+}
+// Zero, of which the compiler does not know: rows at an offset from it are read again (from the caches), not kept in
+// registers from the elimination on.
+__device__ __forceinline__ int opaque_zero()
+{
+    int v = 0;
+    asm volatile("" : "+s"(v));
+    return v;
+}
+
+// LDS values of long_solve: six per position and system, and a flag per system, not 0 if it is to be swept
+__host__ __device__ constexpr int long_lds(int np, int W) { return (6 * np + 1) * W; }
+template <typename T> __device__ __forceinline__ T *long_flag(T *sh, int np, int W) { return sh + 6 * np * W; }
+
+// The sequential sweep of the systems of which `mine` is set (thomas_lu_solver.hpp:125-191)
+template <typename T, int C, typename Row>
+__device__ __forceinline__ void long_sweep(T *sh, int W, int pos, int col, int nf, bool mine, Row &&row, T (&x)[C])
+{
+#pragma clang fp contract(off)
+    const int npos = (nf + C - 1) / C;
+    Eq<T> e[C];  // at hand before the position's turn comes; c becomes gamma
+    if (mine) {
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+            e[j] = row(j);
+    }
+    __syncthreads();
+    for (int p = 0; p < npos; ++p) {
+        if (mine && pos == p) {
+            T gk = p ? sh[col] : (T)0, sk = p ? sh[W + col] : (T)0;
+#pragma unroll
+            for (int j = 0; j < C; ++j) {
+                if (p * C + j >= nf)
+                    continue;
+                const T beta = e[j].b - (e[j].a * gk);
+                e[j].c = gk = e[j].c / beta;
+                x[j] = sk = (e[j].r - (e[j].a * sk)) / beta;
+            }
+            sh[col] = gk;
+            sh[W + col] = sk;
+        }
+        __syncthreads();
+    }
+    for (int p = npos - 1; p >= 0; --p) {
+        if (mine && pos == p) {
+            T xk = sh[2 * W + col];
+#pragma unroll
+            for (int j = C - 1; j >= 0; --j) {
+                if (p * C + j >= nf)
+                    continue;
+                if (p * C + j < nf - 1)
+                    x[j] = x[j] - (e[j].c * xk);
+                xk = x[j];
+            }
+            sh[2 * W + col] = xk;
+        }
+        __syncthreads();
+    }
+}
+
+// Solves for the unknowns x of position pos, whose rows are row(0) .. row(C - 1) (ends folded, identity rows past the
+// end; not asked for where `holds` is not set: a position without rows), sh may
+// be in use by the caller until then.  Every thread of the workgroup calls it (it holds barriers).  Returns whether some system of the workgroup is flagged.
+template <typename T, int C, typename Row>
+__device__ __forceinline__ bool long_solve(T *sh, int np, int W, int pos, int col, bool holds, Row &&row, T (&x)[C])
+{
+    const int st = np * W, at = pos * W + col;
+    T *const flag = long_flag(sh, np, W);
+    const int prev = pos > 0 ? at - W : at, next = pos + 1 < np ? at + W : at;
+    {
+        Chunk<T, C> ch;
+        bool good = true;
+        if (holds) {
+#pragma unroll
+            for (int j = 0; j < C; ++j) {
+                const Eq<T> e = row(j);
+                good &= dominates(e.a, e.b, e.c);
+                ch.put(j, e);
+            }
+            ch.bwd();
+        } else {
+            ch.set_identity();
+        }
+        T PF, QF, RF;
+        ch.first_rel(PF, QF, RF);
+        __syncthreads();
+        sh[at] = PF;
+        sh[st + at] = QF;
+        sh[2 * st + at] = RF;
+        if (pos == 0)
+            flag[col] = (T)0;
+        __syncthreads();
+        if (!good)
+            flag[col] = (T)1;
+        // (a position without a neighbour reads its own row: its coupling to that side is exactly zero)
+        const T nPF = sh[next], nQF = sh[st + next], nRF = sh[2 * st + next];
+        Eq<T> e = ch.interface_eq(nPF, nQF, nRF);
+        T *cur = sh + 3 * st, *oth = sh;
+        {
+            const NEq<T> m = normalized(e);
+            cur[at] = m.a;
+            cur[st + at] = m.c;
+            cur[2 * st + at] = m.r;
+        }
+        __syncthreads();
+        for (int dd = 1; dd < np; dd <<= 1) {
+            const int tl = pos >= dd ? at - dd * W : at, th = pos + dd < np ? at + dd * W : at;
+            const NEq<T> l{cur[tl], cur[st + tl], cur[2 * st + tl]}, h{cur[th], cur[st + th], cur[2 * st + th]};
+            e = pcr_step(e, l, h);
+            T *s = cur;
+            cur = oth;
+            oth = s;
+            const NEq<T> m = normalized(e);
+            cur[at] = m.a;
+            cur[st + at] = m.c;
+            cur[2 * st + at] = m.r;
+            __syncthreads();
+        }
+        const T xi = e.r * fast_rcp(e.b);
+        oth[at] = xi;
+        __syncthreads();
+        const T xl = oth[prev];
+#pragma unroll
+        for (int j = 0; j < C; ++j)
+            x[j] = ch.value(j, xl, xi);
+    }
+    bool any = false;
+    for (int w = 0; w < W; ++w)
+        any = any || flag[w] != (T)0;
+    return any;
+}
+
+// Contiguous systems too long for one wavefront: one workgroup per system.  All loads of the four arrays are coalesced
+// rows of the workgroup, issued together; each array then passes through LDS once to reach the thread that owns its
+// points (positions padded by one per chunk, so that neither side meets a bank conflict), so LDS holds one array and not
+// four.
 template <typename T, int NTMAX>
-__global__ void __launch_bounds__(NTMAX) k_tridiag_long(int64_t B, int n, const T *__restrict__ a,
-                                                        const T *__restrict__ b, const T *__restrict__ c,
-                                                        const T *__restrict__ d, T *__restrict__ x, LineBC<T> bc)
+__global__ void __launch_bounds__(NTMAX)
+k_tridiag_long(int64_t B, int n, const T *__restrict__ a, const T *__restrict__ b, const T *__restrict__ c,
+               const T *__restrict__ d, T *__restrict__ x, LineBC<T> bc)
 {
     constexpr int C = TRI_LONG_C;
     extern __shared__ unsigned char lds_raw[];
@@ -152,68 +305,26 @@ __global__ void __launch_bounds__(NTMAX) k_tridiag_long(int64_t B, int n, const 
     spread(vb);
     spread(vc);
     spread(vd);
-    Chunk<T, C> ch;
-#pragma unroll
-    for (int j = 0; j < C; ++j) {
+    auto own = [&](int j) {
         const int k = t * C + j;
-        Eq<T> e;
-        e.a = va[j];
-        e.b = vb[j];
-        e.c = vc[j];
-        e.r = vd[j];
+        Eq<T> e{va[j], vb[j], vc[j], vd[j]};
         bc.fold(k == 0, k == nf - 1, e.a, e.b, e.c, e.r);
-        if (k >= nf)
-            e = identity_eq<T>();
-        ch.put(j, e);
-    }
-    ch.bwd();
-    {
-        T PF, QF, RF;
-        ch.first_rel(PF, QF, RF);
-        __syncthreads();
-        sh[t] = PF;
-        sh[nt + t] = QF;
-        sh[2 * nt + t] = RF;
-    }
-    __syncthreads();
-    // (a thread without a neighbour reads its own row: its coupling to that side is exactly zero)
-    const int tn = t + 1 < nt ? t + 1 : t;
-    Eq<T> e = ch.interface_eq(sh[tn], sh[nt + tn], sh[2 * nt + tn]);
-    T *cur = sh + 3 * nt, *oth = sh;
-    {
-        const NEq<T> m = normalized(e);
-        cur[t] = m.a;
-        cur[nt + t] = m.c;
-        cur[2 * nt + t] = m.r;
-    }
-    __syncthreads();
-    for (int dd = 1; dd < nt; dd <<= 1) {
-        const int tl = t >= dd ? t - dd : t, th = t + dd < nt ? t + dd : t;
-        NEq<T> l, h;
-        l.a = cur[tl];
-        l.c = cur[nt + tl];
-        l.r = cur[2 * nt + tl];
-        h.a = cur[th];
-        h.c = cur[nt + th];
-        h.r = cur[2 * nt + th];
-        e = pcr_step(e, l, h);
-        T *s = cur;
-        cur = oth;
-        oth = s;
-        const NEq<T> m = normalized(e);
-        cur[t] = m.a;
-        cur[nt + t] = m.c;
-        cur[2 * nt + t] = m.r;
-        __syncthreads();
-    }
-    const T xi = e.r * fast_rcp(e.b);
-    oth[t] = xi;
-    __syncthreads();
-    const T xl = oth[t > 0 ? t - 1 : 0];
+        return k < nf ? e : identity_eq<T>();
+    };
+    T v[C];
+    const bool sweep = long_solve<T, C>(sh, nt, 1, t, 0, t * C < nf, own, v);
+    auto again = [&](int k, int64_t from) {
+        const int64_t q = from + min(k, nf - 1);
+        Eq<T> e{a[q], b[q], c[q], d[q]};
+        bc.fold(k == 0, k >= nf - 1, e.a, e.b, e.c, e.r);
+        return e;
+    };
+    if (sweep)
+        long_sweep<T, C>(sh, 1, t, 0, nf, true, [&](int j) { return again(t * C + j, base + s0 + opaque_zero()); }, v);
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < C; ++j)
-        sh[t * (C + 1) + j] = ch.value(j, xl, xi);
+        sh[t * (C + 1) + j] = v[j];
     __syncthreads();
 #pragma unroll
     for (int j = 0; j < C; ++j) {
@@ -229,6 +340,44 @@ __global__ void __launch_bounds__(NTMAX) k_tridiag_long(int64_t B, int n, const 
     }
 }
 
+// Interleaved systems of more than 1024 unknowns: W systems per workgroup, NC positions of C unknowns each.
+template <typename T, int C, int W, int NC>
+__global__ void __launch_bounds__(W *NC) k_tridiag_cols_long(int64_t B, int n, const T *__restrict__ a,
+                                                             const T *__restrict__ b, const T *__restrict__ c,
+                                                             const T *__restrict__ d, T *__restrict__ x, LineBC<T> bc)
+{
+    __shared__ T sh[long_lds(NC, W)];
+    const int col = threadIdx.x % W, pos = threadIdx.x / W;
+    const int64_t k = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * W + col;
+    const bool live = k < B;
+    const int s0 = bc.start(), e0 = bc.end(n), nf = e0 - s0 + 1;
+    const bool holds = live && pos * C < nf;
+    auto load = [&](int j, int64_t at) {
+        const int i = pos * C + j;
+        const int64_t q = (int64_t)(s0 + min(i, nf - 1)) * B + at;
+        Eq<T> e{a[q], b[q], c[q], d[q]};
+        bc.fold(i == 0, i >= nf - 1, e.a, e.b, e.c, e.r);  // (past the end the last row again, its c zero too)
+        return e;
+    };
+    T v[C];
+    const bool any = long_solve<T, C>(sh, NC, W, pos, col, holds, [&](int j) { return load(j, k); }, v);
+    const bool mine = holds && long_flag(sh, NC, W)[col] != (T)0;
+    if (any)
+        long_sweep<T, C>(sh, W, pos, col, nf, mine, [&](int j) { return load(j, k + opaque_zero()); }, v);
+    if (!live)
+        return;
+#pragma unroll
+    for (int j = 0; j < C; ++j)
+        if (pos * C + j < nf)
+            x[(int64_t)(s0 + pos * C + j) * B + k] = v[j];
+    if (pos == 0) {
+        if (bc.lo == BC_DIRICHLET)
+            x[k] = bc.lo_val;
+        if (bc.hi == BC_DIRICHLET)
+            x[(int64_t)(n - 1) * B + k] = bc.hi_val;
+    }
+}
+
 #define LSS_INST_R(T, M) \
     template __global__ void k_tridiag_rows<T, M>(int64_t, int, const T *, const T *, const T *, const T *, T *, LineBC<T>);
 #define LSS_INST_C(T, M, W, NC)                                                                                     \
@@ -237,6 +386,9 @@ __global__ void __launch_bounds__(NTMAX) k_tridiag_long(int64_t B, int n, const 
 #define LSS_INST_L(T, NTMAX)                                                                                         \
     template __global__ void k_tridiag_long<T, NTMAX>(int64_t, int, const T *, const T *, const T *, const T *, T *, \
                                                       LineBC<T>);
+#define LSS_INST_CL(T, C, W, NC)                                                                                         \
+    template __global__ void k_tridiag_cols_long<T, C, W, NC>(int64_t, int, const T *, const T *, const T *, const T *, \
+                                                              T *, LineBC<T>);
 #define LSS_INST_T(T)                                                                                               \
     LSS_INST_R(T, 1) LSS_INST_R(T, 2) LSS_INST_R(T, 4) LSS_INST_R(T, 8) LSS_INST_R(T, 16) LSS_INST_L(T, 256) \
     LSS_INST_L(T, 1024)
@@ -247,7 +399,6 @@ LSS_INST_C(double, 2, 16, 64)
 LSS_INST_C(double, 4, 16, 64)
 LSS_INST_C(double, 8, 8, 64)
 LSS_INST_C(double, 8, 8, 128)
-LSS_INST_C(double, 16, 4, 128)
 LSS_INST_C(float, 2, 32, 32)
 LSS_INST_C(float, 4, 32, 32)
 LSS_INST_C(float, 8, 32, 32)
@@ -256,9 +407,11 @@ LSS_INST_C(float, 2, 16, 64)
 LSS_INST_C(float, 4, 16, 64)
 LSS_INST_C(float, 8, 16, 64)
 LSS_INST_C(float, 16, 16, 64)
-LSS_INST_C(float, 16, 8, 128)
+LSS_INST_CL(double, 16, 4, 128)
+LSS_INST_CL(float, 16, 8, 128)
 #undef LSS_INST_R
 #undef LSS_INST_C
+#undef LSS_INST_CL
 #undef LSS_INST_L
 #undef LSS_INST_T
 

@@ -155,3 +155,83 @@ def test_edges_of_the_size_ranges(oracle, fp, layout, n, in_place):
 def test_end_conditions_of_long_systems_match_the_oracle(oracle, fp, layout, n):
     # (with two Dirichlet ends 1026 and 2050 points hold 1024 and 2048 unknowns)
     test_end_conditions_match_the_oracle(oracle, fp, layout, n)
+
+
+# ---------------------------------------------------------------------------------------------
+# Long systems (contiguous: 513..7168 unknowns in fp64, 1025..8192 in fp32; interleaved: 1025..2048) whose rows do not
+# dominate, or whose diagonals have no reciprocal in the normal range, are swept in the reference's order: bit for bit
+# the oracle's values, beside dominant systems of the same batch, which keep the tolerance above.
+# ---------------------------------------------------------------------------------------------
+LONG = [(L.FP64, L.LAYOUT_CONTIGUOUS, 513), (L.FP64, L.LAYOUT_CONTIGUOUS, 600), (L.FP64, L.LAYOUT_CONTIGUOUS, 2048),
+        (L.FP64, L.LAYOUT_CONTIGUOUS, 4100), (L.FP64, L.LAYOUT_CONTIGUOUS, 7168), (L.FP32, L.LAYOUT_CONTIGUOUS, 1025),
+        (L.FP32, L.LAYOUT_CONTIGUOUS, 2047), (L.FP32, L.LAYOUT_CONTIGUOUS, 8192), (L.FP64, L.LAYOUT_STRIDED, 1025),
+        (L.FP64, L.LAYOUT_STRIDED, 2048), (L.FP32, L.LAYOUT_STRIDED, 1031), (L.FP32, L.LAYOUT_STRIDED, 2048)]
+
+
+def _solve_plain(fp, layout, a, b, c, d, in_place=False):
+    torch = pytest.importorskip("torch")
+    B, n = a.shape
+    if layout == L.LAYOUT_STRIDED:
+        a, b, c, d = (np.ascontiguousarray(v.T) for v in (a, b, c, d))
+    ta, tb, tc, td = (torch.from_numpy(np.ascontiguousarray(v)).cuda() for v in (a, b, c, d))
+    tx = td if in_place else torch.full_like(td, float("nan"))
+    L.tridiag_batched(fp, layout, B, n, ta.data_ptr(), tb.data_ptr(), tc.data_ptr(), td.data_ptr(), tx.data_ptr(),
+                      torch.cuda.current_stream().cuda_stream)
+    torch.cuda.synchronize()
+    x = tx.cpu().numpy()
+    return x.T if layout == L.LAYOUT_STRIDED else x
+
+
+@pytest.mark.parametrize("fp,layout,n", LONG)
+@pytest.mark.parametrize("in_place", [False, True])
+def test_long_systems_that_do_not_dominate_equal_the_oracle(oracle, fp, layout, n, in_place):
+    dt, B = L.np_dtype(fp), 13
+    a, b, c, d = _systems(B, n, dt, seed=n)
+    for k, kind in ((1, "zero"), (2, "weaker"), (4, "weak"), (5, "one row"), (7, "tiny"), (8, "huge"), (11, "last row")):
+        if kind == "zero":  # only the first diagonal is not zero: beta = -a gamma
+            b[k, 1:] = 0.0
+            a[k], c[k] = -1.0, 1.0
+        elif kind == "weaker":
+            b[k] = (0.95 * (np.abs(a[k]) + np.abs(c[k])) + 0.01).astype(dt)
+        elif kind == "weak":  # (still dominates: the off-diagonals' sum is below 2)
+            b[k] = (0.9 * (np.abs(a[k]) + np.abs(c[k])) + 0.3).astype(dt)
+        elif kind == "one row":
+            b[k, n // 2] = 0.0
+        elif kind == "tiny":  # (c stays: the solution does not overflow)
+            s = dt(1e-38 if fp == L.FP32 else 1e-305)
+            a[k], b[k], c[k], d[k] = (v * s for v in (a[k], b[k], c[k], d[k]))
+        elif kind == "huge":
+            s = dt(1e36 if fp == L.FP32 else 1e305)
+            a[k], b[k], c[k], d[k] = (v * s for v in (a[k], b[k], c[k], d[k]))
+        else:
+            a[k, n - 1] = 9.0
+    other = np.zeros(B, bool)
+    other[[1, 2, 5, 7, 8, 11]] = True
+    with np.errstate(all="ignore"):
+        ref = oracle.thomas_batched(a, b, c, d, B, n, strided=False, fp="f64" if fp == L.FP64 else "f32").reshape(B, n)
+    assert np.isfinite(ref).all()
+    x = _solve_plain(fp, layout, a, b, c, d, in_place)
+    assert np.isfinite(x).all()
+    for k in range(B):
+        if other[k]:
+            assert np.array_equal(x[k], ref[k]), k
+        else:
+            assert np.abs(x[k].astype(np.float64) - ref[k]).max() <= (1e-13 if fp == L.FP64 else 1e-5) * np.abs(ref[k]).max()
+    # a system's values do not depend on its neighbours
+    keep = ~other
+    assert np.array_equal(_solve_plain(fp, layout, a[keep], b[keep], c[keep], d[keep]), x[keep])
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("layout", [L.LAYOUT_CONTIGUOUS, L.LAYOUT_STRIDED])
+def test_long_systems_with_ends_that_do_not_dominate_equal_the_oracle(oracle, fp, layout):
+    # a Robin end whose weight takes away from the diagonal, on Poisson rows (|b| = |a| + |c|)
+    dt, B, n = L.np_dtype(fp), 5, 1300
+    a, b, c = np.full((B, n), -1.0, dt), np.full((B, n), 2.0, dt), np.full((B, n), -1.0, dt)
+    d = np.random.default_rng(5).standard_normal((B, n)).astype(dt)
+    for lower, upper in (((L.BC_ROBIN, 2.0, 0.1), (L.BC_DIRICHLET, 0.4)), ((L.BC_DIRICHLET, 0.4), (L.BC_ROBIN, -2.0, 0.1))):
+        x = _solve_bc(fp, layout, a, b, c, d, lower, upper)
+        lo = (lower[0], lower[1] if len(lower) == 3 else 0.0, lower[-1])
+        hi = (upper[0], upper[1] if len(upper) == 3 else 0.0, upper[-1])
+        ref = np.stack([oracle.thomas_lu(a[k], b[k], c[k], d[k], lo, hi, "f64" if fp == L.FP64 else "f32") for k in range(B)])
+        assert np.isfinite(ref).all() and np.array_equal(x, ref.astype(np.float64))
