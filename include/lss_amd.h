@@ -219,7 +219,9 @@ int lss_plan_problem_shape(const lss_adi_plan *plan, int64_t p, int64_t *nx, int
  * systems (contiguous: more than 512 unknowns in fp64, 1024 in fp32; strided: more than 1024) are looked at row
  * by row, and those that do not dominate, or whose |b_i| leave 2^-900..2^900 (fp32 2^-100..2^100), are swept in
  * the reference's order with divisions, rounding for rounding, several times slower.  Shorter systems are not
- * looked at: there the chunks' first diagonals must not vanish.
+ * looked at: there the chunks' first diagonals must not vanish.  Rounding: the longer systems put the solution
+ * through their rows once more, and with rows of |b_i| = 2.5 + |a_i| + |c_i| are as close to the exact solution
+ * as the sequential sweep (0.9 of its error, root mean square); the shorter ones are at 1.2 to 1.3 of it.
  */
 int lss_tridiag_batched(int32_t fp, int32_t layout, int64_t B, int64_t n, const void *a, const void *b,
                         const void *c, const void *d, void *x, void *stream);

@@ -2180,7 +2180,7 @@ template <typename T> int tridiag_long_threads(int64_t nf)
 }
 
 // Contiguous systems.  One wavefront per system while four staged systems fit 64 KiB of LDS (fp64: 512
-// unknowns, fp32: 1024), else one workgroup per system (k_tridiag_long; 1000 x 2000 in fp64: 16 us against
+// unknowns, fp32: 1024), else one workgroup per system (k_tridiag_long; 1000 x 2000 in fp64: 19 us against
 // 3380 us with one lane per system).  Returns false when neither takes the size.
 template <typename T> bool tridiag_part_rows(const TriArgs<T> &t, int64_t nf)
 {
@@ -2220,7 +2220,8 @@ template <typename T> bool tridiag_part_rows(const TriArgs<T> &t, int64_t nf)
 //         169 against 195; 65536 x 256: 194 against 158, so shorter systems keep 16 x 64;
 //   fp64, 513..1024: 8 x 128 against 16 x 64 (chunks of 8, not 16, which spilled): 205 against 223;
 //   1025..2048: fp64 4 x 128 (209) against 4 x 256 (214), fp32 8 x 128 (121) against 4 x 256 (140), at
-//         8388 x 2000; longer systems keep one lane per system.
+//         8388 x 2000 and without the last pass of k_tridiag_cols_long (with it 320 and 141); longer systems keep one
+//         lane per system (fp64: 2050).
 template <typename T> bool tridiag_part_cols(const TriArgs<T> &t, int64_t nf)
 {
     if constexpr (sizeof(T) == 4) {

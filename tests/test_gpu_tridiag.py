@@ -235,3 +235,24 @@ def test_long_systems_with_ends_that_do_not_dominate_equal_the_oracle(oracle, fp
         hi = (upper[0], upper[1] if len(upper) == 3 else 0.0, upper[-1])
         ref = np.stack([oracle.thomas_lu(a[k], b[k], c[k], d[k], lo, hi, "f64" if fp == L.FP64 else "f32") for k in range(B)])
         assert np.isfinite(ref).all() and np.array_equal(x, ref.astype(np.float64))
+
+
+@pytest.mark.parametrize("fp,layout,n", LONG)
+def test_long_systems_are_as_accurate_as_the_sequential_sweep(oracle, fp, layout, n):
+    """Error against a longer format, root mean square over the batch, of the rows that the module's tests use: no larger
+    than the sequential sweep's in the same precision (host emulation: 0.9 of it)."""
+    dt, B = L.np_dtype(fp), 48
+    wide = np.longdouble if fp == L.FP64 else np.float64
+    a, b, c, d = _systems(B, n, dt, seed=n + 7)
+    seq = oracle.thomas_batched(a, b, c, d, B, n, strided=False, fp="f64" if fp == L.FP64 else "f32").reshape(B, n)
+    wa, wb, wc, wd = (v.astype(wide) for v in (a, b, c, d))
+    g, exact = np.zeros((B, n), wide), np.zeros((B, n), wide)
+    g[:, 0], exact[:, 0] = wc[:, 0] / wb[:, 0], wd[:, 0] / wb[:, 0]
+    for i in range(1, n):
+        beta = wb[:, i] - wa[:, i] * g[:, i - 1]
+        g[:, i], exact[:, i] = wc[:, i] / beta, (wd[:, i] - wa[:, i] * exact[:, i - 1]) / beta
+    for i in range(n - 2, -1, -1):
+        exact[:, i] -= g[:, i] * exact[:, i + 1]
+    err = [float(np.sqrt(np.mean((v.astype(wide) - exact) ** 2))) for v in (_solve_plain(fp, layout, a, b, c, d), seq)]
+    print(f"n={n} layout={layout} fp={fp}: rms error {err[0]:.2e}, sequential {err[1]:.2e}", flush=True)
+    assert err[0] <= err[1]
