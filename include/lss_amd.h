@@ -152,7 +152,8 @@ int lss_adi_set_adjoint_overlap(lss_adi_plan *plan, int32_t mode);
  * compile-time factor pattern and there is no heat source; fewer than 64 problems: at most 5000 points
  * each in fp64, 9000 in fp32); the mapping does not matter to them and the autotuner does not run for
  * them.  Larger books whose state exceeds the last-level cache are stepped in slices, launched directly
- * (use_graph then only selects the two groups).  Partitioned plans of at most 3 million points evaluate
+ * (use_graph then only selects the two groups), unless they are partitioned with FIELDS coefficients only or exact
+ * with SEPARABLE ones.  Partitioned plans of at most 3 million points evaluate
  * boundary stage B in the last v-sweep; a profiled run keeps its launch. */
 enum { LSS_KERNEL_CONFIG_LEN = 13 };
 int lss_plan_kernel_config(const lss_adi_plan *plan, int32_t *config);

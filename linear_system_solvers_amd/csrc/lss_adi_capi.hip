@@ -173,12 +173,19 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     // slice find most of it cached.  Smaller slices leave CUs idle and pay more launches.  Measured in fp64 (ms a
     // solve by the bytes of a slice, MB): 1024 mixed Heston problems of up to 512 x 256, 50..500 steps: 130: 376, 160:
     // 348, 200: 329, 260: 313, 320: 335, 450: 379, one slice: 377; 256 MCS problems of 512 x 256, 60 steps: 260: 46,
-    // 320: 54, 550: 62, one slice: 62.  So as many slices as bring each nearest to the cache's 256 MB.
+    // 320: 54, 550: 62, one slice: 62.  So as many slices as bring each nearest to the cache's 256 MB.  Explicit Euler
+    // steps likewise: 256 problems of 512 x 256, 200 steps 55.0 ms, 60.1 with slices of 1.5 times that, one slice 65.2.
+    // Exact plans stream a workspace of 12 surfaces besides the state, which no slice that fills the GPU could keep in
+    // the cache (128 mixed problems of 512 x 256, SEPARABLE: slices of 256 MB with it 49.1 ms, of 256 MB of state 30.1,
+    // one slice 27.6); only with FIELDS coefficients, 7 more surfaces, are slices worth it (38.0 against 39.1 ms; fp32,
+    // 256 DR problems: 27.4 against 28.9).  Partitioned plans are the other way round: SEPARABLE ones gain, FIELDS
+    // ones do not (128 mixed problems 19.6 against 19.5 ms; fp32, 256 HV problems: 25.3 against 24.7).
     // A sliced loop is launched directly: its kernels last longer than their launches take the host (312.6 ms against
     // 313.8 ms as a graph), and capturing its hundred thousand launches would cost a first solve 0.3 s.
     static constexpr double SLICE_BYTES = 256e6;
     std::vector<int64_t> slices;       // slice k: internal problems slices[k] .. slices[k + 1] - 1
     int64_t slice_q0 = 0, slice_q1 = 0;  // problems of the launches (default: all)
+    int64_t tune_q1 = 0;                 // problems of the autotuner's launches: a slice's, whether the loop is sliced or not
     void all_problems()
     {
         slice_q0 = 0;
@@ -199,6 +206,9 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
             at += bytes(probs[q]);
         }
         slices.push_back(count);
+        tune_q1 = slices[1];
+        if (!euler && all_fields != (line_solver == LINE_EXACT))
+            slices = {0, count};
         all_problems();
     }
 
@@ -850,7 +860,7 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
         if (line_solver != LINE_PARTITIONED || euler)
             return;
         const int nst = std::min(max_steps, 8);
-        slice_q1 = slices[1];  // (the first slice stands for the others)
+        slice_q1 = tune_q1;  // (a slice's problems stand for the others)
         hipEvent_t e0, e1;
         HIPCHK(hipEventCreate(&e0));
         HIPCHK(hipEventCreate(&e1));

@@ -541,3 +541,26 @@ def test_exact_sweeps_round_like_the_oracle_at_any_magnitude(oracle, fp, rate, s
         with np.errstate(all="ignore"):
             c = oracle.step(oracle_pde(oracle, m), oracle_cfg(oracle, m), u, 0.0, ofp)  # (its data do not see the time)
         assert np.array_equal(g, c, equal_nan=True) and np.array_equal(np.signbit(g[g == 0]), np.signbit(c[c == 0])), z
+
+
+def test_an_exact_book_of_sampled_coefficients_equals_its_problems_solved_alone():
+    """Exact plans run in slices of problems only if every problem has FIELDS coefficients (2 slices here: 200 problems of
+    about 3.0 or 1.8 MB of state); no tolerance."""
+    torch = pytest.importorskip("torch")
+    rng = np.random.default_rng(43)
+    models = [_stable(int(rng.integers(290, 311)), int(rng.integers(240, 261)), steps=int(rng.integers(1, 6)),
+                      splitting=q % 4, strike=float(rng.uniform(60, 140)), coeff_mode=L.COEFF_FIELDS,
+                      line_solver=L.LINE_EXACT) for q in range(200)]
+    plan = L.Plan.from_models(models)
+    ins = [torch.from_numpy(plan.initial(p)).cuda() for p in range(plan.count)]
+    st = torch.cuda.current_stream().cuda_stream
+    res = []
+    for graph in (False, True):
+        outs = [torch.full_like(u, float("nan")) for u in ins]
+        plan.run_dev([u.data_ptr() for u in ins], [o.data_ptr() for o in outs], st, graph=graph)
+        res.append([(o * 1.0).cpu().numpy() for o in outs])
+        torch.cuda.synchronize()
+    plan.close()
+    assert all(np.array_equal(a, b) for a, b in zip(*res))
+    for q in range(0, 200, 23):
+        assert np.array_equal(_solve(models[q]), res[0][q]), q
