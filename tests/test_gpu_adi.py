@@ -564,3 +564,41 @@ def test_an_exact_book_of_sampled_coefficients_equals_its_problems_solved_alone(
     assert all(np.array_equal(a, b) for a, b in zip(*res))
     for q in range(0, 200, 23):
         assert np.array_equal(_solve(models[q]), res[0][q]), q
+
+
+@pytest.mark.parametrize("fp", [L.FP64, L.FP32])
+@pytest.mark.parametrize("model", ["heston", "sabr"])
+@pytest.mark.parametrize("nx,ny,count", [(4, 4, 4), (19, 18, 4), (35, 51, 4), (66, 67, 4), (101, 60, 64)])
+def test_resident_loop_steps_like_the_step_by_step_kernels(fp, model, nx, ny, count):
+    """Every level of the resident loop against a profiled run of as many steps, which is stepped launch by launch (within
+    the partitioned solver's tolerance above).  That the loop was resident shows in the autotuner, which runs before a
+    step-by-step plan's first solve and never for a resident one."""
+    torch = pytest.importorskip("torch")
+    steps = 5
+
+    def problems(n):
+        if model == "heston":
+            return [_stable(nx, ny, steps=n, splitting=q % 4, coeff_mode=L.COEFF_SEPARABLE,
+                            line_solver=L.LINE_PARTITIONED) for q in range(count)]
+        return [_sabr_small(nx, ny, n, q % 4) for q in range(count)]
+
+    plan = L.Plan.from_models(problems(steps), fp)
+    ins = [torch.from_numpy(plan.initial(p)).cuda() for p in range(count)]
+    pin = [u.data_ptr() for u in ins]
+    outs = [torch.full_like(u, float("nan")) for u in ins]
+    levels = [torch.full((steps + 1, nx, ny), float("nan"), dtype=u.dtype, device="cuda") for u in ins]
+    plan.run_levels_dev(pin, [v.data_ptr() for v in levels])
+    plan.run_dev(pin, [o.data_ptr() for o in outs])
+    torch.cuda.synchronize()
+    assert plan.kernel_config()["tuned"] == 0
+    plan.close()
+    tol = 1e-12 if fp == L.FP64 else 1e-5
+    for n in range(1, steps + 1):
+        short = L.Plan.from_models(problems(n), fp)
+        own = [torch.full_like(u, float("nan")) for u in ins]
+        L.run_profiled(short, pin, [o.data_ptr() for o in own], torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        short.close()
+        for p in range(count):
+            e = _normwise(levels[p][n].cpu().numpy().astype(np.float64), own[p].cpu().numpy().astype(np.float64))
+            assert e <= tol, (n, p, e)
