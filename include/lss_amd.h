@@ -106,7 +106,9 @@ int32_t lss_version(void);
 /*
  * Plans.  A plan holds `count` independent problems (count == 1: the single-problem stepper that
  * general_heston_equation::solve's device branch uses, heston_equation.hpp:221-233; count > 1: a
- * batched book stepping all problems in the same launches).  All problems share fp.
+ * batched book stepping all problems in the same launches).  All problems share fp.  Device memory per grid point
+ * of an ADI problem: 3 values of state (DR) or 5, in exact plans 12 of workspace, and per set of FIELDS
+ * coefficients 7.
  */
 int lss_adi_plan_create(const lss_adi_desc *descs, int64_t count, lss_adi_plan **plan);
 int lss_adi_plan_destroy(lss_adi_plan *plan);
@@ -267,7 +269,8 @@ int lss_tridiag_batched_noalloc(int32_t fp, int32_t layout, int64_t B, int64_t n
  * Same time loop as lss_adi_run_dev (device pointers, no graph) with a hipEvent pair recorded on
  * `stream` around every launch; synchronous.  For each kernel kind k < LSS_K_COUNT it returns the
  * summed launch time ms[k], the summed algorithmic HBM bytes bytes[k] (compulsory reads and writes
- * of the 2-D state arrays of the problems active in each launch) and the number of launches.
+ * of the 2-D state arrays of the problems active in each launch) and the number of launches.  (LSS_K_BND_A and
+ * LSS_K_HV_Y3 have none: other kernels evaluate both.  Exact plans have none of LSS_K_BND_B either.)
  */
 enum {
     LSS_K_BND_A = 0, LSS_K_XSWEEP1 = 1, LSS_K_VSWEEP1 = 2, LSS_K_HV_Y3 = 3, LSS_K_XSWEEP2 = 4, LSS_K_VSWEEP2 = 5,

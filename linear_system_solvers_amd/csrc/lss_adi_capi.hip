@@ -348,11 +348,11 @@ template <typename T> struct PlanImpl final : lss_adi_plan {
     static constexpr int64_t FOLD_POINTS = 3000000;
     // The resident loop (k_adi_res) takes a plan whose problems all have lines of at most 16 ARES_C interior points and
     // fit LDS.  A step takes it the same time for 1 to 256 problems, in proportion to their points; the step-by-step
-    // loop, which spreads a problem over the GPU, takes 10.6 us for one problem of any such size in fp64, 18.5 us for
-    // 64.  Measured (DR steps, us, fp64: 1 and 64 problems step by step against resident): 100 x 50: 10.6, 18.5, 8.7;
-    // 100 x 64: 10.5, 18.7, 10.9; 130 x 66: 10.9, 19.8, 16.8; fp32: 100 x 90: 10.0, 16.6, 8.3; 130 x 100: 10.2, 17.3,
-    // 13.1; HV: fp64 100 x 50: 19.4, 33.7, 19.6; fp32 100 x 90: 18.1, 29.6, 17.8.  So larger problems need a book.  (Resident times before the
-    // v-lines' matrix was eliminated once; they are 0.85 of these since.)
+    // loop spreads a problem over the GPU and grows with their number.  Measured (us a step; 1, 16, 63 problems step by
+    // step against resident): fp64 DR 100 x 50: 9.0, 13.1, 16.3 against 7.3 to 7.6; 100 x 64: 9.0, 13.2, 16.6 against
+    // 11.6 to 11.8; HV 100 x 50: 17.9, 25.0, 31.7 against 16.9 to 17.3; fp32 DR 100 x 90: 8.2, 11.9, 14.5 against 7.6
+    // to 7.8; 114 x 114: 8.3, 12.1, 15.4 against 8.7 to 9.0; HV 100 x 90: 16.4, 22.9, 28.1 against 16.2 to 16.6.  So
+    // one larger problem is better off step by step; several are not, and the bound for fewer than 64 is one's.
     static constexpr int64_t RES_POINTS = sizeof(T) == 8 ? 5000 : 9000, RES_BOOK = 64;
     static bool resident_ok(const Prob<T> &p, int64_t problems)
     {

@@ -23,7 +23,7 @@ enum : int32_t { TRI_THOMAS = 0, TRI_DSWEEP = 1 };
 //   SEPARABLE: each transformed coefficient q in {a,b,c,d,e,f} is q(i,j) = X0q[i]*Y0q[j] + X1q[i]*Y1q[j]
 //              (12 nx vectors, 12 ny vectors); M..W are formed in the kernel.
 enum : int32_t { COEFF_FIELDS = 0, COEFF_SEPARABLE = 1 };
-// line solver of the sweeps: the reference's sequential order (one lane per line) or partitioned
+// line solver of the sweeps: the reference's sequential order (four lanes per line) or partitioned
 enum : int32_t { LINE_EXACT = 0, LINE_PARTITIONED = 1 };
 
 constexpr int TILE = 64;  // lines (or points) per workgroup tile: one wavefront

@@ -1,6 +1,6 @@
 """GPU 1-D implicit heat / Black-Scholes solver (include/lss_heat1d.h) against the oracle.
 
-* The exact kernel (one lane per problem, the reference's Thomas LU / double-sweep order, no
+* The exact kernel (four lanes per problem, the reference's Thomas LU / double-sweep order, no
   contraction) equals the oracle's restatement of the reference's host solver bit for bit, final level
   and every level, fp64 and fp32, Euler and Crank-Nicolson, Forward and Backward, both grids.
 * The partitioned kernel (one wavefront per problem, the whole loop in registers, fused multiply-adds)
